@@ -18,26 +18,49 @@ __device__ __forceinline__ void two_sum_fold(float &hi, float &lo, float p) {
   lo += e;
 }
 
-template <int K, bool MASK>
-__device__ __forceinline__ void pair_f32(const float4 q, const int j, const float (&xi)[K],
-                                         const float (&yi)[K], const float (&zi)[K],
-                                         const int (&ii)[K], const float eps2, float (&px)[K],
-                                         float (&py)[K], float (&pz)[K]) {
+// U j-bodies q[u] (indices j + u) against the K bodies of a lane, added in the order of u.
+// PRIO: their rsq together at a raised wave priority (prio_up), taken by the loop of two j-bodies
+// per step.  MI355X, without and with it: 2^18 bodies with (1, 16) 16.38 and 15.51 ms; the j-split
+// form at 16384 bodies 74.6 and 70.0 us, at 49999 605 and 569 us; the batched per-step schedule
+// on 1024 universes of 32-2048 bodies 0.147 and 0.137 ms per step.  One s_setprio pair per body
+// instead of two bodies: 15.69 ms, 70.9 us, 573 us, 0.138 ms, and 1758 against 1746 us for the
+// forward and backward of 128 such universes, whose last wavefronts run alone on their SIMDs.
+// The loop of eight serves launches of about one wavefront per SIMD, which it slows down (2000
+// bodies in 32 workgroups: a step of 36.7 against 35.7 us).
+template <int K, bool MASK, bool PRIO, int U>
+__device__ __forceinline__ void pairs_f32(const float4 (&q)[U], const int j,
+                                          const float (&xi)[K], const float (&yi)[K],
+                                          const float (&zi)[K], const int (&ii)[K],
+                                          const float eps2, float (&px)[K], float (&py)[K],
+                                          float (&pz)[K]) {
+  float dx[U][K], dy[U][K], dz[U][K], inv[U][K];
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const float dx = q.x - xi[k];
-    const float dy = q.y - yi[k];
-    const float dz = q.z - zi[k];
-    float r2 = __builtin_fmaf(dx, dx, eps2);
-    r2 = __builtin_fmaf(dy, dy, r2);
-    r2 = __builtin_fmaf(dz, dz, r2);
-    float inv = __builtin_amdgcn_rsqf(r2);
-    if (MASK) inv = (j == ii[k]) ? 0.0f : inv;
-    const float s = (q.w * inv) * (inv * inv);
-    px[k] = __builtin_fmaf(dx, s, px[k]);
-    py[k] = __builtin_fmaf(dy, s, py[k]);
-    pz[k] = __builtin_fmaf(dz, s, pz[k]);
-  }
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      dx[u][k] = q[u].x - xi[k];
+      dy[u][k] = q[u].y - yi[k];
+      dz[u][k] = q[u].z - zi[k];
+      float r2 = __builtin_fmaf(dx[u][k], dx[u][k], eps2);
+      r2 = __builtin_fmaf(dy[u][k], dy[u][k], r2);
+      inv[u][k] = __builtin_fmaf(dz[u][k], dz[u][k], r2);
+    }
+  if constexpr (PRIO) prio_up();
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int k = 0; k < K; ++k) inv[u][k] = __builtin_amdgcn_rsqf(inv[u][k]);
+  if constexpr (PRIO) prio_down();
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (MASK) inv[u][k] = (j + u == ii[k]) ? 0.0f : inv[u][k];
+      const float s = (q[u].w * inv[u][k]) * (inv[u][k] * inv[u][k]);
+      px[k] = __builtin_fmaf(dx[u][k], s, px[k]);
+      py[k] = __builtin_fmaf(dy[u][k], s, py[k]);
+      pz[k] = __builtin_fmaf(dz[u][k], s, pz[k]);
+    }
 }
 
 // s_waitcnt immediate that waits for every scalar (and LDS) access and no other counter:
@@ -54,7 +77,7 @@ constexpr unsigned kWaitScalar = 0xC07F;
 // of them; the explicit wait comes before the next load is issued).  MI355X, Plummer:
 // 16.57-16.64 against 17.12-17.17 ms at 2^18 with (1, 16), the j-split form at 16384 bodies
 // 0.079 against 0.081 ms, the batched per-step schedule on 4096 universes of 32-2048 bodies
-// 0.548 against 0.563 ms per step.  It made
+// 0.548 against 0.563 ms per step (before the raised priority).  It made
 // the j-split form with two bodies per lane slower (2^18: 18.7 against 17.4 ms), and with
 // eight j-bodies per step the second set pushed SGPRs into VGPRs (K = 2: 51 to 118).
 template <int K, bool MASK, int JB>
@@ -74,23 +97,17 @@ __device__ __forceinline__ void pair_range_f32(const float4 *__restrict__ posm, 
 #pragma unroll
         for (int u = 0; u < JB; ++u) b[u] = posm[j + JB + u];
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < JB; ++u)
-          pair_f32<K, MASK>(a[u], j + u, xi, yi, zi, ii, eps2, px, py, pz);
+        pairs_f32<K, MASK, true>(a, j, xi, yi, zi, ii, eps2, px, py, pz);
         // the next step of set a, or (past the end) a step in range that is not used
         const int jn = min(j + 2 * JB, j1 - JB);
         __builtin_amdgcn_s_waitcnt(kWaitScalar);
 #pragma unroll
         for (int u = 0; u < JB; ++u) a[u] = posm[jn + u];
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < JB; ++u)
-          pair_f32<K, MASK>(b[u], j + JB + u, xi, yi, zi, ii, eps2, px, py, pz);
+        pairs_f32<K, MASK, true>(b, j + JB, xi, yi, zi, ii, eps2, px, py, pz);
       }
       if (j + JB <= j1) {
-#pragma unroll
-        for (int u = 0; u < JB; ++u)
-          pair_f32<K, MASK>(a[u], j + u, xi, yi, zi, ii, eps2, px, py, pz);
+        pairs_f32<K, MASK, true>(a, j, xi, yi, zi, ii, eps2, px, py, pz);
         j += JB;
       }
     }
@@ -99,14 +116,12 @@ __device__ __forceinline__ void pair_range_f32(const float4 *__restrict__ posm, 
       float4 q[JB];
 #pragma unroll
       for (int u = 0; u < JB; ++u) q[u] = posm[j + u];
-#pragma unroll
-      for (int u = 0; u < JB; ++u)
-        pair_f32<K, MASK>(q[u], j + u, xi, yi, zi, ii, eps2, px, py, pz);
+      pairs_f32<K, MASK, (JB <= 2)>(q, j, xi, yi, zi, ii, eps2, px, py, pz);
     }
   }
   for (; j < j1; ++j) {
-    const float4 q = posm[j];
-    pair_f32<K, MASK>(q, j, xi, yi, zi, ii, eps2, px, py, pz);
+    const float4 q[1] = {posm[j]};
+    pairs_f32<K, MASK, (JB <= 2)>(q, j, xi, yi, zi, ii, eps2, px, py, pz);
   }
 }
 
