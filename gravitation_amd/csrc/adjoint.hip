@@ -322,8 +322,7 @@ __device__ __forceinline__ void stage1_vjp_f32_block(
     const int b = max(a, min(j1, iend));
     // eps2 in a VGPR, so that the first r2 FMA takes no SGPR operand (2^18 j-split VJP:
     // 34.85 against 35.27-35.37 ms)
-    float eps2v;
-    asm volatile("v_mov_b32 %0, %1" : "=v"(eps2v) : "s"(eps2));
+    const float eps2v = in_vgpr(eps2);
     vjp_segment<K, false>(posm, mu4, j0, a, jblock, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2v, hi,
                           lo);
     vjp_segment<K, true>(posm, mu4, a, b, jblock, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2v, hi,

@@ -55,6 +55,13 @@ bool sym_batched_supported(int K, int W);
 __device__ __forceinline__ void prio_up() { __builtin_amdgcn_s_setprio(1); }
 __device__ __forceinline__ void prio_down() { __builtin_amdgcn_s_setprio(0); }
 
+// A wave-uniform value in a VGPR, so that FP32 instructions using it take no constant-bus operand.
+__device__ __forceinline__ float in_vgpr(float x) {
+  float v;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(v) : "s"(x));
+  return v;
+}
+
 // 1/sqrt(x) in FP64: the v_rsq_f64 seed refined by one Newton-Raphson step
 // y <- y + (y/2)(1 - x y^2).  Measured on gfx950 over 2^20 arguments spanning 2^-60..2^61,
 // the seed's relative error is at most 5.2e-8 (2^-24.2) and the refined value's at most

@@ -224,8 +224,7 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
   const int j1 = min(jhi, j0 + chunk);
   // eps2 in a VGPR, so that the first r2 FMA takes no SGPR operand (an SGPR operand adds
   // issue cycles to an FP32 instruction): 2^18 with (1, 16) 16.86 against 17.14 ms
-  float eps2v;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(eps2v) : "s"(eps2));
+  const float eps2v = in_vgpr(eps2);
   if (mask_self)
     sum_segment_f32<K, true, JB>(posm, j0, j1, jblock, ibase, iend, xi, yi, zi, ii, eps2v, hx,
                                  hy, hz, lx, ly, lz);

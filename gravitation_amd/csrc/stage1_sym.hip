@@ -52,22 +52,35 @@ __device__ __forceinline__ float4 load_or_far(const float4 *__restrict__ posm, i
 }
 
 // One block pair (beta, gamma) for one workgroup: its wavefronts hold K block-beta bodies per
-// lane (xi..mi) and take the K*W chunks of 64 block-gamma bodies from jb0 (bodies at or past
+// lane (xi..zi, the masses negated in mn) and take the K*W chunks of 64 block-gamma bodies from jb0 (bodies at or past
 // jend load as far, massless padding).  The i-side sums of every chunk fold into the TwoSum
 // pairs (hx, lx) .. (hz, lz), which the caller may carry over several gamma blocks; the j-side
 // sums of a chunk, added over the W wavefronts through the double-buffered LDS `red` (buffer
 // chunk & 1, chunk counting on across calls), go to pj[c * IB + jc * 64 + l], 3 * IB floats.
+//
+// Bound by the issue of VALU instructions: per pair 16 FP32, one v_rsq_f32 and 7/K DPP moves,
+// about 44 + 30 / K cycles per SIMD if every two FP32 instructions of different wavefronts go
+// side by side.  For that the rsq (of G = 2 pairs together) and the DPP moves are issued at a
+// raised priority (prio_up), eps2 sits in a VGPR and the masses come negated, so that the j side
+// needs no negating (8-byte) FMA.  MI355X, (8, 2), before and after: 2^18 bodies 13.40 and
+// 11.13 ms (65.7 to 54 cycles per pair of bodies and wavefront), 2^17 3.44 and 2.87 ms; (4, 2) at
+// 49999 bodies 0.652 and 0.496 ms.  G = 4 pairs need 138 VGPRs with K = 8 for 11.05 ms, G = 1
+// takes 11.19 ms.  Measured and not kept: the j-bodies read from LDS instead of rotated (3 DPP
+// moves per step instead of 7) is no faster once the moves have priority (2.95 against 2.86 ms
+// at 2^17), and temporaries pinned to registers of alternating parity (an FMA whose three
+// operands have register numbers of one parity issues alone) gain 1 %.
 template <int K, int W>
 __device__ __forceinline__ void sym_block_pair(const float4 *__restrict__ posm, int jb0,
                                                int jend, float eps2, const float (&xi)[K],
                                                const float (&yi)[K], const float (&zi)[K],
-                                               const float (&mi)[K], float (&hx)[K],
+                                               const float (&mn)[K], float (&hx)[K],
                                                float (&hy)[K], float (&hz)[K], float (&lx)[K],
                                                float (&ly)[K], float (&lz)[K],
                                                float *__restrict__ pj,
                                                float (&red)[2][W][3][kWave], int &chunk,
                                                int lane, int wave) {
   constexpr int IB = kWave * K * W;
+  constexpr int G = 2;
   for (int jc = 0; jc < K * W; ++jc, ++chunk) {
     const float4 q = load_or_far(posm, jb0 + jc * kWave + lane, jend);
     float xj = q.x, yj = q.y, zj = q.z, mj = q.w;
@@ -75,29 +88,40 @@ __device__ __forceinline__ void sym_block_pair(const float4 *__restrict__ posm, 
     float px[K], py[K], pz[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) px[k] = py[k] = pz[k] = 0.0f;
-    // not unrolled: the 169-instruction body of one step ran 4 % faster than the 318 of two
-    // steps (MI355X, 2^18: 13.36 against 13.96 ms; 2^20: 212 against 221 ms)
+    // not unrolled: the body of one step ran 4 % faster than that of two steps (2^18: 13.36
+    // against 13.96 ms, before the raised priority)
 #pragma unroll 1
     for (int t = 0; t < kWave; ++t) {
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const float dx = xj - xi[k];
-        const float dy = yj - yi[k];
-        const float dz = zj - zi[k];
-        float r2 = __builtin_fmaf(dx, dx, eps2);
-        r2 = __builtin_fmaf(dy, dy, r2);
-        r2 = __builtin_fmaf(dz, dz, r2);
-        const float inv = __builtin_amdgcn_rsqf(r2);
-        const float inv3 = inv * (inv * inv);
-        const float si = mj * inv3;
-        const float sj = mi[k] * inv3;
-        px[k] = __builtin_fmaf(dx, si, px[k]);
-        py[k] = __builtin_fmaf(dy, si, py[k]);
-        pz[k] = __builtin_fmaf(dz, si, pz[k]);
-        ajx = __builtin_fmaf(-dx, sj, ajx);
-        ajy = __builtin_fmaf(-dy, sj, ajy);
-        ajz = __builtin_fmaf(-dz, sj, ajz);
+      for (int k = 0; k < K; k += G) {
+        float dx[G], dy[G], dz[G], inv[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          dx[g] = xj - xi[k + g];
+          dy[g] = yj - yi[k + g];
+          dz[g] = zj - zi[k + g];
+          float r2 = __builtin_fmaf(dx[g], dx[g], eps2);
+          r2 = __builtin_fmaf(dy[g], dy[g], r2);
+          inv[g] = __builtin_fmaf(dz[g], dz[g], r2);
+        }
+        prio_up();
+#pragma unroll
+        for (int g = 0; g < G; ++g) inv[g] = __builtin_amdgcn_rsqf(inv[g]);
+        prio_down();
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const float inv3 = inv[g] * (inv[g] * inv[g]);
+          const float si = mj * inv3;
+          const float sj = mn[k + g] * inv3;
+          px[k + g] = __builtin_fmaf(dx[g], si, px[k + g]);
+          py[k + g] = __builtin_fmaf(dy[g], si, py[k + g]);
+          pz[k + g] = __builtin_fmaf(dz[g], si, pz[k + g]);
+          ajx = __builtin_fmaf(dx[g], sj, ajx);
+          ajy = __builtin_fmaf(dy[g], sj, ajy);
+          ajz = __builtin_fmaf(dz[g], sj, ajz);
+        }
       }
+      prio_up();
       xj = rot1(xj);
       yj = rot1(yj);
       zj = rot1(zj);
@@ -105,6 +129,7 @@ __device__ __forceinline__ void sym_block_pair(const float4 *__restrict__ posm, 
       ajx = rot1(ajx);
       ajy = rot1(ajy);
       ajz = rot1(ajz);
+      prio_down();
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -146,7 +171,7 @@ __global__ __launch_bounds__(kWave *W) void k_sym_pairs(const float4 *__restrict
   const int4 it = items[blockIdx.x];
   const size_t base = static_cast<size_t>(blockIdx.x) * 3 * IB;
 
-  float xi[K], yi[K], zi[K], mi[K];
+  float xi[K], yi[K], zi[K], mn[K];
   float hx[K], hy[K], hz[K], lx[K], ly[K], lz[K];
   const int i0 = it.x + wave * (K * kWave);
 #pragma unroll
@@ -155,11 +180,12 @@ __global__ __launch_bounds__(kWave *W) void k_sym_pairs(const float4 *__restrict
     xi[k] = p.x;
     yi[k] = p.y;
     zi[k] = p.z;
-    mi[k] = p.w;
+    mn[k] = -p.w;
     hx[k] = hy[k] = hz[k] = lx[k] = ly[k] = lz[k] = 0.0f;
   }
   int chunk = 0;
-  sym_block_pair<K, W>(posm, it.y, it.w, eps2, xi, yi, zi, mi, hx, hy, hz, lx, ly, lz,
+  const float eps2v = in_vgpr(eps2);
+  sym_block_pair<K, W>(posm, it.y, it.w, eps2v, xi, yi, zi, mn, hx, hy, hz, lx, ly, lz,
                        p_j + base, red, chunk, lane, wave);
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -242,7 +268,7 @@ __global__ __launch_bounds__(kWave *W) void k_sym_segments(const float4 *__restr
   const int g1 = min(nb, g0 + (1 << lg));
   const size_t local = blockIdx.x;
 
-  float xi[K], yi[K], zi[K], mi[K];
+  float xi[K], yi[K], zi[K], mn[K];
   float hx[K], hy[K], hz[K], lx[K], ly[K], lz[K];
   const int i0 = beta * IB + wave * (K * kWave);
 #pragma unroll
@@ -251,13 +277,14 @@ __global__ __launch_bounds__(kWave *W) void k_sym_segments(const float4 *__restr
     xi[k] = p.x;
     yi[k] = p.y;
     zi[k] = p.z;
-    mi[k] = p.w;
+    mn[k] = -p.w;
     hx[k] = hy[k] = hz[k] = lx[k] = ly[k] = lz[k] = 0.0f;
   }
   int chunk = 0;
+  const float eps2v = in_vgpr(eps2);
   for (int gamma = g0; gamma < g1; ++gamma) {
     float *pj = p_j + ((local << lg) + (gamma - g0)) * (3 * IB);
-    sym_block_pair<K, W>(posm, gamma * IB, n, eps2, xi, yi, zi, mi, hx, hy, hz, lx, ly, lz,
+    sym_block_pair<K, W>(posm, gamma * IB, n, eps2v, xi, yi, zi, mn, hx, hy, hz, lx, ly, lz,
                          pj, red, chunk, lane, wave);
   }
   const size_t base = local * 3 * IB;
