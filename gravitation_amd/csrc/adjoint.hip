@@ -211,24 +211,66 @@ __device__ __forceinline__ void vjp_segment(const float4 *__restrict__ posm,
     float px[K], py[K], pz[K], pg[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) px[k] = py[k] = pz[k] = pg[k] = 0.0f;
-    // j-bodies (position and cotangent) per loop step: two with one body per lane, four
-    // otherwise.  Same order of pairs, same bits.  MI355X, Plummer, j-split VJP (1, 8, 16):
-    // 2^18 35.6-35.7 against 36.7-37.1 ms, 16384 0.188 against 0.195 ms, a 4096-body
-    // universe's forward + adjoint over 200 steps 7.48-7.50 against 7.56-7.59 ms; with two per
-    // step the owner-computes VJP of two bodies per lane took 4.41 against 3.96 ms at 2^16.
-    constexpr int JB = K == 1 ? 2 : 4;
+    // j-bodies (position and cotangent) per loop step.  With one body per lane three, their rsq
+    // together at a raised priority and their loads one step ahead in two SGPR sets (the
+    // scheme of pair_range_f32: each half-step waits for its set, issues the other's next load
+    // and then computes); otherwise four, plain.  The order of the pairs, hence the bits, does
+    // not depend on it.  Bound by VALU issue in large launches (29 FP32 and a v_rsq_f32: 72 cycles
+    // per pair and SIMD at best, 79 at 65536 bodies) and by the latency of the scalar loads in
+    // launches of few wavefronts per SIMD, which the loads ahead hide.  MI355X, plain loop of two
+    // and this one: j-split VJP of 4096 bodies 18.4 and 16.2 us, 16384 149.8 and 146.7 us, 65536
+    // 2185 and 2161 us; forward and backward of 128 universes of 64-2048 bodies over 12 steps 1744
+    // and 1297 us.  Loads ahead of two: 17.1, 147.2, 2163 and 1462 us; of four: 16.3, 148.0, 2180
+    // and 1331 us; of two without the priority: 17.5, 163.4, 2396 and 1444 us.
+    constexpr int JB = K == 1 ? 3 : 4;
     int j = jb;
-    for (; j + JB <= je; j += JB) {
-      float4 q[JB], u[JB];
+    if constexpr (K == 1) {
+      if (j + JB <= je) {
+        float4 qa[JB], ua[JB], qb[JB], ub[JB];
 #pragma unroll
-      for (int t = 0; t < JB; ++t) {
-        q[t] = posm[j + t];
-        u[t] = mu4[j + t];
+        for (int t = 0; t < JB; ++t) {
+          qa[t] = posm[j + t];
+          ua[t] = mu4[j + t];
+        }
+        for (; j + 2 * JB <= je; j += 2 * JB) {
+          __builtin_amdgcn_s_waitcnt(kWaitScalar);
+#pragma unroll
+          for (int t = 0; t < JB; ++t) {
+            qb[t] = posm[j + JB + t];
+            ub[t] = mu4[j + JB + t];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          vjp_pairs<K, MASK, true>(qa, ua, j, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2, px, py,
+                                   pz, pg);
+          // the next step of set a, or (past the end) a step in range that is not used
+          const int jn = min(j + 2 * JB, je - JB);
+          __builtin_amdgcn_s_waitcnt(kWaitScalar);
+#pragma unroll
+          for (int t = 0; t < JB; ++t) {
+            qa[t] = posm[jn + t];
+            ua[t] = mu4[jn + t];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          vjp_pairs<K, MASK, true>(qb, ub, j + JB, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2, px,
+                                   py, pz, pg);
+        }
+        if (j + JB <= je) {
+          vjp_pairs<K, MASK, true>(qa, ua, j, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2, px, py,
+                                   pz, pg);
+          j += JB;
+        }
       }
+    } else {
+      for (; j + JB <= je; j += JB) {
+        float4 q[JB], u[JB];
 #pragma unroll
-      for (int t = 0; t < JB; ++t)
-        vjp_pair<K, MASK>(q[t], u[t], j + t, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2, px, py,
-                          pz, pg);
+        for (int t = 0; t < JB; ++t) {
+          q[t] = posm[j + t];
+          u[t] = mu4[j + t];
+        }
+        vjp_pairs<K, MASK, false>(q, u, j, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2, px, py, pz,
+                                  pg);
+      }
     }
     for (; j < je; ++j)
       vjp_pair<K, MASK>(posm[j], mu4[j], j, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2, px, py, pz,
@@ -510,10 +552,9 @@ __global__ __launch_bounds__(kWave *S) void k_backward_pair(
                                 part_a, eslot, b % tiles_a, b / tiles_a, splits_a, red);
   } else {
     const int c = b - nba;
-    // j-bodies per pair-loop step as pair_loop_width takes them for the paired launches, which
-    // serve universes of a few thousand bodies (hundreds of workgroups): two with one body
-    // per lane (its loop loads the next step ahead), eight otherwise
-    constexpr int JB = KR == 1 ? 2 : 8;
+    // j-bodies per pair-loop step: four with one body per lane (with two, forward and backward
+    // of 4096 bodies over 60 steps took 2.07 against 2.00 ms), eight otherwise
+    constexpr int JB = KR == 1 ? 4 : 8;
     stage1_f32_block<KR, S, JB>(pr, nullptr, n, 0, n, 1.0f, eps2, mask, 256, nullptr, 0, part_r,
                                 c % tiles_r, c / tiles_r, splits_r, red);
   }

@@ -18,6 +18,7 @@
 //   * eps == 0 excludes the self term: only the j-segment overlapping the workgroup's own
 //     i-range runs the masked pair routine, the rest runs unmasked.
 #include <algorithm>
+#include <type_traits>
 
 #include "grav_common.h"
 #include "stage1_f32.h"
@@ -219,8 +220,8 @@ int launch_f32(const float4 *posm, float *acc, int n, int i0, int m, float G, fl
   const int grid = items ? nitems : (m + per_block - 1) / per_block;
   const size_t lds = (S > 1) ? sizeof(float) * (S - 1) * 6 * per_block : 0;
   if (grid == 0) return GRAV_OK;
-  constexpr int kNarrow = K >= 4 ? 8 : 2;   // pair_loop_width: eight from K = 4 on
-  if (pair_loop_width(grid, K) == 8)
+  constexpr int kNarrow = K >= 4 ? 8 : K == 1 ? 4 : 2;   // pair_loop_width's other value
+  if (pair_loop_width(grid, K, false) == 8)
     hipLaunchKernelGGL((k_stage1_f32<K, S, 8>), dim3(grid), dim3(kWave * S), lds, stream, posm,
                        acc, n, i0, m, G, eps2, mask, jblock, items, items ? 0 : nitems,
                        static_cast<double *>(nullptr));
@@ -238,15 +239,17 @@ int launch_f32_split(const float4 *posm, double *part, int n, int i0, int m, flo
   const int per_block = kWave * K;
   const int tiles = (m + per_block - 1) / per_block;
   const size_t lds = (S > 1) ? sizeof(float) * (S - 1) * 6 * per_block : 0;
-  constexpr int kNarrow = K >= 4 ? 8 : 2;   // pair_loop_width: eight from K = 4 on
-  if (pair_loop_width(int64_t(tiles) * splits, K) == 8)
-    hipLaunchKernelGGL((k_stage1_f32<K, S, 8>), dim3(tiles, splits), dim3(kWave * S), lds,
-                       stream, posm, static_cast<float *>(nullptr), n, i0, m, 1.0f, eps2, mask,
-                       256, static_cast<const int4 *>(nullptr), 0, part);
-  else
-    hipLaunchKernelGGL((k_stage1_f32<K, S, kNarrow>), dim3(tiles, splits), dim3(kWave * S),
-                       lds, stream, posm, static_cast<float *>(nullptr), n, i0, m, 1.0f, eps2,
-                       mask, 256, static_cast<const int4 *>(nullptr), 0, part);
+  auto launch = [&](auto jb) {
+    hipLaunchKernelGGL((k_stage1_f32<K, S, decltype(jb)::value>), dim3(tiles, splits),
+                       dim3(kWave * S), lds, stream, posm, static_cast<float *>(nullptr), n, i0,
+                       m, 1.0f, eps2, mask, 256, static_cast<const int4 *>(nullptr), 0, part);
+  };
+  constexpr int kMiddle = K == 1 ? 4 : 8;   // four only with one body per lane
+  switch (pair_loop_width(int64_t(tiles) * splits, K, true)) {
+    case 2: launch(std::integral_constant<int, 2>()); break;
+    case 4: launch(std::integral_constant<int, kMiddle>()); break;
+    default: launch(std::integral_constant<int, 8>());
+  }
   return check_launch("k_stage1_f32 (j-split)");
 }
 

@@ -19,14 +19,15 @@ __device__ __forceinline__ void two_sum_fold(float &hi, float &lo, float p) {
 }
 
 // U j-bodies q[u] (indices j + u) against the K bodies of a lane, added in the order of u.
-// PRIO: their rsq together at a raised wave priority (prio_up), taken by the loop of two j-bodies
-// per step.  MI355X, without and with it: 2^18 bodies with (1, 16) 16.38 and 15.51 ms; the j-split
-// form at 16384 bodies 74.6 and 70.0 us, at 49999 605 and 569 us; the batched per-step schedule
-// on 1024 universes of 32-2048 bodies 0.147 and 0.137 ms per step.  One s_setprio pair per body
-// instead of two bodies: 15.69 ms, 70.9 us, 573 us, 0.138 ms, and 1758 against 1746 us for the
-// forward and backward of 128 such universes, whose last wavefronts run alone on their SIMDs.
-// The loop of eight serves launches of about one wavefront per SIMD, which it slows down (2000
-// bodies in 32 workgroups: a step of 36.7 against 35.7 us).
+// PRIO: their rsq together at a raised wave priority (prio_up), taken by the loops of two and of
+// four j-bodies per step.  MI355X, two per step, without and with it: 2^18 bodies with (1, 16)
+// 16.38 and 15.51 ms; the j-split form at 16384 bodies 74.6 and 70.0 us, at 49999 605 and 569 us;
+// the batched per-step schedule on 1024 universes of 32-2048 bodies 0.147 and 0.137 ms per step.
+// One s_setprio pair per body instead of two bodies: 15.69 ms, 70.9 us, 573 us, 0.138 ms, and
+// 1758 against 1746 us for the forward and backward of 128 such universes, whose last
+// wavefronts run alone on their SIMDs.  The loop of eight serves launches of about one
+// wavefront per SIMD, which it slows down (2000 bodies in 32 workgroups: a step of 36.7
+// against 35.7 us).
 template <int K, bool MASK, bool PRIO, int U>
 __device__ __forceinline__ void pairs_f32(const float4 (&q)[U], const int j,
                                           const float (&xi)[K], const float (&yi)[K],
@@ -69,13 +70,13 @@ constexpr unsigned kWaitScalar = 0xC07F;
 
 // Accumulates j in [j0, j1) into the block partials px/py/pz, JB j-bodies per loop step (one
 // s_load of JB float4).  The order of the pairs, hence the result, is the same for any JB.
-// Two per step is the faster loop in launches of many workgroups, eight in smaller ones
-// (pair_loop_width).  With two and one body per lane, the loads run one step ahead in two
-// SGPR sets a and b: each half-step waits for the set it is about to use, issues the load of
+// Two or four per step is the faster loop in launches of many workgroups, eight in smaller
+// ones (pair_loop_width).  With one body per lane these loops run their loads one step ahead in
+// two SGPR sets a and b: each half-step waits for the set it is about to use, issues the load of
 // the other set's next step and only then computes, so the scalar load's latency hides
 // behind a step of pairs (scalar loads can return out of order, so a wait is always for all
-// of them; the explicit wait comes before the next load is issued).  MI355X, Plummer:
-// 16.57-16.64 against 17.12-17.17 ms at 2^18 with (1, 16), the j-split form at 16384 bodies
+// of them; the explicit wait comes before the next load is issued).  MI355X, Plummer, two per
+// step: 16.57-16.64 against 17.12-17.17 ms at 2^18 with (1, 16), the j-split form at 16384 bodies
 // 0.079 against 0.081 ms, the batched per-step schedule on 4096 universes of 32-2048 bodies
 // 0.548 against 0.563 ms per step (before the raised priority).  It made
 // the j-split form with two bodies per lane slower (2^18: 18.7 against 17.4 ms), and with
@@ -87,7 +88,7 @@ __device__ __forceinline__ void pair_range_f32(const float4 *__restrict__ posm, 
                                                const float eps2, float (&px)[K],
                                                float (&py)[K], float (&pz)[K]) {
   int j = j0;
-  if constexpr (JB <= 2 && K == 1) {
+  if constexpr (JB <= 4 && K == 1) {
     if (j + JB <= j1) {
       float4 a[JB], b[JB];
 #pragma unroll
@@ -97,17 +98,17 @@ __device__ __forceinline__ void pair_range_f32(const float4 *__restrict__ posm, 
 #pragma unroll
         for (int u = 0; u < JB; ++u) b[u] = posm[j + JB + u];
         __builtin_amdgcn_sched_barrier(0);
-        pairs_f32<K, MASK, true>(a, j, xi, yi, zi, ii, eps2, px, py, pz);
+        pairs_f32<K, MASK, (JB <= 4)>(a, j, xi, yi, zi, ii, eps2, px, py, pz);
         // the next step of set a, or (past the end) a step in range that is not used
         const int jn = min(j + 2 * JB, j1 - JB);
         __builtin_amdgcn_s_waitcnt(kWaitScalar);
 #pragma unroll
         for (int u = 0; u < JB; ++u) a[u] = posm[jn + u];
         __builtin_amdgcn_sched_barrier(0);
-        pairs_f32<K, MASK, true>(b, j + JB, xi, yi, zi, ii, eps2, px, py, pz);
+        pairs_f32<K, MASK, (JB <= 4)>(b, j + JB, xi, yi, zi, ii, eps2, px, py, pz);
       }
       if (j + JB <= j1) {
-        pairs_f32<K, MASK, true>(a, j, xi, yi, zi, ii, eps2, px, py, pz);
+        pairs_f32<K, MASK, (JB <= 4)>(a, j, xi, yi, zi, ii, eps2, px, py, pz);
         j += JB;
       }
     }
@@ -116,12 +117,12 @@ __device__ __forceinline__ void pair_range_f32(const float4 *__restrict__ posm, 
       float4 q[JB];
 #pragma unroll
       for (int u = 0; u < JB; ++u) q[u] = posm[j + u];
-      pairs_f32<K, MASK, (JB <= 2)>(q, j, xi, yi, zi, ii, eps2, px, py, pz);
+      pairs_f32<K, MASK, (JB <= 4)>(q, j, xi, yi, zi, ii, eps2, px, py, pz);
     }
   }
   for (; j < j1; ++j) {
     const float4 q[1] = {posm[j]};
-    pairs_f32<K, MASK, (JB <= 2)>(q, j, xi, yi, zi, ii, eps2, px, py, pz);
+    pairs_f32<K, MASK, (JB <= 4)>(q, j, xi, yi, zi, ii, eps2, px, py, pz);
   }
 }
 
@@ -168,7 +169,7 @@ __device__ __forceinline__ void sum_segment_f32(const float4 *__restrict__ posm,
 // partial to part[by][c][i - i0] in FP64, and a reduce kernel sums the ranges).  Outputs are
 // rows i - i0 of (3, m) arrays; a whole universe is i0 = 0, m = n, and with items i0 = 0 and
 // m is the row stride.  The item list lets one launch cover many universes (one item per
-// universe tile).  JB: j-bodies per step of the pair loop (pair_range_f32), 2 or 8; the
+// universe tile).  JB: j-bodies per step of the pair loop (pair_range_f32), 2, 4 or 8; the
 // result does not depend on it.  red: (S - 1) * 6 * (64 * K) floats of LDS.
 template <int K, int S, int JB>
 __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm,
@@ -290,18 +291,20 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
 }
 
 // The pair loop's j-bodies per step for a launch of `workgroups` workgroups of K bodies per
-// lane.  MI355X, ms: 2^18 bodies, 4096 workgroups of (1, 16): 2 per step 17.90 against 18.43
-// for 8; 4096 universes of 32-2048 bodies in the batched per-step schedule (thousands of
-// workgroups) 0.56 against 0.62 per step; but one launch per universe (at most 32 workgroups)
-// 44.0 against 33.9 per step of all 4096, and a 4096-body universe (512 workgroups) forward +
-// adjoint 7.92 against 7.69.  From K = 4 eight per step always: the K registers of the
-// i-bodies leave no room for the shorter loop's gain.  With one body per lane the loop of two
-// loads its next step ahead, and then two per step wins from 256 workgroups on: the j-split
-// form at 4096 bodies (512 workgroups) 0.0125 against 0.0133 ms, that universe's forward +
-// adjoint 7.26-7.29 against 7.58-7.60 ms; one launch per universe of 32-2048 bodies (at
-// most 32 workgroups) still 38.3 against 34.0 ms per step of all 4096.
-inline int pair_loop_width(int64_t workgroups, int K) {
-  if (K == 1) return workgroups < 256 ? 8 : 2;
+// lane; split: the j-split form.
+//   * K = 1 from 256 workgroups: four, or two in the j-split form from 2048 workgroups.  MI355X,
+//     two and four per step: owner-computes 16384 bodies 77.4 and 71.8 us, 2^18 15.39 and
+//     15.20 ms; the batched per-step schedule on 1024 universes of 32-2048 bodies 1.387 and
+//     1.348 ms per 10 steps; forward and backward of 4096
+//     bodies over 60 steps (512 workgroups) 2.03 and 2.00 ms; but the j-split form at 16384
+//     bodies (4096 workgroups) 70.2 and 70.8 us, at 32768 248.8 and 251.2 us.  (Six: 70.8 us and 17.5 ms; eight, without loads ahead: 18.4 ms.)
+//   * Fewer workgroups: eight.  One launch per universe of 32-2048 bodies (at most 32
+//     workgroups) takes 38.3 ms per step of 4096 universes with two and 34.0 with eight.
+//   * K = 2, plain loop: two from 1024 workgroups (2^18 bodies, (2, 16): 17.9 against 18.4 ms),
+//     else eight.  From K = 4 eight always: the K registers of the i-bodies leave no room for
+//     the shorter loop's gain.
+inline int pair_loop_width(int64_t workgroups, int K, bool split) {
+  if (K == 1) return workgroups < 256 ? 8 : split && workgroups >= 2048 ? 2 : 4;
   return (K >= 4 || workgroups < 1024) ? 8 : 2;
 }
 
