@@ -30,6 +30,7 @@
 
 #include "grav_common.h"
 #include "pair_vjp.h"
+#include "stage1_f32.h"
 
 namespace grav {
 
@@ -89,12 +90,49 @@ namespace {
 
 constexpr int kLdsBytes = 160 * 1024;
 
-__device__ __forceinline__ void two_sum_fold_b(float &hi, float &lo, float p) {
-  const float s = hi + p;
-  const float bp = s - hi;
-  const float e = (hi - (s - bp)) + (p - bp);
-  hi = s;
-  lo += e;
+// Accumulates j in [j0, j1) of the LDS bodies `cur` into the block partials, JB j-bodies per
+// half-step, whose LDS broadcast reads run one half-step ahead in two register sets and whose rsq
+// are issued together at a raised priority (pairs_f32).  The order of the pairs is that of j.
+//
+// A bin's step lasts as long as its largest universe's tiles, so small batches are bound by the
+// rate of one wavefront alone (one VALU instruction per 4 cycles, plus the LDS latency that a
+// plain loop exposes), full ones by VALU issue.  MI355X, plain loop unrolled by four and this one:
+// 512 universes of 32-256 bodies over 20 steps 196 and 171 us; 1000 of 100-1024 over 10 steps
+// 1016 and 891 us; 1000 of 32-2048 over 5 steps 1778 and 1495 us.  Half-steps of four and
+// without priority: 174, 1001, 1748 us; of four with it: 180, 897, 1537 us.
+template <int KT, bool MASK>
+__device__ __forceinline__ void tile_range(const float4 *cur, int j0, int j1,
+                                           const float (&xi)[KT], const float (&yi)[KT],
+                                           const float (&zi)[KT], const int (&li)[KT],
+                                           float eps2, float (&px)[KT], float (&py)[KT],
+                                           float (&pz)[KT]) {
+  constexpr int JB = KT == 1 ? 8 : 4;
+  int j = j0;
+  if (j + JB <= j1) {
+    float4 a[JB], b[JB];
+#pragma unroll
+    for (int u = 0; u < JB; ++u) a[u] = cur[j + u];
+    for (; j + 2 * JB <= j1; j += 2 * JB) {
+#pragma unroll
+      for (int u = 0; u < JB; ++u) b[u] = cur[j + JB + u];
+      __builtin_amdgcn_sched_barrier(0);
+      pairs_f32<KT, MASK, true>(a, j, xi, yi, zi, li, eps2, px, py, pz);
+      // the next step of set a, or (past the end) a step in range that is not used
+      const int jn = min(j + 2 * JB, j1 - JB);
+#pragma unroll
+      for (int u = 0; u < JB; ++u) a[u] = cur[jn + u];
+      __builtin_amdgcn_sched_barrier(0);
+      pairs_f32<KT, MASK, true>(b, j + JB, xi, yi, zi, li, eps2, px, py, pz);
+    }
+    if (j + JB <= j1) {
+      pairs_f32<KT, MASK, true>(a, j, xi, yi, zi, li, eps2, px, py, pz);
+      j += JB;
+    }
+  }
+  for (; j < j1; ++j) {
+    const float4 q[1] = {cur[j]};
+    pairs_f32<KT, MASK, true>(q, j, xi, yi, zi, li, eps2, px, py, pz);
+  }
 }
 
 // Accelerations of KT bodies per lane (LDS indices li[k]) against j in [j0, j1) of `cur`.
@@ -109,30 +147,12 @@ __device__ __forceinline__ void tile_pairs(const float4 *cur, int j0, int j1, co
     float px[KT], py[KT], pz[KT];
 #pragma unroll
     for (int k = 0; k < KT; ++k) px[k] = py[k] = pz[k] = 0.0f;
-#pragma unroll 4
-    for (int j = jb; j < je; ++j) {
-      const float4 q = cur[j];
-#pragma unroll
-      for (int k = 0; k < KT; ++k) {
-        const float dx = q.x - xi[k];
-        const float dy = q.y - yi[k];
-        const float dz = q.z - zi[k];
-        float r2 = __builtin_fmaf(dx, dx, eps2);
-        r2 = __builtin_fmaf(dy, dy, r2);
-        r2 = __builtin_fmaf(dz, dz, r2);
-        float inv = __builtin_amdgcn_rsqf(r2);
-        if (MASK) inv = (j == li[k]) ? 0.0f : inv;
-        const float s = (q.w * inv) * (inv * inv);
-        px[k] = __builtin_fmaf(dx, s, px[k]);
-        py[k] = __builtin_fmaf(dy, s, py[k]);
-        pz[k] = __builtin_fmaf(dz, s, pz[k]);
-      }
-    }
+    tile_range<KT, MASK>(cur, jb, je, xi, yi, zi, li, eps2, px, py, pz);
 #pragma unroll
     for (int k = 0; k < KT; ++k) {
-      two_sum_fold_b(hx[k], lx[k], px[k]);
-      two_sum_fold_b(hy[k], ly[k], py[k]);
-      two_sum_fold_b(hz[k], lz[k], pz[k]);
+      two_sum_fold(hx[k], lx[k], px[k]);
+      two_sum_fold(hy[k], ly[k], py[k]);
+      two_sum_fold(hz[k], lz[k], pz[k]);
     }
   }
 }
@@ -263,6 +283,55 @@ __global__ __launch_bounds__(512) void k_batched_fused(
   }
 }
 
+// The VJP pairs of j in [j0, j1), as tile_range.  MI355X, forward and backward, plain loop
+// unrolled by two (with the forward above) and this one: 120 universes of 100-500 bodies over 8
+// steps 594 and 532 us, 200 of 64-2048 over 4 steps 4.11 and 3.81 ms; half-steps of two: 542 us
+// and 3.89 ms.
+template <int KT, bool MASK>
+__device__ __forceinline__ void vjp_tile_range(
+    const float4 *pos, const float4 *mub, int j0, int j1, const float (&xk)[KT],
+    const float (&yk)[KT], const float (&zk)[KT], const float (&mk)[KT], const float (&uxk)[KT],
+    const float (&uyk)[KT], const float (&uzk)[KT], const int (&li)[KT], float eps2,
+    float (&px)[KT], float (&py)[KT], float (&pz)[KT], float (&pg)[KT]) {
+  constexpr int JB = KT == 1 ? 4 : 2;
+  int j = j0;
+  if (j + JB <= j1) {
+    float4 qa[JB], ua[JB], qb[JB], ub[JB];
+#pragma unroll
+    for (int t = 0; t < JB; ++t) {
+      qa[t] = pos[j + t];
+      ua[t] = mub[j + t];
+    }
+    for (; j + 2 * JB <= j1; j += 2 * JB) {
+#pragma unroll
+      for (int t = 0; t < JB; ++t) {
+        qb[t] = pos[j + JB + t];
+        ub[t] = mub[j + JB + t];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      vjp_pairs<KT, MASK, true>(qa, ua, j, xk, yk, zk, mk, uxk, uyk, uzk, li, eps2, px, py, pz,
+                                pg);
+      const int jn = min(j + 2 * JB, j1 - JB);
+#pragma unroll
+      for (int t = 0; t < JB; ++t) {
+        qa[t] = pos[jn + t];
+        ua[t] = mub[jn + t];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      vjp_pairs<KT, MASK, true>(qb, ub, j + JB, xk, yk, zk, mk, uxk, uyk, uzk, li, eps2, px, py,
+                                pz, pg);
+    }
+    if (j + JB <= j1) {
+      vjp_pairs<KT, MASK, true>(qa, ua, j, xk, yk, zk, mk, uxk, uyk, uzk, li, eps2, px, py, pz,
+                                pg);
+      j += JB;
+    }
+  }
+  for (; j < j1; ++j)
+    vjp_pair<KT, MASK>(pos[j], mub[j], j, xk, yk, zk, mk, uxk, uyk, uzk, li, eps2, px, py, pz,
+                       pg);
+}
+
 // Backward over `steps` steps (t = steps-1 .. 0) of every universe of the bin, reading the
 // positions each forward step used from traj[t].  Per step: trajectory positions -> LDS,
 // owners form mu = nu + h rho (FP64, HBM) and take their universe's largest exponent
@@ -390,16 +459,12 @@ __global__ __launch_bounds__(512) void k_batched_adjoint(
           float px[KT], py[KT], pz[KT], pg[KT];
 #pragma unroll
           for (int k = 0; k < KT; ++k) px[k] = py[k] = pz[k] = pg[k] = 0.0f;
-          if (part == 1) {
-            for (int j = jb; j < je; ++j)
-              vjp_pair<KT, true>(pos[j], mub[j], j, xk, yk, zk, mk, uxk, uyk, uzk, li, eps2, px,
-                                 py, pz, pg);
-          } else {
-#pragma unroll 2
-            for (int j = jb; j < je; ++j)
-              vjp_pair<KT, false>(pos[j], mub[j], j, xk, yk, zk, mk, uxk, uyk, uzk, li, eps2,
-                                  px, py, pz, pg);
-          }
+          if (part == 1)
+            vjp_tile_range<KT, true>(pos, mub, jb, je, xk, yk, zk, mk, uxk, uyk, uzk, li, eps2,
+                                     px, py, pz, pg);
+          else
+            vjp_tile_range<KT, false>(pos, mub, jb, je, xk, yk, zk, mk, uxk, uyk, uzk, li, eps2,
+                                      px, py, pz, pg);
 #pragma unroll
           for (int k = 0; k < KT; ++k) {
             two_sum_acc(hi[0][k], lo[0][k], px[k]);
