@@ -9,7 +9,9 @@
 //   * per 64-body chunk of block gamma, every lane holds K bodies of block beta in registers and
 //     one j-body (x, y, z, m and its three accumulators) that moves one lane per step with a
 //     DPP wave rotate; after 64 steps each lane has met every j-body of the chunk and the
-//     j-bodies are back in their home lanes.  A pair costs 16 VALU ops + 1 v_rsq_f32 for two
+//     j-bodies are back in their home lanes.  A step's K j-side terms are summed first and added
+//     to the accumulator as it moves (v_add_f32 with a DPP operand), so that a chain of FP32
+//     additions is 64 long, not 64*K.  A pair costs 16 VALU ops + 1 v_rsq_f32 for two
 //     directed interactions, plus 7 rotations per K pairs;
 //   * i-side sums fold into FP32 (hi, lo) TwoSum pairs once per chunk; the W wavefronts' j-side
 //     sums of a chunk are added through double-buffered LDS and written as one partial;
@@ -18,6 +20,8 @@
 //     the rows are walked in slabs whose partials fit the caller's workspace: after every slab
 //     a fold kernel adds its partials into each body's FP64 sum in a fixed order, so the
 //     workspace is bounded (one slab down to one row) and the result is deterministic;
+//   * one universe of middle size (sizes at kUnitsFrom) has the work of all rows, the pairs inside
+//     the blocks among it, divided evenly among workgroups that are resident at once;
 //   * batched universes list their block pairs as items, and one reduction kernel adds every
 //     body's diagonal-block sum and partials in a fixed order in FP64.
 #include <algorithm>
@@ -51,24 +55,96 @@ __device__ __forceinline__ float4 load_or_far(const float4 *__restrict__ posm, i
   return b < n ? posm[b] : make_float4(kFar, kFar, kFar, 0.0f);
 }
 
-// One block pair (beta, gamma) for one workgroup: its wavefronts hold K block-beta bodies per
-// lane (xi..zi, the masses negated in mn) and take the K*W chunks of 64 block-gamma bodies from jb0 (bodies at or past
-// jend load as far, massless padding).  The i-side sums of every chunk fold into the TwoSum
-// pairs (hx, lx) .. (hz, lz), which the caller may carry over several gamma blocks; the j-side
-// sums of a chunk, added over the W wavefronts through the double-buffered LDS `red` (buffer
-// chunk & 1, chunk counting on across calls), go to pj[c * IB + jc * 64 + l], 3 * IB floats.
+// One 64-body chunk (a lane's j-body q) against the K bodies of a lane: 64 rotations, after which
+// every j-body and its sums are back in their home lane.  The i-side sums are added to p, the
+// j-side sums (without OWN) to aj.  mn: the i-bodies' masses, negated.  OWN: the chunk is one
+// of the i-bodies' own block; only the i side is summed (the other order of each pair has its
+// own lane), and the self pairs of sub-chunk kself, met before the first rotation, are left out.
 //
 // Bound by the issue of VALU instructions: per pair 16 FP32, one v_rsq_f32 and 7/K DPP moves,
 // about 44 + 30 / K cycles per SIMD if every two FP32 instructions of different wavefronts go
 // side by side.  For that the rsq (of G = 2 pairs together) and the DPP moves are issued at a
 // raised priority (prio_up), eps2 sits in a VGPR and the masses come negated, so that the j side
-// needs no negating (8-byte) FMA.  MI355X, (8, 2), before and after: 2^18 bodies 13.40 and
+// needs no negating (8-byte) FMA.  Adding the step's j-side sum in the move itself leaves the time
+// as it was (2^18 11.36 against 11.43 ms on one box) and about halves the error against 64 bits
+// (Plummer, eps 1e-3: 20000 bodies 1.5e-7 to 7e-8, 65536 9.3e-8 to 5.7e-8).  MI355X, (8, 2), before and after: 2^18 bodies 13.40 and
 // 11.13 ms (65.7 to 54 cycles per pair of bodies and wavefront), 2^17 3.44 and 2.87 ms; (4, 2) at
 // 49999 bodies 0.652 and 0.496 ms.  G = 4 pairs need 138 VGPRs with K = 8 for 11.05 ms, G = 1
 // takes 11.19 ms.  Measured and not kept: the j-bodies read from LDS instead of rotated (3 DPP
 // moves per step instead of 7) is no faster once the moves have priority (2.95 against 2.86 ms
 // at 2^17), and temporaries pinned to registers of alternating parity (an FMA whose three
 // operands have register numbers of one parity issues alone) gain 1 %.
+template <int K, bool OWN>
+__device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const float eps2,
+                                          const float (&xi)[K], const float (&yi)[K],
+                                          const float (&zi)[K], const float (&mn)[K],
+                                          float (&px)[K], float (&py)[K], float (&pz)[K],
+                                          float &ajx, float &ajy, float &ajz) {
+  constexpr int G = 2;
+  float xj = q.x, yj = q.y, zj = q.z, mj = q.w;
+  // not unrolled: the body of one step ran 4 % faster than that of two steps (2^18: 13.36
+  // against 13.96 ms, before the raised priority)
+#pragma unroll 1
+  for (int t = 0; t < kWave; ++t) {
+    float tx = 0.0f, ty = 0.0f, tz = 0.0f;   // the j-body's sums over the K pairs of this step
+#pragma unroll
+    for (int k = 0; k < K; k += G) {
+      float dx[G], dy[G], dz[G], inv[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        dx[g] = xj - xi[k + g];
+        dy[g] = yj - yi[k + g];
+        dz[g] = zj - zi[k + g];
+        float r2 = __builtin_fmaf(dx[g], dx[g], eps2);
+        r2 = __builtin_fmaf(dy[g], dy[g], r2);
+        inv[g] = __builtin_fmaf(dz[g], dz[g], r2);
+      }
+      prio_up();
+#pragma unroll
+      for (int g = 0; g < G; ++g) inv[g] = __builtin_amdgcn_rsqf(inv[g]);
+      prio_down();
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        if (OWN && t == 0 && k + g == kself) inv[g] = 0.0f;
+        const float inv3 = inv[g] * (inv[g] * inv[g]);
+        const float si = mj * inv3;
+        px[k + g] = __builtin_fmaf(dx[g], si, px[k + g]);
+        py[k + g] = __builtin_fmaf(dy[g], si, py[k + g]);
+        pz[k + g] = __builtin_fmaf(dz[g], si, pz[k + g]);
+        if constexpr (!OWN) {
+          const float sj = mn[k + g] * inv3;
+          tx = k + g == 0 ? dx[g] * sj : __builtin_fmaf(dx[g], sj, tx);
+          ty = k + g == 0 ? dy[g] * sj : __builtin_fmaf(dy[g], sj, ty);
+          tz = k + g == 0 ? dz[g] * sj : __builtin_fmaf(dz[g], sj, tz);
+        }
+      }
+    }
+    prio_up();
+    if constexpr (!OWN) {
+      // the sums so far come from the lane that held this j-body in the step before
+      ajx = rot1(ajx) + tx;
+      ajy = rot1(ajy) + ty;
+      ajz = rot1(ajz) + tz;
+    }
+    xj = rot1(xj);
+    yj = rot1(yj);
+    zj = rot1(zj);
+    mj = rot1(mj);
+    prio_down();
+  }
+  if constexpr (!OWN) {   // home
+    ajx = rot1(ajx);
+    ajy = rot1(ajy);
+    ajz = rot1(ajz);
+  }
+}
+
+// One block pair (beta, gamma) for one workgroup: its wavefronts hold K block-beta bodies per
+// lane (xi..zi, the masses negated in mn) and take the K*W chunks of 64 block-gamma bodies from
+// jb0 (bodies at or past jend load as far, massless padding).  The i-side sums of every chunk fold into the TwoSum
+// pairs (hx, lx) .. (hz, lz), which the caller may carry over several gamma blocks; the j-side
+// sums of a chunk, added over the W wavefronts through the double-buffered LDS `red` (buffer
+// chunk & 1, chunk counting on across calls), go to pj[c * IB + jc * 64 + l], 3 * IB floats.
 template <int K, int W>
 __device__ __forceinline__ void sym_block_pair(const float4 *__restrict__ posm, int jb0,
                                                int jend, float eps2, const float (&xi)[K],
@@ -80,66 +156,21 @@ __device__ __forceinline__ void sym_block_pair(const float4 *__restrict__ posm, 
                                                float (&red)[2][W][3][kWave], int &chunk,
                                                int lane, int wave) {
   constexpr int IB = kWave * K * W;
-  constexpr int G = 2;
   for (int jc = 0; jc < K * W; ++jc, ++chunk) {
     const float4 q = load_or_far(posm, jb0 + jc * kWave + lane, jend);
-    float xj = q.x, yj = q.y, zj = q.z, mj = q.w;
     float ajx = 0.0f, ajy = 0.0f, ajz = 0.0f;
     float px[K], py[K], pz[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) px[k] = py[k] = pz[k] = 0.0f;
-    // not unrolled: the body of one step ran 4 % faster than that of two steps (2^18: 13.36
-    // against 13.96 ms, before the raised priority)
-#pragma unroll 1
-    for (int t = 0; t < kWave; ++t) {
-#pragma unroll
-      for (int k = 0; k < K; k += G) {
-        float dx[G], dy[G], dz[G], inv[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          dx[g] = xj - xi[k + g];
-          dy[g] = yj - yi[k + g];
-          dz[g] = zj - zi[k + g];
-          float r2 = __builtin_fmaf(dx[g], dx[g], eps2);
-          r2 = __builtin_fmaf(dy[g], dy[g], r2);
-          inv[g] = __builtin_fmaf(dz[g], dz[g], r2);
-        }
-        prio_up();
-#pragma unroll
-        for (int g = 0; g < G; ++g) inv[g] = __builtin_amdgcn_rsqf(inv[g]);
-        prio_down();
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const float inv3 = inv[g] * (inv[g] * inv[g]);
-          const float si = mj * inv3;
-          const float sj = mn[k + g] * inv3;
-          px[k + g] = __builtin_fmaf(dx[g], si, px[k + g]);
-          py[k + g] = __builtin_fmaf(dy[g], si, py[k + g]);
-          pz[k + g] = __builtin_fmaf(dz[g], si, pz[k + g]);
-          ajx = __builtin_fmaf(dx[g], sj, ajx);
-          ajy = __builtin_fmaf(dy[g], sj, ajy);
-          ajz = __builtin_fmaf(dz[g], sj, ajz);
-        }
-      }
-      prio_up();
-      xj = rot1(xj);
-      yj = rot1(yj);
-      zj = rot1(zj);
-      mj = rot1(mj);
-      ajx = rot1(ajx);
-      ajy = rot1(ajy);
-      ajz = rot1(ajz);
-      prio_down();
-    }
+    sym_chunk<K, false>(q, -1, eps2, xi, yi, zi, mn, px, py, pz, ajx, ajy, ajz);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       two_sum_sym(hx[k], lx[k], px[k]);
       two_sum_sym(hy[k], ly[k], py[k]);
       two_sum_sym(hz[k], lz[k], pz[k]);
     }
-    // After 64 rotations every j-body and its sums are back in their home lane.  The next
-    // chunk writes the other buffer, and a wave can only come back to this one after the
-    // next chunk's barrier, which every wave reaches after it has read this one.
+    // The next chunk writes the other buffer, and a wave can only come back to this one after
+    // the next chunk's barrier, which every wave reaches after it has read this one.
     float(*r)[3][kWave] = red[chunk & 1];
     r[wave][0][lane] = ajx;
     r[wave][1][lane] = ajy;
@@ -314,6 +345,49 @@ __device__ __forceinline__ double4 load_or_far_d(const double4 *__restrict__ pos
   return b < n ? posm[b] : make_double4(1e30, 1e30, 1e30, 0.0);
 }
 
+// sym_chunk in FP64 (mi: the i-bodies' masses).
+template <int K, bool OWN>
+__device__ __forceinline__ void sym_chunk(const double4 q, const int kself, const double eps2,
+                                          const double (&xi)[K], const double (&yi)[K],
+                                          const double (&zi)[K], const double (&mi)[K],
+                                          double (&px)[K], double (&py)[K], double (&pz)[K],
+                                          double &ajx, double &ajy, double &ajz) {
+  double xj = q.x, yj = q.y, zj = q.z, mj = q.w;
+  for (int t = 0; t < kWave; ++t) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const double dx = xj - xi[k];
+      const double dy = yj - yi[k];
+      const double dz = zj - zi[k];
+      double r2 = __builtin_fma(dx, dx, eps2);
+      r2 = __builtin_fma(dy, dy, r2);
+      r2 = __builtin_fma(dz, dz, r2);
+      double inv = rsqrt_nr64(r2);
+      if (OWN && t == 0 && k == kself) inv = 0.0;
+      const double inv3 = inv * (inv * inv);
+      const double si = mj * inv3;
+      px[k] = __builtin_fma(dx, si, px[k]);
+      py[k] = __builtin_fma(dy, si, py[k]);
+      pz[k] = __builtin_fma(dz, si, pz[k]);
+      if constexpr (!OWN) {
+        const double sj = mi[k] * inv3;
+        ajx = __builtin_fma(-dx, sj, ajx);
+        ajy = __builtin_fma(-dy, sj, ajy);
+        ajz = __builtin_fma(-dz, sj, ajz);
+      }
+    }
+    xj = rot1d(xj);
+    yj = rot1d(yj);
+    zj = rot1d(zj);
+    mj = rot1d(mj);
+    if constexpr (!OWN) {
+      ajx = rot1d(ajx);
+      ajy = rot1d(ajy);
+      ajz = rot1d(ajz);
+    }
+  }
+}
+
 // A segment of the FP64 form (the row-segment scheme of k_sym_segments, FP64 sums).
 template <int K, int W>
 __global__ __launch_bounds__(kWave *W) void k_sym_segments_f64(const double4 *__restrict__ posm,
@@ -349,38 +423,9 @@ __global__ __launch_bounds__(kWave *W) void k_sym_segments_f64(const double4 *__
     double *pj = p_j + ((local << lg) + (gamma - g0)) * (3 * IB);
     for (int jc = 0; jc < K * W; ++jc, ++chunk) {
       const double4 q = load_or_far_d(posm, gamma * IB + jc * kWave + lane, n);
-      double xj = q.x, yj = q.y, zj = q.z, mj = q.w;
       double ajx = 0.0, ajy = 0.0, ajz = 0.0;
-      for (int t = 0; t < kWave; ++t) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          const double dx = xj - xi[k];
-          const double dy = yj - yi[k];
-          const double dz = zj - zi[k];
-          double r2 = __builtin_fma(dx, dx, eps2);
-          r2 = __builtin_fma(dy, dy, r2);
-          r2 = __builtin_fma(dz, dz, r2);
-          const double inv = rsqrt_nr64(r2);
-          const double inv3 = inv * (inv * inv);
-          const double si = mj * inv3;
-          const double sj = mi[k] * inv3;
-          px[k] = __builtin_fma(dx, si, px[k]);
-          py[k] = __builtin_fma(dy, si, py[k]);
-          pz[k] = __builtin_fma(dz, si, pz[k]);
-          ajx = __builtin_fma(-dx, sj, ajx);
-          ajy = __builtin_fma(-dy, sj, ajy);
-          ajz = __builtin_fma(-dz, sj, ajz);
-        }
-        xj = rot1d(xj);
-        yj = rot1d(yj);
-        zj = rot1d(zj);
-        mj = rot1d(mj);
-        ajx = rot1d(ajx);
-        ajy = rot1d(ajy);
-        ajz = rot1d(ajz);
-      }
-      // After 64 rotations every j-body and its sums are back in their home lane; buffers
-      // alternate with the chunk count as in sym_block_pair.
+      sym_chunk<K, false>(q, -1, eps2, xi, yi, zi, mi, px, py, pz, ajx, ajy, ajz);
+      // buffers alternate with the chunk count as in sym_block_pair
       double(*r)[3][kWave] = red[chunk & 1];
       r[wave][0][lane] = ajx;
       r[wave][1][lane] = ajy;
@@ -403,6 +448,236 @@ __global__ __launch_bounds__(kWave *W) void k_sym_segments_f64(const double4 *__
     p_i[base + IB + bl] = py[k];
     p_i[base + 2 * IB + bl] = pz[k];
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// One universe, balanced form.  The work of row beta is a list of units: the 64-body chunks
+// c = beta*K*W .. nc-1 (nc chunks in all), first the K*W chunks of block beta itself (i side
+// only: every ordered pair of the block once) and then those of the later blocks (both sides).
+// The units of all rows, numbered row-major, are divided evenly among `groups` workgroups, all
+// resident at once: group g takes units [g*U/groups, (g+1)*U/groups).  It keeps the i-side sums
+// of a row in registers while it stays in that row and writes them once, to slot g + beta of
+// p_i (3*IB values; g + beta is unique to the pair); the j-side sums of a unit go to p_j at block
+// pair (beta, gamma) as in the row-segment form.  A fold kernel adds every body's partials in
+// FP64 in a fixed order.
+
+constexpr int kCus = 256;   // compute units of an MI355X
+
+// First unit of row beta; a row's units end where the next row's begin.
+__host__ __device__ inline int64_t unit_row(int64_t beta, int64_t nc, int kw) {
+  return beta * nc - kw * (beta * (beta - 1) / 2);
+}
+// The group that holds unit u: the largest g with g*U/groups <= u.
+__host__ __device__ inline int64_t unit_group(int64_t u, int64_t groups, int64_t U) {
+  return ((u + 1) * groups - 1) / U;
+}
+// Block pairs of the rows before beta.
+__host__ __device__ inline int64_t pair_row(int64_t beta, int64_t nb) {
+  return beta * (nb - 1) - beta * (beta - 1) / 2;
+}
+
+// The i-side sums of K bodies per lane: FP32 chunk sums folded into TwoSum pairs, FP64 as is.
+template <typename T, int K>
+struct ISum;
+template <int K>
+struct ISum<float, K> {
+  float h[3][K], l[3][K];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int k = 0; k < K; ++k) h[c][k] = l[c][k] = 0.0f;
+  }
+  template <bool OWN>
+  __device__ __forceinline__ void chunk(const float4 q, int kself, float eps2,
+                                        const float (&x)[4][K], float (&aj)[3]) {
+    float px[K], py[K], pz[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) px[k] = py[k] = pz[k] = 0.0f;
+    sym_chunk<K, OWN>(q, kself, eps2, x[0], x[1], x[2], x[3], px, py, pz, aj[0], aj[1], aj[2]);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      two_sum_sym(h[0][k], l[0][k], px[k]);
+      two_sum_sym(h[1][k], l[1][k], py[k]);
+      two_sum_sym(h[2][k], l[2][k], pz[k]);
+    }
+  }
+  __device__ __forceinline__ float get(int c, int k) const { return h[c][k] + l[c][k]; }
+};
+template <int K>
+struct ISum<double, K> {
+  double p[3][K];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int k = 0; k < K; ++k) p[c][k] = 0.0;
+  }
+  template <bool OWN>
+  __device__ __forceinline__ void chunk(const double4 q, int kself, double eps2,
+                                        const double (&x)[4][K], double (&aj)[3]) {
+    sym_chunk<K, OWN>(q, kself, eps2, x[0], x[1], x[2], x[3], p[0], p[1], p[2], aj[0], aj[1],
+                      aj[2]);
+  }
+  __device__ __forceinline__ double get(int c, int k) const { return p[c][k]; }
+};
+
+__device__ __forceinline__ float4 body_or_far(const float4 *__restrict__ posm, int b, int n) {
+  return load_or_far(posm, b, n);
+}
+__device__ __forceinline__ double4 body_or_far(const double4 *__restrict__ posm, int b, int n) {
+  return load_or_far_d(posm, b, n);
+}
+__device__ __forceinline__ float uniform_operand(float x) { return in_vgpr(x); }
+__device__ __forceinline__ double uniform_operand(double x) { return x; }
+// The sign of the i-bodies' masses that sym_chunk takes.
+template <typename T>
+constexpr T kMassSign = sizeof(T) == 4 ? T(-1) : T(1);
+
+// Bound by VALU issue (sym_chunk).  Against the row segments: no block-diagonal pass of its own
+// (FP64, 40000 bodies: 23 of 690 us), no last round of workgroups that leaves half the compute
+// units idle, i-side partials once per group and row.  FP32 65536 bodies: 744 us = 55 cycles per
+// unordered pair and SIMD, of 50 that the loop can reach; 32768: 200 us, 59 cycles.
+template <typename T, typename T4, int K, int W>
+__global__ __launch_bounds__(kWave *W) void k_sym_units(const T4 *__restrict__ posm, int n,
+                                                         int nb, int nc, int64_t units, T eps2,
+                                                         T *__restrict__ p_i,
+                                                         T *__restrict__ p_j) {
+  constexpr int KW = K * W, IB = kWave * KW;
+  __shared__ T red[2][W][3][kWave];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  // workgroups b, b + kCus, b + 2*kCus, .. go to one compute unit: they take neighbouring ranges, so
+  // that the units of a compute unit differ by at most one
+  const int64_t groups = gridDim.x;
+  const int64_t g = groups % kCus == 0
+                        ? int64_t(blockIdx.x % kCus) * (groups / kCus) + blockIdx.x / kCus
+                        : blockIdx.x;
+  int64_t u = g * units / groups;
+  const int64_t u_end = (g + 1) * units / groups;
+  int beta = 0;
+  {  // the row of unit u: the last one that begins at or before it
+    int lo = 0, hi = nb - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (unit_row(mid, nc, KW) <= u)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    beta = lo;
+  }
+  const T eps2v = uniform_operand(eps2);
+  int buf = 0;
+  for (; u < u_end; ++beta) {
+    const int64_t r0 = unit_row(beta, nc, KW), r1 = unit_row(beta + 1, nc, KW);
+    int c = beta * KW + static_cast<int>(u - r0);
+    const int c_end = beta * KW + static_cast<int>((u_end < r1 ? u_end : r1) - r0);
+    u += c_end - c;
+    T x[4][K];
+    ISum<T, K> sum;
+    sum.clear();
+    const int i0 = beta * IB + wave * (K * kWave);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const T4 p = body_or_far(posm, i0 + k * kWave + lane, n);
+      x[0][k] = p.x;
+      x[1][k] = p.y;
+      x[2][k] = p.z;
+      x[3][k] = kMassSign<T> * p.w;
+    }
+    T aj[3] = {0, 0, 0};
+    const int own_end = min(c_end, (beta + 1) * KW);
+    T4 q = body_or_far(posm, c * kWave + lane, n), qn;   // each chunk is loaded one ahead
+#pragma unroll 1
+    for (; c < own_end; ++c, q = qn) {
+      qn = body_or_far(posm, (c + 1) * kWave + lane, n);
+      sum.template chunk<true>(q, c - beta * KW - wave * K, eps2v, x, aj);
+    }
+#pragma unroll 1
+    for (; c < c_end; ++c, q = qn) {
+      qn = body_or_far(posm, (c + 1) * kWave + lane, n);
+      aj[0] = aj[1] = aj[2] = 0;
+      sum.template chunk<false>(q, -1, eps2v, x, aj);
+      const int gamma = c / KW;
+      T *pj = p_j + (pair_row(beta, nb) + (gamma - beta - 1)) * (3 * IB) +
+              (c - gamma * KW) * kWave;
+      if constexpr (W == 1) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) pj[q * IB + lane] = aj[q];
+      } else {
+        // two buffers: a wave writes one again only after the other's barrier, which every
+        // wave reaches after it has read this one
+        T(*r)[3][kWave] = red[buf];
+        buf ^= 1;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) r[wave][q][lane] = aj[q];
+        __syncthreads();
+        for (int t = threadIdx.x; t < 3 * kWave; t += kWave * W) {
+          const int q = t / kWave, l = t % kWave;
+          T v = 0;
+#pragma unroll
+          for (int w = 0; w < W; ++w) v += r[w][q][l];
+          pj[q * IB + l] = v;
+        }
+      }
+    }
+    T *out = p_i + (g + beta) * (3 * IB) + wave * (K * kWave) + lane;
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int k = 0; k < K; ++k) out[q * IB + k * kWave] = sum.get(q, k);
+  }
+}
+
+// acc = G * (every partial of the body) of the balanced form, or with `sums` the unscaled FP64
+// sum itself, for the 64 bodies of chunk blockIdx.x: 3 * 64 (component, body) columns in kFoldSlices slices of the body's partials
+// (its row's i-side slots, then its j-side partials from the rows before), each slice added in
+// order in FP64, the slices' sums in order.  A wave keeps eight coalesced reads in flight.
+constexpr int kFoldSlices = 4;
+template <typename T>
+__global__ __launch_bounds__(3 * kWave *kFoldSlices) void k_sym_units_fold(
+    T *__restrict__ acc, double *__restrict__ sums, const T *__restrict__ p_i,
+    const T *__restrict__ p_j, int n, int nb, int nc, int kw, int64_t units, int64_t groups, double G) {
+  __shared__ double part[kFoldSlices][3 * kWave];
+  const int ib = kw * kWave;
+  const size_t stride = static_cast<size_t>(3) * ib;
+  const int chunk = blockIdx.x, row = chunk / kw;
+  const int col = threadIdx.x % (3 * kWave), slice = threadIdx.x / (3 * kWave);
+  const int comp = col / kWave, lane = col % kWave;
+  const size_t at = static_cast<size_t>(comp) * ib + (chunk - row * kw) * kWave + lane;
+  const int64_t g0 = unit_group(unit_row(row, nc, kw), groups, units);
+  const int64_t g1 = unit_group(unit_row(row + 1, nc, kw) - 1, groups, units);
+  const int ni = static_cast<int>(g1 - g0) + 1, m = ni + row;
+  const T *qi = p_i + (g0 + row) * stride + at;
+  // partial t: i-side slot t, then the j side of block pair (t - ni, row)
+  auto load = [&](int t) {
+    if (t < ni) return qi[static_cast<size_t>(t) * stride];
+    const int beta = t - ni;
+    return p_j[(pair_row(beta, nb) + (row - beta - 1)) * stride + at];
+  };
+  int t = static_cast<int>(static_cast<int64_t>(slice) * m / kFoldSlices);
+  const int t_end = static_cast<int>(static_cast<int64_t>(slice + 1) * m / kFoldSlices);
+  double s = 0.0;
+  for (; t + 8 <= t_end; t += 8) {
+    T v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = load(t + k);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += v[k];
+  }
+  for (; t < t_end; ++t) s += load(t);
+  part[slice][col] = s;
+  __syncthreads();
+  if (slice != 0) return;
+#pragma unroll
+  for (int k = 1; k < kFoldSlices; ++k) s += part[k][col];
+  const int b = chunk * kWave + lane;
+  if (b >= n) return;
+  if (sums != nullptr)
+    sums[static_cast<size_t>(comp) * n + b] = s;
+  else
+    acc[static_cast<size_t>(comp) * n + b] = static_cast<T>(G * s);
 }
 
 // Fold of one slab into every body's FP64 sum s, one thread per (body, component),
@@ -676,6 +951,61 @@ int sym_run(const SymPlan &P, const SymRange &R, int n, T *acc, double *sums, do
   return GRAV_OK;
 }
 
+// The balanced form of n bodies in blocks of 64*K*W: `groups` workgroups of W wavefronts.
+struct UnitPlan {
+  int nb, nc, kw;
+  int64_t units, groups, j_bytes;
+};
+
+// Ten workgroups per compute unit, five of which are resident at once (FP32, 84 VGPRs): the
+// second half is dispatched as the first ends, which evens out what oldest-first issue leaves
+// uneven.  FP32 stage 1 with 4, 5, 10 and 16 per compute unit, us: 40000 bodies 300, 300, 291,
+// 291; 65536 773, 762, 744, 746; 100000 1788, 1773, 1696, 1690.
+constexpr int64_t kUnitGroups = 10 * kCus;
+
+// Where the default shape (named or as (0, 0)) takes the balanced form, in blocks of 1024 bodies
+// (K 4, W 4) whatever that shape is, if its workspace holds it.  Below, only one group per compute unit fits the workspace (FP32
+// 18500 bodies: 128 us against 124 for the row segments); above, a static division into few
+// thousand groups loses to the row segments, whose workgroups are dispatched as they end.
+// Stage 1, us, row segments in their default shape and this form (in parentheses the j-split
+// form): FP32 19000 bodies 124 and 81 (92), 20480 124 and 92 (104), 32768 221 and 200 (251), 49999
+// 479 and 450 (577), 65536 922 and 744 (971), 100000 1795 and 1709, 114687 2297 and 2237, 131072
+// 2854 and 2862; FP64 9000 74 and 50 (52), 12288 100 and 77 (88), 20000 202 and 168 (227), 40000
+// 690 and 592 (876), 60000 1332 and 1297.
+constexpr int64_t kUnitsFrom = 18945, kUnitsTo = 114688;
+constexpr int64_t kUnitsFromF64 = 8961, kUnitsToF64 = 65536;
+
+// groups: kUnitGroups, or the multiple of kCus below it whose i-side slots fit the workspace;
+// 0: the form does not fit.
+UnitPlan unit_plan(int64_t n, int K, int W, int64_t elem, int64_t workspace_bytes) {
+  UnitPlan P{};
+  P.kw = K * W;
+  const int64_t ib = int64_t(kWave) * P.kw, slot = 3 * ib * elem;
+  P.nb = static_cast<int>((n + ib - 1) / ib);
+  P.nc = static_cast<int>((n + kWave - 1) / kWave);
+  P.units = unit_row(P.nb, P.nc, P.kw);
+  P.j_bytes = int64_t(P.nb) * (P.nb - 1) / 2 * slot;
+  const int64_t room = (workspace_bytes - P.j_bytes) / slot - P.nb;
+  const int64_t g = std::min({kUnitGroups, room, P.units});
+  P.groups = std::max<int64_t>(g / kCus * kCus, 0);
+  return P;
+}
+
+template <typename T, typename T4, int K, int W>
+int sym_units_run(const T4 *posm, T *acc, double *sums, int n, const UnitPlan &P, double G,
+                  T eps2, void *ws, hipStream_t s) {
+  T *p_j = static_cast<T *>(ws);
+  T *p_i = reinterpret_cast<T *>(static_cast<char *>(ws) + P.j_bytes);
+  hipLaunchKernelGGL((k_sym_units<T, T4, K, W>), dim3(static_cast<unsigned>(P.groups)),
+                     dim3(kWave * W), 0, s, posm, n, P.nb, P.nc, P.units, eps2, p_i, p_j);
+  const int rc = check_launch("k_sym_units");
+  if (rc != GRAV_OK) return rc;
+  hipLaunchKernelGGL((k_sym_units_fold<T>), dim3(static_cast<unsigned>(P.nc)),
+                     dim3(3 * kWave * kFoldSlices), 0, s, acc, sums, p_i, p_j, n, P.nb, P.nc,
+                     P.kw, P.units, P.groups, G);
+  return check_launch("k_sym_units_fold");
+}
+
 // Share `share` of `shares` when the symmetric form is divided among GPUs by rows of block
 // pairs.  Row beta holds nb - 1 - beta block pairs, so rows beta and nb - 2 - beta together
 // hold nb: these row couples (the middle row alone when the row count is odd) are the units,
@@ -747,6 +1077,13 @@ void sym_shape(int64_t n, int &K, int &W) {
   }
 }
 
+// Whether n bodies in shape (K, W) go through the balanced form (kUnitsFrom).
+bool sym_units_shape(int64_t n, int K, int W) {
+  int K0 = 0, W0 = 0;
+  sym_shape(n, K0, W0);
+  return K == K0 && W == W0 && n >= kUnitsFrom && n < kUnitsTo;
+}
+
 template <int K, int W>
 int launch_segments(const float4 *posm, int n, const SymPlan &P, const SegSpan &sp, int nseg,
                     float eps2, float *pi, float *pj, hipStream_t s) {
@@ -767,6 +1104,12 @@ void sym_shape_f64(int64_t n, int &K, int &W) {
     K = n < 24576 ? 2 : 4;
     W = n < 65536 ? 2 : 4;
   }
+}
+
+bool sym_units_shape_f64(int64_t n, int K, int W) {
+  int K0 = 0, W0 = 0;
+  sym_shape_f64(n, K0, W0);
+  return K == K0 && W == W0 && n >= kUnitsFromF64 && n < kUnitsToF64;
 }
 
 template <int K, int W>
@@ -888,6 +1231,12 @@ int grav_stage1_sym_f32(const void *posm, void *acc, int64_t n, double G, double
   const int mask = eps == 0.0 ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const float4 *p = static_cast<const float4 *>(posm);
+  if (sym_units_shape(n, K, W)) {
+    const UnitPlan U = unit_plan(n, 4, 4, 4, workspace_bytes);
+    if (U.groups > 0)
+      return sym_units_run<float, float4, 4, 4>(p, static_cast<float *>(acc), nullptr, nn, U, G,
+                                                eps2, workspace, s);
+  }
   // pairs inside each block: owner-computes over the blocks of IB bodies (a multiple of 256)
   auto diag_fn = [&](float *diag) {
     return stage1_f32_launch(p, diag, nn, 1.0f, eps2, mask, 4, 4, 256, nullptr, P.ib, s);
@@ -953,6 +1302,12 @@ int grav_stage1_sym_f32_share(const void *posm, void *sums64, int64_t n, double 
   const int mask = eps == 0.0 ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const float4 *p = static_cast<const float4 *>(posm);
+  if (shares == 1 && sym_units_shape(n, K, W)) {   // the one-GPU form
+    const UnitPlan U = unit_plan(n, 4, 4, 4, workspace_bytes);
+    if (U.groups > 0)
+      return sym_units_run<float, float4, 4, 4>(p, nullptr, static_cast<double *>(sums64), nn, U,
+                                                1.0, eps2, workspace, s);
+  }
   const int i0 = R.d_lo * P.ib;
   const int m = std::min(nn, R.d_hi * P.ib) - i0;
   auto diag_fn = [&](float *diag) {
@@ -1018,6 +1373,12 @@ int grav_stage1_sym_f64(const void *posm64, void *acc64, int64_t n, double G, do
   const int mask = eps == 0.0 ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const double4 *p = static_cast<const double4 *>(posm64);
+  if (sym_units_shape_f64(n, K, W)) {
+    const UnitPlan U = unit_plan(n, 4, 4, 8, workspace_bytes);
+    if (U.groups > 0)
+      return sym_units_run<double, double4, 4, 4>(p, static_cast<double *>(acc64), nullptr, nn,
+                                                  U, G, eps2, workspace, s);
+  }
   auto diag_fn = [&](double *diag) {
     return stage1_f64_launch(p, diag, nn, 1.0, eps2, mask, P.ib, s);
   };

@@ -96,17 +96,16 @@ _workspaces = {}
 
 # Form thresholds, from stage-1 times on Plummer spheres on an MI355X.  FP32: one launch
 # (owner-computes) beats the two of the j-split form below 2048 bodies; the j-split form beats
-# the symmetric one, whose few block pairs cannot fill the GPU, below 65536 bodies (ms, best
-# of 10, j-split against the symmetric form's default shape: 40960 0.44 against 0.48, 49152
-# 0.61 against 0.60, 57344 0.80 against 0.94, 61440 0.91 against 0.94, 65536 1.04 against
-# 0.98).  FP64: j-split from 1024 bodies
-# (3.2 against 11.8 us of kernel time at 512), symmetric from 14336, between the measured
-# points (ms, best of 20, j-split against symmetric: 8192 0.053 against 0.076, 12288 0.096
-# against 0.110, 16384 0.160 against 0.140, 20480 0.250 against 0.213).
+# the symmetric one below 19456, where few groups of its balanced form fit its workspace (us,
+# j-split against symmetric: 17000 76 against 114, 18500 92 against 128, 19456 95 against 82,
+# 24576 146 against 132, 32768 251 against 200, 49999 577 against 450).  FP64: j-split from 1024
+# bodies (3.2 against 11.8 us of kernel time at 512), symmetric from 10500 (us, j-split against
+# symmetric: 9000 52 against 50, 10000 62 against 63, 10500 70 against 64, 12288 88 against 77,
+# 16384 151 against 119, 40000 876 against 591).
 SPLIT_FROM = 2048
-SYMMETRIC_FROM = 65536
+SYMMETRIC_FROM = 19456
 SPLIT_F64_FROM = 1024
-SYMMETRIC_F64_FROM = 14336
+SYMMETRIC_F64_FROM = 10500
 VJP_SPLIT_FROM = 1024
 
 

@@ -80,10 +80,12 @@ int grav_stage1_f32_cfg(const void *posm, void *acc, int64_t n, double G, double
  * grav_stage1_f32 (acc[3*n], FP32 pair terms, compensated accumulation, deterministic).
  * Bodies are grouped in blocks of 64*i_chunks_per_wave*waves; (i_chunks_per_wave, waves) in
  * {4,8} x {2,4}, or (0, 0) for the library's choice by n ((4, 2) below 57344 bodies, (8, 2)
- * from there; the form pays off over grav_stage1_f32 from about 24576 bodies and over
- * grav_stage1_f32_split from about 36000 on an MI355X, below which its few block pairs cannot
- * fill the GPU).  A row of block pairs is cut into segments of up to 8 pairs, one workgroup
- * each, whose partial sums go to a device workspace (256-byte aligned).
+ * from there; the form pays off over grav_stage1_f32_split from about 19000 bodies on an
+ * MI355X).  A row of block pairs is cut into segments of up to 8 pairs, one workgroup
+ * each, whose partial sums go to a device workspace (256-byte aligned).  In the default shape
+ * of 19000 to 115000 bodies the work of all rows is instead divided evenly among up to 2560
+ * workgroups, where the workspace holds their partial sums (grav_stage1_sym_workspace's size
+ * does).
  * grav_stage1_sym_workspace gives the size that holds every segment at once (12 n bytes +
  * 12 block (1 + seglen) bytes per segment: about 12 n + 6 n^2 / block (1 + seglen) / seglen,
  * 510 MB at 2^18 bodies); any size down to grav_stage1_sym_workspace_min's (one row of block

@@ -532,6 +532,39 @@ def test_stage1_symmetric_slabs(cuda, dtype, n, cfg):
     stages.release_workspaces()
 
 
+@pytest.mark.parametrize('n, dtype', [(n, torch.float32) for n in
+                                      (18944, 18945, 20479, 20480, 20481, 33000, 57343, 57344,
+                                       65537, 114687, 114688)]
+                         + [(n, torch.float64) for n in (8960, 8961, 11264, 12289, 30000, 65535)])
+def test_symmetric_default_shape_at_its_size_limits(cuda, n, dtype):
+    # The default shape divides the work evenly among workgroups between two sizes (as far as
+    # the workspace holds their partials) and works in row segments otherwise: both sides of
+    # the limits, bodies that fill their last block or chunk and not, workspaces that hold all,
+    # some or none of the workgroups, with and without softening, masses of mixed size.
+    f64 = dtype == torch.float64
+    print('sym default n=%d %s' % (n, 'f64' if f64 else 'f32'), flush=True)
+    rng = np.random.default_rng(n)
+    posm = _posm(rng.normal(size=(n, 3)), np.exp(rng.uniform(-3, 3, n)), cuda, dtype)
+    pos, m = _inputs(posm)
+    rows = np.unique(np.concatenate([rng.choice(n, 200, replace=False), [0, 63, 64, 1023, 1024],
+                                     np.arange(n - 66, n)]))
+    of = stages.sym_f64_workspace_bytes if f64 else stages.sym_workspace_bytes
+    run = stages.stage1_sym_f64 if f64 else stages.stage1_sym_f32
+    full, least = of(n), of(n, minimum=True)
+    for eps in (0.0, 1e-3):
+        ref = oracle_rows(pos, m, 0.7, eps, rows)
+        for size in (full, 2 * full // 3 // 256 * 256, least):
+            ws = torch.full((size,), 255, dtype=torch.uint8, device=cuda)   # NaN where unwritten
+            acc = torch.full((3, n), float('nan'), dtype=dtype, device=cuda)
+            run(posm, acc, 0.7, eps, None, ws)
+            a = acc.cpu().numpy().T.astype(np.float64)
+            assert np.all(np.isfinite(a)), (eps, size)
+            assert O.rel_err(a[rows], ref) < (TOL64 if f64 else TOL32), (eps, size)
+            run(posm, acc, 0.7, eps, None, ws)
+            assert np.array_equal(acc.cpu().numpy().T.astype(np.float64), a), (eps, size)
+    stages.release_workspaces()
+
+
 @pytest.mark.parametrize('n', [65, 4096, 5000, 20000])
 def test_split_step_io_is_bitwise_in_place(cuda, n):
     # grav_step_split_f64m_io (new positions to another buffer, as the recomputed segments of
