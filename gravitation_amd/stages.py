@@ -94,15 +94,16 @@ def stage1_f32(posm, acc, G, eps=0.0, accum='kahan', cfg=None):
 _workspaces = {}
 
 
-# Form thresholds, from stage-1 times on Plummer spheres on an MI355X.  FP32: one launch
-# (owner-computes) beats the two of the j-split form below 2048 bodies; the j-split form beats
-# the symmetric one below 19456, where few groups of its balanced form fit its workspace (us,
-# j-split against symmetric: 17000 76 against 114, 18500 92 against 128, 19456 95 against 82,
-# 24576 146 against 132, 32768 251 against 200, 49999 577 against 450).  FP64: j-split from 1024
-# bodies (3.2 against 11.8 us of kernel time at 512), symmetric from 10500 (us, j-split against
-# symmetric: 9000 52 against 50, 10000 62 against 63, 10500 70 against 64, 12288 88 against 77,
-# 16384 151 against 119, 40000 876 against 591).
-SPLIT_FROM = 2048
+# Form thresholds, from times on an MI355X.  FP32: one launch (owner-computes) beats the two of
+# the j-split form below 1088 bodies (a hip1 step of the galaxy, us, owner-computes against
+# j-split: 512 24.8 and 27.5, 1000 28.2 and 27.2, 1500 31.6 and 27.4, 2000 35.7 and 27.7).  The
+# j-split form beats the symmetric one below 19456, where few groups of its balanced form fit
+# its workspace (stage 1, Plummer, us, j-split against symmetric: 17000 76 against 114, 18500 92
+# against 128, 19456 95 against 82, 24576 146 against 132, 32768 251 against 200, 49999 577
+# against 450).  FP64: j-split from 1024 bodies (3.2 against 11.8 us of kernel time at 512),
+# symmetric from 10500 (us, j-split against symmetric: 9000 52 against 50, 10000 62 against 63,
+# 10500 70 against 64, 12288 88 against 77, 16384 151 against 119, 40000 876 against 591).
+SPLIT_FROM = 1088
 SYMMETRIC_FROM = 19456
 SPLIT_F64_FROM = 1024
 SYMMETRIC_F64_FROM = 10500
