@@ -9,9 +9,9 @@ and FP64 position/velocity masters, by one of two schedules of the same plan:
 * ``fused``: whole universes bin-packed into workgroups, positions in LDS, all steps of a
   call in ONE launch (``grav_batched_step_f32`` / ``grav_batched_adjoint_f32``); best when
   the universes are small and many;
-* ``perstep``: one launch per stage per step over every universe's i-tiles, largest first,
-  so a big universe is spread over the whole GPU (``grav_batched_stage1_f32`` +
-  ``grav_stage2_f64m``; ``grav_batched_adjoint_mu`` + ``grav_batched_stage1_vjp_f32``);
+* ``perstep``: one launch per step over every universe's i-tiles, largest first, so a big
+  universe is spread over the whole GPU (``grav_batched_step_items_f32``;
+  ``grav_batched_adjoint_mu`` + ``grav_batched_stage1_vjp_f32``);
   best when a few large universes dominate the cost;
 * ``perstep-sym``: ``perstep`` with stage 1 in the symmetric form (each pair of bodies of a
   universe once, in blocks of 64*K*W bodies: ``grav_batched_stage1_sym_f32``), which halves
@@ -155,6 +155,16 @@ def _check_mode(mode, sym):
                          % (SYM_SHAPES, sym))
 
 
+def _slots_of(traj, posm, steps, n):
+    """Whether traj[0 .. steps-1] are float32 (n, 4) buffers that a step can read and write in
+    place of posm: contiguous, 16-byte aligned and apart from posm."""
+    if (traj.dtype != torch.float32 or traj.dim() != 3 or tuple(traj.shape[1:]) != (n, 4)
+            or traj.shape[0] < steps or not traj.is_contiguous() or traj.data_ptr() % 16):
+        return False
+    a, b, size = traj.data_ptr(), posm.data_ptr(), 16 * n
+    return a + steps * size <= b or b + size <= a
+
+
 class Engine:
     """A plan plus a schedule ('fused', 'perstep' or 'perstep-sym'); advances and
     differentiates the concatenated state of all universes on the current stream."""
@@ -184,6 +194,7 @@ class Engine:
         self.j_waves = int(jw)
         self.config = (mode,) + self.plan.config + (int(jw),)
         self._acc = None
+        self._pos2 = None
         self._mu4 = None
         self._ws = None
         if mode == 'perstep-sym':
@@ -227,18 +238,52 @@ class Engine:
                              r64.data_ptr(), v64.data_ptr(), G, eps, dt, int(steps),
                              None if traj is None else traj.data_ptr(), _stream(dev))
                 return
+            if self._ws is None:
+                self._forward_items(posm, r64, v64, G, eps, dt, steps, traj)
+                return
             acc = self._buf('_acc', (3, self.n), torch.float32, dev)
             for t in range(steps):
                 if traj is not None:
                     traj[t].copy_(posm)
-                if self._ws is not None:
-                    _native.call('grav_batched_stage1_sym_f32', self.plan.handle,
-                                 posm.data_ptr(), acc.data_ptr(), G, eps, self._ws.data_ptr(),
-                                 self._ws.numel(), _stream(dev))
-                else:
-                    _native.call('grav_batched_stage1_f32', self.plan.handle, posm.data_ptr(),
-                                 acc.data_ptr(), G, eps, self.j_waves, _stream(dev))
+                _native.call('grav_batched_stage1_sym_f32', self.plan.handle, posm.data_ptr(),
+                             acc.data_ptr(), G, eps, self._ws.data_ptr(), self._ws.numel(),
+                             _stream(dev))
                 stages.stage2_f64m(posm, r64, v64, acc, dt)
+
+    def _forward_items(self, posm, r64, v64, G, eps, dt, steps, traj):
+        """``forward`` of the 'perstep' schedule: a step is one launch from one position buffer
+        to another, through the record's slots or back and forth between posm and a buffer of
+        the engine's.  A single step without a record, and steps into a record whose slots are
+        no float32 position buffers of their own, run their two stages in place."""
+        n = self.n
+        for t, name, dtype, shape in ((posm, 'posm', torch.float32, (n, 4)),
+                                      (r64, 'r64', torch.float64, (3, n)),
+                                      (v64, 'v64', torch.float64, (3, n))):
+            stages._check(t, name, dtype, shape)
+        dev = posm.device
+        stream = _stream(dev)
+        bufs, in_place = [posm], steps % 2
+        if traj is None:
+            if steps > 1:
+                other = self._buf('_pos2', (n, 4), torch.float32, dev)
+                bufs = [posm, other] * (steps // 2) + [posm]
+        elif steps and _slots_of(traj, posm, steps, n):
+            in_place = 0
+            traj[0].copy_(posm)
+            bufs = [traj[t] for t in range(steps)] + [posm]
+        else:
+            in_place = steps
+        for t in range(in_place):
+            acc = self._buf('_acc', (3, n), torch.float32, dev)
+            if traj is not None:
+                traj[t].copy_(posm)
+            _native.call('grav_batched_stage1_f32', self.plan.handle, posm.data_ptr(),
+                         acc.data_ptr(), G, eps, self.j_waves, stream)
+            stages.stage2_f64m(posm, r64, v64, acc, dt)
+        for a, b in zip(bufs, bufs[1:]):
+            _native.call('grav_batched_step_items_f32', self.plan.handle, a.data_ptr(),
+                         b.data_ptr(), r64.data_ptr(), v64.data_ptr(), G, eps, dt,
+                         self.j_waves, stream)
 
     def adjoint(self, traj, rho, nu, gamma, G, eps, dt, steps):
         """``steps`` backward steps (t = steps-1 .. 0) at the positions traj[t]."""
@@ -318,6 +363,7 @@ class Batch:
         with torch.cuda.stream(s):
             if self.engine.mode != 'fused':
                 self.engine._buf('_acc', (3, self.n), torch.float32, self.device)
+                self.engine._buf('_pos2', (self.n, 4), torch.float32, self.device)
             with torch.cuda.graph(g, stream=s):
                 self.step(steps)
         torch.cuda.current_stream(self.device).wait_stream(s)

@@ -801,6 +801,35 @@ int grav_batched_stage1_f32(const grav_batched_plan *plan, const void *posm, voi
                            256, plan->items, plan->nitems, static_cast<hipStream_t>(stream));
 }
 
+int grav_batched_step_items_f32(const grav_batched_plan *plan, const void *posm_in,
+                                void *posm_out, void *r64, void *v64, double G, double eps,
+                                double dt, int j_waves, void *stream) {
+  clear_error();
+  const char *fn = "grav_batched_step_items_f32";
+  GRAV_REQUIRE(plan != nullptr, "%s: plan is NULL", fn);
+  if (int rc = plan_on_current_device(plan, fn)) return rc;
+  GRAV_REQUIRE(posm_in != nullptr && posm_out != nullptr && r64 != nullptr && v64 != nullptr,
+               "%s: NULL buffer", fn);
+  GRAV_REQUIRE(aligned(posm_in, 16) && aligned(posm_out, 16) && aligned(r64, 8) &&
+                   aligned(v64, 8),
+               "%s: misaligned buffer", fn);
+  const uintptr_t a = reinterpret_cast<uintptr_t>(posm_in);
+  const uintptr_t b = reinterpret_cast<uintptr_t>(posm_out);
+  const uintptr_t bytes = 16 * static_cast<uintptr_t>(plan->n_bodies);
+  GRAV_REQUIRE(a + bytes <= b || b + bytes <= a, "%s: posm_out overlaps posm_in", fn);
+  GRAV_REQUIRE(G == G && G > -1e300 && G < 1e300, "%s: G must be finite", fn);
+  GRAV_REQUIRE(eps >= 0.0 && eps < 1e150, "%s: eps must be >= 0", fn);
+  GRAV_REQUIRE(dt == dt && dt > -1e300 && dt < 1e300, "%s: dt must be finite", fn);
+  GRAV_REQUIRE(j_waves == 1 || j_waves == 2 || j_waves == 4 || j_waves == 8,
+               "%s: j_waves must be 1, 2, 4 or 8", fn);
+  return step_items_f64m_launch(static_cast<const float4 *>(posm_in),
+                                static_cast<float4 *>(posm_out), static_cast<double *>(r64),
+                                static_cast<double *>(v64), static_cast<int>(plan->n_bodies),
+                                static_cast<float>(G), static_cast<float>(eps * eps),
+                                eps == 0.0 ? 1 : 0, dt, plan->kt, j_waves, plan->items,
+                                plan->nitems, static_cast<hipStream_t>(stream));
+}
+
 int grav_batched_sym_prepare(grav_batched_plan *plan, int i_chunks_per_wave, int waves) {
   clear_error();
   GRAV_REQUIRE(plan != nullptr, "grav_batched_sym_prepare: plan is NULL");

@@ -87,6 +87,13 @@ int stage1_f32_launch(const float4 *posm, float *acc, int n, float G, float eps2
                       int K, int S, int jblock, const int4 *items, int nitems,
                       hipStream_t stream);
 
+// One step of the items' bodies in one launch: stage1_f32_launch's accelerations, then the
+// FP64-master stage 2, bit for bit the two kernels'; the new positions go to out, which must not
+// overlap posm.  K in {1,2,4}, S in {1,2,4,8}.  (stage1.hip)
+int step_items_f64m_launch(const float4 *posm, float4 *out, double *r64, double *v64, int n,
+                           float G, float eps2, int mask, double dt, int K, int S,
+                           const int4 *items, int nitems, hipStream_t stream);
+
 // Unscaled FP32 sums of the bodies [i0, i0 + m) against their own blocks of diag_block bodies
 // (i0 and diag_block multiples of 256), into acc (3, m): the block-diagonal pass of the
 // symmetric form for a range of blocks, (K, S) = (4, 4).  (stage1.hip)

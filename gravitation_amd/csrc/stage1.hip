@@ -211,6 +211,36 @@ __global__ __launch_bounds__(kWave *S) void k_stage1_f64(const double4 *__restri
   }
 }
 
+// One whole step of the items (stage1_f32_block with STEP): stage 1 and the FP64-master stage 2.
+// A step of a batch was this kernel's pair loop, a launch of 5 to 13 us that reads and writes 124
+// bytes per body, and, for a record, a copy of the positions.  MI355X, two launches and one: 1024
+// universes of 32-2048 bodies 0.136 and 0.130 ms per step, forward and backward of 128
+// universes over 12 steps 1.22 and 1.16 ms.
+template <int K, int S, int JB>
+__global__ __launch_bounds__(kWave *S) void k_step_items_f64m(const float4 *__restrict__ posm,
+                                                               int n, float G, float eps2,
+                                                               int mask_self,
+                                                               const int4 *__restrict__ items,
+                                                               StepIO io) {
+  extern __shared__ float red[];  // (S - 1) * 6 * (64 * K)
+  stage1_f32_block<K, S, JB, true>(posm, nullptr, n, 0, n, G, eps2, mask_self, 256, items, 0,
+                                   nullptr, static_cast<int>(blockIdx.x), 0, 1, red, io);
+}
+
+template <int K, int S>
+int launch_step_items(const float4 *posm, int n, float G, float eps2, int mask,
+                      const int4 *items, int nitems, const StepIO &io, hipStream_t stream) {
+  const size_t lds = (S > 1) ? sizeof(float) * (S - 1) * 6 * kWave * K : 0;
+  constexpr int kNarrow = K >= 4 ? 8 : K == 1 ? 4 : 2;   // pair_loop_width's other value
+  if (pair_loop_width(nitems, K, false) == 8)
+    hipLaunchKernelGGL((k_step_items_f64m<K, S, 8>), dim3(nitems), dim3(kWave * S), lds, stream,
+                       posm, n, G, eps2, mask, items, io);
+  else
+    hipLaunchKernelGGL((k_step_items_f64m<K, S, kNarrow>), dim3(nitems), dim3(kWave * S), lds,
+                       stream, posm, n, G, eps2, mask, items, io);
+  return check_launch("k_step_items_f64m");
+}
+
 // i-tiles of the shard [i0, i0 + m) (items == NULL) or the nitems items, each against all n
 // bodies; see stage1_f32_block.
 template <int K, int S>
@@ -360,6 +390,20 @@ int launch_f32_ks(int K, int S, const float4 *posm, float *acc, int n, int i0, i
   return fail(GRAV_EINVAL, "i_per_lane must be 1, 2, 4 or 8 (got %d)", K);
 }
 }  // namespace
+
+int step_items_f64m_launch(const float4 *posm, float4 *out, double *r64, double *v64, int n,
+                           float G, float eps2, int mask, double dt, int K, int S,
+                           const int4 *items, int nitems, hipStream_t stream) {
+  const StepIO io{out, r64, v64, dt};
+#define GRAV_STEP(KK, SS) \
+  if (K == KK && S == SS)  \
+    return launch_step_items<KK, SS>(posm, n, G, eps2, mask, items, nitems, io, stream);
+  GRAV_STEP(1, 1) GRAV_STEP(1, 2) GRAV_STEP(1, 4) GRAV_STEP(1, 8)
+  GRAV_STEP(2, 1) GRAV_STEP(2, 2) GRAV_STEP(2, 4) GRAV_STEP(2, 8)
+  GRAV_STEP(4, 1) GRAV_STEP(4, 2) GRAV_STEP(4, 4) GRAV_STEP(4, 8)
+#undef GRAV_STEP
+  return fail(GRAV_EINVAL, "step of items: (i_per_lane, j_waves) = (%d, %d) not supported", K, S);
+}
 
 int stage1_f32_launch(const float4 *posm, float *acc, int n, float G, float eps2, int mask,
                       int K, int S, int jblock, const int4 *items, int nitems,

@@ -161,6 +161,34 @@ __device__ __forceinline__ void sum_segment_f32(const float4 *__restrict__ posm,
   }
 }
 
+// The FP64-master stage 2 of body i from its FP32 acceleration a, without contraction as
+// k_stage2_f64m does it (v = a dt + v, r = v dt + r): r and v come as r64 and v64 hold them (stride
+// n), the new ones go back there and the new FP32 position, with mass m, to out[i].
+__device__ __forceinline__ void stage2_f64m_body(const float (&a)[3], double (&r)[3],
+                                                 double (&v)[3], float m, float4 *out,
+                                                 double *__restrict__ r64,
+                                                 double *__restrict__ v64, int n, double dt,
+                                                 int i) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    v[c] = static_cast<double>(a[c]) * dt + v[c];
+    r[c] = v[c] * dt + r[c];
+    v64[c * n + i] = v[c];
+    r64[c * n + i] = r[c];
+  }
+  out[i] = make_float4(static_cast<float>(r[0]), static_cast<float>(r[1]),
+                       static_cast<float>(r[2]), m);
+}
+
+// Where a fused step of the item-list form puts its results: the FP64 masters (stride m) and
+// the new positions, which must not overlap the old ones.
+struct StepIO {
+  float4 *out;
+  double *r64, *v64;
+  double dt;
+};
+
 // The workgroup at (bx, by) of an (x, ny) grid owns i in [items[bx].x, items[bx].y) (at most
 // 64*K bodies) against j in [items[bx].z, items[bx].w); items == NULL means one universe:
 // i-tile bx of the shard [i0, i0 + m) against all n bodies, or, with diag_block > 0, against
@@ -171,14 +199,18 @@ __device__ __forceinline__ void sum_segment_f32(const float4 *__restrict__ posm,
 // m is the row stride.  The item list lets one launch cover many universes (one item per
 // universe tile).  JB: j-bodies per step of the pair loop (pair_range_f32), 2, 4 or 8; the
 // result does not depend on it.  red: (S - 1) * 6 * (64 * K) floats of LDS.
-template <int K, int S, int JB>
+// STEP (with items): instead of acc, the bodies' FP64-master stage 2 into io, bit for bit
+// k_stage1_f32 followed by k_stage2_f64m.  With one body per lane the masters are loaded before
+// the pair loop.
+template <int K, int S, int JB, bool STEP = false>
 __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm,
                                                  float *__restrict__ acc, int n, int i0, int m,
                                                  float G, float eps2, int mask_self,
                                                  int jblock,
                                                  const int4 *__restrict__ items,
                                                  int diag_block, double *__restrict__ part,
-                                                 int bx, int by, int ny, float *red) {
+                                                 int bx, int by, int ny, float *red,
+                                                 const StepIO io = StepIO{}) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   int ibase, iend, jlo, jhi;
@@ -212,6 +244,18 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
     xi[k] = p.x;
     yi[k] = p.y;
     zi[k] = p.z;
+  }
+
+  double mr[3], mv[3];
+  if constexpr (STEP && K == 1) {
+    if (wave == 0) {
+      const int ic = min(ii[0], iend - 1);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        mr[c] = io.r64[c * m + ic];
+        mv[c] = io.v64[c * m + ic];
+      }
+    }
   }
 
   float hx[K], hy[K], hz[K], lx[K], ly[K], lz[K];
@@ -279,6 +323,24 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
     }
     return;
   }
+  if constexpr (STEP) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int i = ii[k];
+      if (i < iend) {
+        const float a[3] = {G * (hx[k] + lx[k]), G * (hy[k] + ly[k]), G * (hz[k] + lz[k])};
+        if constexpr (K != 1) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            mr[c] = io.r64[c * m + i];
+            mv[c] = io.v64[c * m + i];
+          }
+        }
+        stage2_f64m_body(a, mr, mv, posm[i].w, io.out, io.r64, io.v64, m, io.dt, i);
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int i = ii[k];
@@ -295,9 +357,10 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
 //   * K = 1 from 256 workgroups: four, or two in the j-split form from 2048 workgroups.  MI355X,
 //     two and four per step: owner-computes 16384 bodies 77.4 and 71.8 us, 2^18 15.39 and
 //     15.20 ms; the batched per-step schedule on 1024 universes of 32-2048 bodies 1.387 and
-//     1.348 ms per 10 steps; forward and backward of 4096
-//     bodies over 60 steps (512 workgroups) 2.03 and 2.00 ms; but the j-split form at 16384
-//     bodies (4096 workgroups) 70.2 and 70.8 us, at 32768 248.8 and 251.2 us.  (Six: 70.8 us and 17.5 ms; eight, without loads ahead: 18.4 ms.)
+//     1.348 ms per 10 steps; forward and backward of 4096 bodies over 60 steps (512 workgroups)
+//     2.03 and 2.00 ms; but the j-split form at 16384 bodies (4096 workgroups) 70.2 and 70.8 us,
+//     at 32768 248.8 and 251.2 us.  (Six: 70.8 us and 17.5 ms; eight, without loads ahead:
+//     18.4 ms.)
 //   * Fewer workgroups: eight.  One launch per universe of 32-2048 bodies (at most 32
 //     workgroups) takes 38.3 ms per step of 4096 universes with two and 34.0 with eight.
 //   * K = 2, plain loop: two from 1024 workgroups (2^18 bodies, (2, 16): 17.9 against 18.4 ms),

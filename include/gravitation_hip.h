@@ -251,6 +251,10 @@ int grav_adjoint_mu_ws(const void *rho64, void *nu64, void *mu4, int64_t n, doub
  * limit on a universe's size beyond the plan's):
  *   grav_batched_stage1_f32     acc[3*n] of every universe (FP32 compensated), j_waves in
  *                               {1,2,4,8} wavefronts splitting each tile's j-range;
+ *   grav_batched_step_items_f32 a whole step in one launch: grav_batched_stage1_f32 from
+ *                               posm_in, then grav_stage2_f64m on r64 and v64, the new
+ *                               positions (x, y, z, m) to posm_out, which must not overlap
+ *                               posm_in; the same bits;
  *   grav_batched_adjoint_mu     grav_adjoint_mu for every universe, each with its own E;
  *   grav_batched_stage1_vjp_f32 the all-pairs adjoint part of grav_stage1_vjp_f32 for every
  *                               universe (plan i_per_lane <= 4).
@@ -259,6 +263,9 @@ int grav_adjoint_mu_ws(const void *rho64, void *nu64, void *mu4, int64_t n, doub
  */
 int grav_batched_stage1_f32(const grav_batched_plan *plan, const void *posm, void *acc,
                             double G, double eps, int j_waves, void *stream);
+int grav_batched_step_items_f32(const grav_batched_plan *plan, const void *posm_in,
+                                void *posm_out, void *r64, void *v64, double G, double eps,
+                                double dt, int j_waves, void *stream);
 int grav_batched_adjoint_mu(const grav_batched_plan *plan, const void *rho64, void *nu64,
                             void *mu4, double dt, void *stream);
 int grav_batched_stage1_vjp_f32(const grav_batched_plan *plan, const void *posm,

@@ -303,3 +303,46 @@ def test_shares_step_like_the_whole_batch(cuda, cfg):
         rb, vb = b.state()
         want_r, want_v, _, _ = batched.take_universes(rw, vw, m, off, share)
         assert np.array_equal(rb, want_r) and np.array_equal(vb, want_v), share
+
+
+@pytest.mark.parametrize('sizes', [[1], [63, 64, 65, 1, 130], [256, 255, 700, 33],
+                                   [70] * 260])
+@pytest.mark.parametrize('kt, jw', [(1, 4), (1, 1), (2, 8), (4, 2)])
+def test_perstep_fused_step_is_bitwise_its_two_stages(cuda, sizes, kt, jw):
+    # grav_batched_step_items_f32 == grav_batched_stage1_f32 + grav_stage2_f64m bit for bit:
+    # odd and even numbers of steps, with a record (one the steps run through, and one that
+    # only takes copies) and without, few and many workgroups, eps = 0 and > 0
+    from gravitation_amd import stages
+    print('fused step', len(sizes), kt, jw, flush=True)
+    rng = np.random.default_rng(len(sizes) + kt)
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    n = int(off[-1])
+    r, v = rng.normal(size=(n, 3)), rng.normal(size=(n, 3))
+    m = rng.uniform(0.1, 1.0, n)
+    config = ('perstep', 8, kt, 8 // kt, 0, jw)
+    for eps in (0.0, 1e-2):
+        for steps in (1, 2, 3):
+            ref = batched.Batch(r, v, m, off, eps=eps, config=config)
+            acc = torch.empty((3, n), dtype=torch.float32, device=cuda)
+            seen = []
+            for _ in range(steps):
+                seen.append(ref.posm.clone())
+                _native.call('grav_batched_stage1_f32', ref.plan.handle, ref.posm.data_ptr(),
+                             acc.data_ptr(), ref.G, eps, jw,
+                             torch.cuda.current_stream().cuda_stream)
+                stages.stage2_f64m(ref.posm, ref.r64, ref.v64, acc, ref.dt)
+            for dtype in (None, torch.float32, torch.float64):
+                b = batched.Batch(r, v, m, off, eps=eps, config=config)
+                traj = None if dtype is None else torch.zeros((steps, n, 4), dtype=dtype,
+                                                              device=cuda)
+                b.engine.forward(b.posm, b.r64, b.v64, b.G, eps, b.dt, steps, traj)
+                for x, y in ((b.posm, ref.posm), (b.r64, ref.r64), (b.v64, ref.v64)):
+                    assert torch.equal(x, y), (eps, steps, dtype)
+                if traj is not None:
+                    assert torch.equal(traj, torch.stack(seen).to(dtype)), (eps, steps, dtype)
+    with pytest.raises(TypeError):
+        b.engine.forward(b.posm, b.r64.float(), b.v64, 1.0, 0.0, 1e-3, 2)
+    with pytest.raises(_native.GravError, match='overlap'):
+        _native.call('grav_batched_step_items_f32', b.plan.handle, b.posm.data_ptr(),
+                     b.posm.data_ptr(), b.r64.data_ptr(), b.v64.data_ptr(), 1.0, 0.0, 1e-3, jw,
+                     torch.cuda.current_stream().cuda_stream)
