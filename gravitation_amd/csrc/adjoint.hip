@@ -438,58 +438,52 @@ __global__ __launch_bounds__(kWave *S) void k_stage1_vjp_f32(
                              static_cast<int>(gridDim.y), red);
 }
 
-// rho[c][i] += hs * sum_p part[p][c][i], gamma[i] -= hs * sum_p part[p][3][i], hs = hG 2^E
-// with the universe's exponent E from mu4[i].w; sums in FP64 in range order.
-__device__ __forceinline__ void split_reduce_vjp_body(const double *__restrict__ part,
-                                                      const float4 *mu4,
-                                                      double *__restrict__ rho,
-                                                      double *__restrict__ gamma, int n,
-                                                      int splits, double hG, int i) {
-  const size_t stride = static_cast<size_t>(4) * n;
-  double s[4] = {0.0, 0.0, 0.0, 0.0};
-  int p = 0;
-  for (; p + 2 <= splits; p += 2) {  // eight loads in flight, added in range order
-    double v[2][4];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) v[t][c] = part[(p + t) * stride + static_cast<size_t>(c) * n + i];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) s[c] += v[t][c];
+// Component c of body i: rho[c][i] += hs * sum_p part[p][c][i] (c < 3) or gamma[i] -= hs * sum_p
+// part[p][3][i], hs = hG 2^E; sums in FP64 in range order.  Returns the new rho.
+__device__ __forceinline__ double split_reduce_vjp_component(const double *__restrict__ part,
+                                                             double *__restrict__ rho,
+                                                             double *__restrict__ gamma, int n,
+                                                             int splits, double hG, int E, int c,
+                                                             int i) {
+  const size_t at = static_cast<size_t>(c) * n + i;
+  const double old = c < 3 ? rho[at] : gamma[i];
+  const double s = split_sum<4>(part, c, i, n, splits);
+  const double hs = ldexp(hG, E);
+  if (c == 3) {
+    gamma[i] = old - hs * s;
+    return 0.0;
   }
-  for (; p < splits; ++p) {
-    const double *q = part + p * stride + i;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) s[c] += q[static_cast<size_t>(c) * n];
-  }
-  const double hs = ldexp(hG, __float_as_int(mu4[i].w));
-#pragma unroll
-  for (int c = 0; c < 3; ++c) rho[static_cast<size_t>(c) * n + i] += hs * s[c];
-  gamma[i] -= hs * s[3];
+  const double r = old + hs * s;
+  rho[at] = r;
+  return r;
 }
 
-__global__ __launch_bounds__(256) void k_split_reduce_vjp(const double *__restrict__ part,
-                                                          const float4 *__restrict__ mu4,
-                                                          double *__restrict__ rho,
-                                                          double *__restrict__ gamma, int n,
-                                                          int splits, double hG) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) split_reduce_vjp_body(part, mu4, rho, gamma, n, splits, hG, i);
+__global__ __launch_bounds__(4 * kReduceBodies) void k_split_reduce_vjp(
+    const double *__restrict__ part, const float4 *__restrict__ mu4, double *__restrict__ rho,
+    double *__restrict__ gamma, int n, int splits, double hG) {
+  const int i = blockIdx.x * kReduceBodies + threadIdx.x % kReduceBodies;
+  const int c = __builtin_amdgcn_readfirstlane(threadIdx.x / kReduceBodies);
+  if (i < n)
+    split_reduce_vjp_component(part, rho, gamma, n, splits, hG, __float_as_int(mu4[i].w), c, i);
+}
+
+// nu + dt rho without contraction, as k_adjoint_mu forms it.
+__device__ __forceinline__ double mu_component(double nu, double rho, double dt) {
+#pragma clang fp contract(off)
+  return nu + dt * rho;
 }
 
 // The chained backward step's reduce: k_split_reduce_vjp, then, for the next backward step,
-// mu = nu + h rho into nu (as k_adjoint_mu_tiles) and its FP32 copy mu * 2^-E into mu4 (each
-// thread reads body i's current exponent before it overwrites body i's entry; no other thread
-// touches it).  E is the exponent gathered for the previous mu (eslot[0], put there by the
-// VJP kernel), so the scale lags the cotangent by one step: |mu4| may exceed 1 by the growth
-// of one step, far inside the FP32 headroom of the pair terms, and since scaling by a power
+// mu = nu + h rho into nu (as k_adjoint_mu_tiles) and its FP32 copy mu * 2^-E into mu4 (a body's
+// current exponent is read by its four threads before the barrier and overwritten after it; no
+// other thread touches it).  E is the exponent gathered for the previous mu (eslot[0], put there
+// by the VJP kernel), so the scale lags the cotangent by one step: |mu4| may exceed 1 by the
+// growth of one step, far inside the FP32 headroom of the pair terms, and since scaling by a power
 // of two is exact the VJP's result is the same as with the current exponent unless a scaled
 // component is subnormal.  The exponent of this mu goes into eslot[1] by an atomic max (the
 // order of the workgroups does not change a max).
-// Bodies [256 bx, 256 bx + 256) of the chained reduce (every thread of the workgroup calls
-// it: the exponent's maximum goes through LDS).
+// Bodies [kReduceBodies * bx, + kReduceBodies) of the chained reduce (every thread of the
+// workgroup calls it: the largest component goes through LDS).
 __device__ __forceinline__ void split_reduce_vjp_chain_block(const double *__restrict__ part,
                                                              float4 *mu4,
                                                              double *__restrict__ rho,
@@ -498,37 +492,47 @@ __device__ __forceinline__ void split_reduce_vjp_chain_block(const double *__res
                                                              int splits, double hG, double dt,
                                                              unsigned *__restrict__ eslot,
                                                              int bx) {
-  __shared__ int wmax[256 / kWave];
-  const int i = bx * 256 + static_cast<int>(threadIdx.x);
-  int e = INT_MIN;
+  __shared__ double size[3][kReduceBodies];
+  const int lane = static_cast<int>(threadIdx.x) % kReduceBodies;
+  const int c = __builtin_amdgcn_readfirstlane(threadIdx.x / kReduceBodies);
+  const int i = bx * kReduceBodies + lane;
+  double mu = 0.0;
   if (i < n) {
-    split_reduce_vjp_body(part, mu4, rho, gamma, n, splits, hG, i);
-    double m[3];
-    e = mu_body(rho, nu, n, i, dt, m);
-    const int E = static_cast<int>(eslot[0] - 0x80000000u);
-    mu4[i] = make_float4(static_cast<float>(ldexp(m[0], -E)), static_cast<float>(ldexp(m[1], -E)),
-                         static_cast<float>(ldexp(m[2], -E)), __int_as_float(E));
+    const size_t at = static_cast<size_t>(c) * n + i;
+    const double nv = c < 3 ? nu[at] : 0.0;
+    const double r = split_reduce_vjp_component(part, rho, gamma, n, splits, hG,
+                                                __float_as_int(mu4[i].w), c, i);
+    if (c < 3) {
+      mu = mu_component(nv, r, dt);
+      nu[at] = mu;
+      size[c][lane] = fabs(mu);
+    }
   }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) e = max(e, __shfl_xor(e, off));
-  if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x / kWave] = e;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int b = wmax[0];
+  const int E = static_cast<int>(eslot[0] - 0x80000000u);
+  if (c == 3) {
+    // the body's largest component; NaN components drop out, as in mu_body
+    int e = INT_MIN;
+    if (i < n) {
+      const double a = fmax(fmax(fmax(0.0, size[0][lane]), size[1][lane]), size[2][lane]);
+      if (a > 0.0 && a <= DBL_MAX) frexp(a, &e);
+      reinterpret_cast<int *>(mu4 + i)[3] = E;
+    }
 #pragma unroll
-    for (int w = 1; w < 256 / kWave; ++w) b = max(b, wmax[w]);
-    if (b != INT_MIN) atomicMax(eslot + 1, exp_bias(b));
+    for (int off = kWave / 2; off > 0; off >>= 1) e = max(e, __shfl_xor(e, off));
+    if (lane == 0 && e != INT_MIN) atomicMax(eslot + 1, exp_bias(e));
+  } else if (i < n) {
+    reinterpret_cast<float *>(mu4 + i)[c] = static_cast<float>(ldexp(mu, -E));
   }
 }
 
-__global__ __launch_bounds__(256) void k_split_reduce_vjp_chain(const double *__restrict__ part,
-                                                                float4 *mu4,
-                                                                double *__restrict__ rho,
-                                                                double *__restrict__ nu,
-                                                                double *__restrict__ gamma,
-                                                                int n, int splits, double hG,
-                                                                double dt,
-                                                                unsigned *__restrict__ eslot) {
+// MI355X, forward and backward of 4096 bodies over 60 steps with one thread per body in workgroups
+// of 256 and with one per component in workgroups of 64 bodies, here and in the other reduce
+// kernels: 2.00 and 1.82 ms.
+__global__ __launch_bounds__(4 * kReduceBodies) void k_split_reduce_vjp_chain(
+    const double *__restrict__ part, float4 *mu4, double *__restrict__ rho,
+    double *__restrict__ nu, double *__restrict__ gamma, int n, int splits, double hG, double dt,
+    unsigned *__restrict__ eslot) {
   split_reduce_vjp_chain_block(part, mu4, rho, nu, gamma, n, splits, hG, dt, eslot,
                                static_cast<int>(blockIdx.x));
 }
@@ -562,7 +566,7 @@ __global__ __launch_bounds__(kWave *S) void k_backward_pair(
 
 // ... and its reduce: the first nb workgroups the chained reduce of the backward step, the
 // other nb the reduce + FP64-master stage 2 of the recomputed step (positions pr -> pr_out).
-__global__ __launch_bounds__(256) void k_backward_pair_reduce(
+__global__ __launch_bounds__(4 * kReduceBodies) void k_backward_pair_reduce(
     const double *__restrict__ part_a, float4 *mu4, double *__restrict__ rho,
     double *__restrict__ nu, double *__restrict__ gamma, int splits_a, double hG,
     unsigned *__restrict__ eslot, const double *__restrict__ part_r, const float4 *pr,
@@ -572,8 +576,10 @@ __global__ __launch_bounds__(256) void k_backward_pair_reduce(
   if (b < nb) {
     split_reduce_vjp_chain_block(part_a, mu4, rho, nu, gamma, n, splits_a, hG, dt, eslot, b);
   } else {
-    const int i = (b - nb) * 256 + static_cast<int>(threadIdx.x);
-    if (i < n) split_step_body(part_r, pr, pr_out, r64, v64, n, splits_r, G, dt, i);
+    const int i = (b - nb) * kReduceBodies + static_cast<int>(threadIdx.x) % kReduceBodies;
+    const int c = __builtin_amdgcn_readfirstlane(threadIdx.x / kReduceBodies);
+    if (c < 3 && i < n)
+      split_step_component(part_r, pr, pr_out, r64, v64, n, splits_r, G, dt, c, i);
   }
 }
 
@@ -650,8 +656,8 @@ int stage1_vjp_split_launch(const float4 *posm, const float4 *mu4, double *rho, 
   const int rc =
       vjp_split_partials(posm, mu4, part, n, 0, n, eps2, K, S, splits, nullptr, stream);
   if (rc != GRAV_OK) return rc;
-  hipLaunchKernelGGL(k_split_reduce_vjp, dim3((n + 255) / 256), dim3(256), 0, stream, part, mu4,
-                     rho, gamma, n, splits, hG);
+  hipLaunchKernelGGL(k_split_reduce_vjp, dim3((n + kReduceBodies - 1) / kReduceBodies),
+                     dim3(4 * kReduceBodies), 0, stream, part, mu4, rho, gamma, n, splits, hG);
   return check_launch("k_split_reduce_vjp");
 }
 
@@ -674,8 +680,9 @@ int stage1_vjp_shard_launch(const float4 *posm, const float4 *mu4, double *rho, 
   const int rc = vjp_split_partials(posm, mu4, part, n, i0, m, eps2, K, S, splits, nullptr,
                                     stream);
   if (rc != GRAV_OK) return rc;
-  hipLaunchKernelGGL(k_split_reduce_vjp, dim3((m + 255) / 256), dim3(256), 0, stream, part,
-                     mu4 + i0, rho, gamma, m, splits, hG);
+  hipLaunchKernelGGL(k_split_reduce_vjp, dim3((m + kReduceBodies - 1) / kReduceBodies),
+                     dim3(4 * kReduceBodies), 0, stream, part, mu4 + i0, rho, gamma, m, splits,
+                     hG);
   return check_launch("k_split_reduce_vjp");
 }
 
@@ -695,9 +702,9 @@ int launch_backward_pair(const float4 *pa, float4 *mu4, double *rho, double *nu,
                      n, eps2);
   int rc = check_launch("k_backward_pair");
   if (rc != GRAV_OK) return rc;
-  const int nb = (n + 255) / 256;
-  hipLaunchKernelGGL(k_backward_pair_reduce, dim3(2 * nb), dim3(256), 0, stream, part_a, mu4,
-                     rho, nu, gamma, splits_a, hG, eslot, part_r, pr, pr_out, r64, v64, splits_r,
+  const int nb = (n + kReduceBodies - 1) / kReduceBodies;
+  hipLaunchKernelGGL(k_backward_pair_reduce, dim3(2 * nb), dim3(4 * kReduceBodies), 0, stream,
+                     part_a, mu4, rho, nu, gamma, splits_a, hG, eslot, part_r, pr, pr_out, r64, v64, splits_r,
                      G, dt, n, nb);
   return check_launch("k_backward_pair_reduce");
 }
@@ -733,12 +740,13 @@ int stage1_vjp_split_chain_launch(const float4 *posm, float4 *mu4, double *rho, 
       vjp_split_partials(posm, mu4, part, n, 0, n, eps2, K, S, splits, eslot, stream);
   if (rc != GRAV_OK) return rc;
   if (!next_mu) {
-    hipLaunchKernelGGL(k_split_reduce_vjp, dim3((n + 255) / 256), dim3(256), 0, stream, part,
-                       mu4, rho, gamma, n, splits, hG);
+    hipLaunchKernelGGL(k_split_reduce_vjp, dim3((n + kReduceBodies - 1) / kReduceBodies),
+                       dim3(4 * kReduceBodies), 0, stream, part, mu4, rho, gamma, n, splits, hG);
     return check_launch("k_split_reduce_vjp");
   }
-  hipLaunchKernelGGL(k_split_reduce_vjp_chain, dim3((n + 255) / 256), dim3(256), 0, stream, part,
-                     mu4, rho, nu, gamma, n, splits, hG, dt, eslot);
+  hipLaunchKernelGGL(k_split_reduce_vjp_chain, dim3((n + kReduceBodies - 1) / kReduceBodies),
+                     dim3(4 * kReduceBodies), 0, stream, part, mu4, rho, nu, gamma, n, splits, hG,
+                     dt, eslot);
   return check_launch("k_split_reduce_vjp_chain");
 }
 

@@ -49,17 +49,17 @@ __global__ __launch_bounds__(256) void k_split_reduce(const double *__restrict__
   const int i = blockIdx.x * 256 + threadIdx.x;
   const int c = blockIdx.y;
   if (i >= n) return;
-  acc[static_cast<size_t>(c) * n + i] = static_cast<T>(G * split_sum(part, c, i, n, splits));
+  acc[static_cast<size_t>(c) * n + i] = static_cast<T>(G * split_sum<3>(part, c, i, n, splits));
 }
 
-// split_step_body for every body (out may be in).
-__global__ __launch_bounds__(256) void k_split_step_f64m(const double *__restrict__ part,
-                                                         const float4 *in, float4 *out,
-                                                         double *__restrict__ r64,
-                                                         double *__restrict__ v64, int n,
-                                                         int splits, double G, double dt) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) split_step_body(part, in, out, r64, v64, n, splits, G, dt, i);
+// split_step_component for every body and component (out may be in).  MI355X, 4096 bodies and 8
+// ranges: 3.5 us, against 4.2 with one thread per body in workgroups of 256.
+__global__ __launch_bounds__(3 * kReduceBodies) void k_split_step_f64m(
+    const double *__restrict__ part, const float4 *in, float4 *out, double *__restrict__ r64,
+    double *__restrict__ v64, int n, int splits, double G, double dt) {
+  const int i = blockIdx.x * kReduceBodies + threadIdx.x % kReduceBodies;
+  const int c = __builtin_amdgcn_readfirstlane(threadIdx.x / kReduceBodies);
+  if (i < n) split_step_component(part, in, out, r64, v64, n, splits, G, dt, c, i);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -551,8 +551,9 @@ int split_step_f64m_launch(const float4 *in, float4 *out, double *r64, double *v
   if (rc != GRAV_OK) return rc;
   // the step kernel writes out (which may be in) after the partials kernel, launched before
   // it on the same stream, has read every position
-  hipLaunchKernelGGL(k_split_step_f64m, dim3((n + 255) / 256), dim3(256), 0, stream, part, in,
-                     out, r64, v64, n, splits, static_cast<double>(G), dt);
+  hipLaunchKernelGGL(k_split_step_f64m, dim3((n + kReduceBodies - 1) / kReduceBodies),
+                     dim3(3 * kReduceBodies), 0, stream, part, in, out, r64, v64, n, splits,
+                     static_cast<double>(G), dt);
   return check_launch("k_split_step_f64m");
 }
 

@@ -371,11 +371,12 @@ inline int pair_loop_width(int64_t workgroups, int K, bool split) {
   return (K >= 4 || workgroups < 1024) ? 8 : 2;
 }
 
-// sum over the j-ranges p of part[p][c][i], in FP64 and in range order, eight loads in
-// flight.
+// sum over the j-ranges p of part[p][c][i] (C components a range), in FP64 and in range order,
+// eight loads in flight.
+template <int C>
 __device__ __forceinline__ double split_sum(const double *__restrict__ part, int c, int i, int n,
                                             int splits) {
-  const size_t stride = static_cast<size_t>(3) * n;
+  const size_t stride = static_cast<size_t>(C) * n;
   const double *q = part + static_cast<size_t>(c) * n + i;
   double s = 0.0;
   int p = 0;
@@ -390,33 +391,33 @@ __device__ __forceinline__ double split_sum(const double *__restrict__ part, int
   return s;
 }
 
-// One body's reduce of the FP32 j-split form fused with the FP64-master stage 2: the
-// acceleration is rounded to FP32 exactly as k_split_reduce<float> stores it, then r, v
+// Bodies of a workgroup of the reduce kernels of the fused steps, which give each component of
+// a body a thread of its own: 64 bodies, one wavefront per component.  These kernels move little
+// (4096 bodies, 8 ranges: 1 MB) and last as long as one thread's chain of loads, so they are
+// spread over as many compute units as there are chunks of 64 bodies.
+constexpr int kReduceBodies = kWave;
+
+// Component c of body i in the reduce of the FP32 j-split form fused with the FP64-master stage
+// 2: the acceleration is rounded to FP32 exactly as k_split_reduce<float> stores it, then r, v
 // advance as in k_stage2_f64m (v = a dt + v, r = v dt + r, no contraction), so a step equals
 // the two kernels' bit for bit without writing acc.  The new FP32 position (x, y, z, m) of
-// body i goes to out[i]; out may be in (body i's mass is read before its entry is written).
-__device__ __forceinline__ void split_step_body(const double *__restrict__ part,
-                                                const float4 *in, float4 *out,
-                                                double *__restrict__ r64,
-                                                double *__restrict__ v64, int n, int splits,
-                                                double G, double dt, int i) {
+// body i goes to out[i], its mass with component 0; out may be in (no other thread touches them).
+__device__ __forceinline__ void split_step_component(const double *__restrict__ part,
+                                                     const float4 *in, float4 *out,
+                                                     double *__restrict__ r64,
+                                                     double *__restrict__ v64, int n, int splits,
+                                                     double G, double dt, int c, int i) {
 #pragma clang fp contract(off)
-  double r[3], v[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const float a32 = static_cast<float>(G * split_sum(part, c, i, n, splits));
-    const double a = static_cast<double>(a32);
-    v[c] = a * dt + v64[c * n + i];
-    r[c] = v[c] * dt + r64[c * n + i];
-  }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    v64[c * n + i] = v[c];
-    r64[c * n + i] = r[c];
-  }
-  const float m = in[i].w;
-  out[i] = make_float4(static_cast<float>(r[0]), static_cast<float>(r[1]),
-                       static_cast<float>(r[2]), m);
+  const size_t at = static_cast<size_t>(c) * n + i;
+  const double v0 = v64[at], r0 = r64[at];
+  const float a32 = static_cast<float>(G * split_sum<3>(part, c, i, n, splits));
+  const double v = static_cast<double>(a32) * dt + v0;
+  const double r = v * dt + r0;
+  v64[at] = v;
+  r64[at] = r;
+  float *o = reinterpret_cast<float *>(out + i);
+  if (c == 0) o[3] = in[i].w;
+  o[c] = static_cast<float>(r);
 }
 
 }  // namespace
