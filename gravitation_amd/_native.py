@@ -32,6 +32,7 @@ _i = ctypes.c_int
 SIGNATURES = {
     'grav_version': [],
     'grav_device_count': [ctypes.POINTER(_i)],
+    'grav_stream_synchronize': [_vp],
     'grav_stage1_f32': [_vp, _vp, _i64, _d, _d, _i, _vp],
     'grav_stage1_f32_cfg': [_vp, _vp, _i64, _d, _d, _i, _i, _i, _i, _vp],
     'grav_stage1_f64': [_vp, _vp, _i64, _d, _d, _vp],

@@ -48,7 +48,7 @@ def adjoint_mu(rho, nu, mu4, dt, workspace=None):
                                   (mu4, 'mu4', torch.float32, (n, 4))):
         stages._check(t, name, dtype, shape)
     stages.same_device(rho, nu, mu4)
-    stream = torch.cuda.current_stream(rho.device).cuda_stream
+    stream = stages.current_stream(rho.device)
     with stages.on_device(rho):
         if workspace is not None and n >= MU_TILES_FROM:
             stages.same_device(rho, workspace)
@@ -72,7 +72,7 @@ def stage1_vjp_f32(posm, mu4, rho, gamma, G, eps, dt):
     with stages.on_device(posm):
         _native.call('grav_stage1_vjp_f32', posm.data_ptr(), mu4.data_ptr(), rho.data_ptr(),
                      gamma.data_ptr(), n, float(G), float(eps), float(dt),
-                     torch.cuda.current_stream(posm.device).cuda_stream)
+                     stages.current_stream(posm.device))
 
 
 def stage1_vjp_split_f32(posm, mu4, rho, gamma, G, eps, dt, cfg=None, workspace=None):
@@ -93,7 +93,7 @@ def stage1_vjp_split_f32(posm, mu4, rho, gamma, G, eps, dt, cfg=None, workspace=
         _native.call('grav_stage1_vjp_f32_split', posm.data_ptr(), mu4.data_ptr(),
                      rho.data_ptr(), gamma.data_ptr(), n, float(G), float(eps), float(dt),
                      int(k), int(s), int(p), workspace.data_ptr(), workspace.numel(),
-                     torch.cuda.current_stream(posm.device).cuda_stream)
+                     stages.current_stream(posm.device))
 
 
 def vjp_shard_cfg(n, m):
@@ -131,7 +131,7 @@ def stage1_vjp_shard_f32(posm, mu4, rho, gamma, i0, G, eps, dt, cfg=None, worksp
         _native.call('grav_stage1_vjp_f32_shard', posm.data_ptr(), mu4.data_ptr(),
                      rho.data_ptr(), gamma.data_ptr(), n, int(i0), m, float(G), float(eps),
                      float(dt), int(cfg[0]), int(cfg[1]), int(cfg[2]), ptr, size,
-                     torch.cuda.current_stream(posm.device).cuda_stream)
+                     stages.current_stream(posm.device))
 
 
 def stage1_vjp_split_chain(posm, mu4, rho, nu, gamma, G, eps, dt, next_mu, eslot, cfg=None,
@@ -159,7 +159,7 @@ def stage1_vjp_split_chain(posm, mu4, rho, nu, gamma, G, eps, dt, next_mu, eslot
                      rho.data_ptr(), nu.data_ptr(), gamma.data_ptr(), n, float(G), float(eps),
                      float(dt), int(k), int(s), int(p), 1 if next_mu else 0,
                      workspace.data_ptr(), workspace.numel(), eslot.data_ptr(),
-                     torch.cuda.current_stream(posm.device).cuda_stream)
+                     stages.current_stream(posm.device))
 
 
 def backward_pair_workspace_bytes(n, cfg=None):
@@ -198,7 +198,7 @@ def backward_pair_split(posm_adj, mu4, rho, nu, gamma, eslot, pos_in, pos_out, r
                      pos_in.data_ptr(), pos_out.data_ptr(), r64.data_ptr(), v64.data_ptr(), n,
                      float(G), float(eps), float(dt), int(ka), int(pa), int(kr), int(pr), int(w),
                      workspace.data_ptr(), workspace.numel(),
-                     torch.cuda.current_stream(posm_adj.device).cuda_stream)
+                     stages.current_stream(posm_adj.device))
 
 
 def default_budget(device):

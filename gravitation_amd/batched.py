@@ -144,7 +144,7 @@ class BatchedPlan:
 
 
 def _stream(dev):
-    return torch.cuda.current_stream(dev).cuda_stream
+    return stages.current_stream(torch.device(dev))
 
 
 def _check_mode(mode, sym):

@@ -43,4 +43,10 @@ int grav_device_count(int *count) {
   return GRAV_OK;
 }
 
+int grav_stream_synchronize(void *stream) {
+  grav::clear_error();
+  GRAV_HIP_CHECK(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
+  return GRAV_OK;
+}
+
 }  // extern "C"

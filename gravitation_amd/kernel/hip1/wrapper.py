@@ -279,12 +279,15 @@ class universe(universe_base):
             else:
                 c2 = ('grav_stage2_f32', (p, v, a, n, T))
         self._direct = [(getattr(lib, name), name, args) for name, args in (c1, c2)]
+        self._wait = lib.grav_stream_synchronize
 
     def _call(self, k):
-        import torch
-        fn, name, args = self._direct[k]
+        self._run(*self._direct[k])
+
+    def _run(self, fn, name, args=()):
+        """fn(*args, stream) on the universe's device and torch's current stream there."""
         with self._stages.on_device(self._device):
-            rc = fn(*args, torch.cuda.current_stream(self._device).cuda_stream)
+            rc = fn(*args, self._stages.current_stream(self._device))
         if rc:
             from gravitation_amd import _native
             _native.check(name, rc)
@@ -342,13 +345,12 @@ class universe(universe_base):
             self._call(0)
 
     def step_stage2(self):
-        import torch
         if self._graphs is not None:
             self._graphs[1].replay()
         else:
             self._call(1)   # with sync_host, the stage-2 kernel also writes the host mirror
         if self._sync_host:
-            torch.cuda.current_stream(self._device).synchronize()
+            self._run(self._wait, 'grav_stream_synchronize')
 
     def stop_kernel(self):
         import torch

@@ -54,6 +54,9 @@ const char *grav_last_error(void);
 /* Number of visible HIP devices (0 if none); returns GRAV_OK even when 0. */
 int grav_device_count(int *count);
 
+/* Waits for the work on `stream` (of the current device) to finish. */
+int grav_stream_synchronize(void *stream);
+
 /*
  * Stage 1, FP32 pair terms: acc[3*n] <- G * sum_j m_j d_ij (d^2 + eps^2)^-3/2.
  * Replaces `step_stage1(struct univ*)` (src/gravitation/kernel/_lib1_/lib.c:52-126) and the
