@@ -506,6 +506,13 @@ class _Single(torch.autograd.Function):
         traj = torch.empty((steps, n, 4), dtype=torch.float32, device=dev) if store else None
         checkpoints = []
         t = 0
+        if store and steps > 0 and _stage1_form(n, form) == 'split':
+            # a step goes from one slot of the record to the next, the last one back into posm
+            traj[0].copy_(posm)
+            for t in range(steps):
+                stages.step_split_f64m(traj[t], r64, v64, G, eps, dt,
+                                       out=traj[t + 1] if t + 1 < steps else posm)
+            t = steps
         while t < steps:
             if store:
                 traj[t].copy_(posm)
