@@ -72,7 +72,7 @@ struct grav_batched_plan {
   int *seg_begin = nullptr;        // [groups + 1]
   int *bin_bodies = nullptr;       // [groups]
   int64_t *offsets = nullptr;      // [U + 1] (host copy kept below)
-  int4 *items = nullptr;           // per-step path: {i0, i1, j0, j1} per i-tile, largest first
+  int4 *items = nullptr;           // per-step path: {i0, i1, j0, j1} per i-tile
   int nitems = 0;
   bool fused_ok = false;           // the fused schedule exists (every universe fits a group)
   char fused_why[256] = "";
@@ -682,7 +682,13 @@ int grav_batched_plan_create(const int64_t *offsets, int n_universes, int waves_
   seg_begin[groups] = static_cast<int>(segs.size());
 
   // Per-step path: every universe's i-tiles of 64*i_per_lane bodies against the universe's
-  // own bodies, costliest (largest universe) first so the long tiles start early.
+  // own bodies, costliest (largest universe) first so the long tiles start early, and every
+  // other row of one item per compute unit backwards: the workgroups of a launch go to the
+  // compute units in turn, so with the rows all falling the first unit of each row got the row's
+  // costliest item every time (128 universes of 64-2048 bodies, 4.8 items per unit: 21 % more
+  // pairs on the busiest unit than on the mean one, 4 % back and forth).  MI355X, falling and back
+  // and forth: forward and backward of those over 12 steps 1.184 and 1.133 ms, 500 universes
+  // of 64-600 bodies over 10 steps 162.6 and 158.2 us, 1024 of 32-2048 bodies 1.291 and 1.274 ms.
   std::vector<int4> items;
   for (int u : order) {
     const int g0 = static_cast<int>(offsets[u]);
@@ -690,6 +696,8 @@ int grav_batched_plan_create(const int64_t *offsets, int n_universes, int waves_
     for (int t0 = 0; t0 < s; t0 += tile_len)
       items.push_back(make_int4(g0 + t0, g0 + std::min(s, t0 + tile_len), g0, g0 + s));
   }
+  for (size_t row = cus; row + cus <= items.size(); row += 2 * cus)
+    std::reverse(items.begin() + row, items.begin() + row + cus);
 
   grav_batched_plan *p = new (std::nothrow) grav_batched_plan();
   GRAV_REQUIRE(p != nullptr, "grav_batched_plan_create: out of host memory");
