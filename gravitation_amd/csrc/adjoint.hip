@@ -197,17 +197,18 @@ __global__ __launch_bounds__(256) void k_adjoint_mu_scale(const double *__restri
   }
 }
 
-template <int K, bool MASK>
+template <int K, bool MASK, typename Mine, typename Fold>
 __device__ __forceinline__ void vjp_segment(const float4 *__restrict__ posm,
                                             const float4 *__restrict__ mu4, int j0, int j1,
                                             int jblock, const float (&xk)[K],
                                             const float (&yk)[K], const float (&zk)[K],
                                             const float (&mk)[K], const float (&uxk)[K],
                                             const float (&uyk)[K], const float (&uzk)[K],
-                                            const int (&kk)[K], float eps2, float (&hi)[4][K],
-                                            float (&lo)[4][K]) {
+                                            const int (&kk)[K], float eps2, Mine &&mine,
+                                            Fold &&fold) {
   for (int jb = j0, je; jb < j1; jb = je) {
     je = (j1 - jb > jblock) ? jb + jblock : j1;
+    if (!mine(jb, je)) continue;
     float px[K], py[K], pz[K], pg[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) px[k] = py[k] = pz[k] = pg[k] = 0.0f;
@@ -275,13 +276,7 @@ __device__ __forceinline__ void vjp_segment(const float4 *__restrict__ posm,
     for (; j < je; ++j)
       vjp_pair<K, MASK>(posm[j], mu4[j], j, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2, px, py, pz,
                         pg);
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      two_sum_acc(hi[0][k], lo[0][k], px[k]);
-      two_sum_acc(hi[1][k], lo[1][k], py[k]);
-      two_sum_acc(hi[2][k], lo[2][k], pz[k]);
-      two_sum_acc(hi[3][k], lo[3][k], pg[k]);
-    }
+    fold(px, py, pz, pg);
   }
 }
 
@@ -297,14 +292,18 @@ __device__ __forceinline__ void vjp_segment(const float4 *__restrict__ posm,
 // moves the exponent that the previous chained reduce gathered, eslot[1], to eslot[0], where
 // this step's reduce reads it (none gathered yet: mu4's own exponent), and clears eslot[1] for
 // this step's reduce to gather into.  Nothing in this kernel reads eslot otherwise.
-template <int K, int S>
+// HALVES = 2: 2 S wavefronts, see halves_of; slots is half_slots, and red is larger by
+// S * slots * 4 * (64 * K) floats.
+template <int K, int S, int HALVES = 1>
 __device__ __forceinline__ void stage1_vjp_f32_block(
     const float4 *__restrict__ posm, const float4 *__restrict__ mu4, double *__restrict__ rho,
     double *__restrict__ gamma, int n, int i0, int m, double hG, float eps2, int jblock,
     const int4 *__restrict__ items, double *__restrict__ part, unsigned *__restrict__ eslot,
-    int bx, int by, int ny, float *red) {
+    int bx, int by, int ny, float *red, int slots = 0) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int any = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int half = HALVES == 2 && any >= S ? 1 : 0;
+  const int wave = any - half * S;
   if (eslot != nullptr && bx == 0 && by == 0 && threadIdx.x == 0) {
     const unsigned b = eslot[1];
     eslot[0] = b != 0u ? b : exp_bias(__float_as_int(mu4[0].w));
@@ -329,6 +328,11 @@ __device__ __forceinline__ void stage1_vjp_f32_block(
       jhi = min(n, jlo + span);
     }
   }
+  const int chunk = ((jhi - jlo + S - 1) / S + 3) & ~3;
+  const int j0 = min(jhi, jlo + wave * chunk);
+  const int j1 = min(jhi, j0 + chunk);
+  const bool shared = HALVES == 2 && j1 - j0 > jblock;
+  if (half != 0 && !shared) return;
   float xk[K], yk[K], zk[K], mk[K], uxk[K], uyk[K], uzk[K];
   int kk[K], ek[K];
 #pragma unroll
@@ -353,9 +357,6 @@ __device__ __forceinline__ void stage1_vjp_f32_block(
 #pragma unroll
     for (int k = 0; k < K; ++k) hi[c][k] = lo[c][k] = 0.0f;
 
-  const int chunk = ((jhi - jlo + S - 1) / S + 3) & ~3;
-  const int j0 = min(jhi, jlo + wave * chunk);
-  const int j1 = min(jhi, j0 + chunk);
   {
     // the masked segment is the workgroup's own bodies, so the compensation blocks depend on
     // where its i-tile starts: a share's rows equal the whole universe's bit for bit when the
@@ -365,17 +366,75 @@ __device__ __forceinline__ void stage1_vjp_f32_block(
     // eps2 in a VGPR, so that the first r2 FMA takes no SGPR operand (2^18 j-split VJP:
     // 34.85 against 35.27-35.37 ms)
     const float eps2v = in_vgpr(eps2);
-    vjp_segment<K, false>(posm, mu4, j0, a, jblock, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2v, hi,
-                          lo);
-    vjp_segment<K, true>(posm, mu4, a, b, jblock, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2v, hi,
-                         lo);
-    vjp_segment<K, false>(posm, mu4, b, j1, jblock, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2v, hi,
-                          lo);
+    auto fold = [&](const float (&px)[K], const float (&py)[K], const float (&pz)[K],
+                    const float (&pg)[K]) {
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        two_sum_acc(hi[0][k], lo[0][k], px[k]);
+        two_sum_acc(hi[1][k], lo[1][k], py[k]);
+        two_sum_acc(hi[2][k], lo[2][k], pz[k]);
+        two_sum_acc(hi[3][k], lo[3][k], pg[k]);
+      }
+    };
+    auto segments = [&](auto &&mine, auto &&f) {
+      vjp_segment<K, false>(posm, mu4, j0, a, jblock, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2v,
+                            mine, f);
+      vjp_segment<K, true>(posm, mu4, a, b, jblock, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2v,
+                           mine, f);
+      vjp_segment<K, false>(posm, mu4, b, j1, jblock, xk, yk, zk, mk, uxk, uyk, uzk, kk, eps2v,
+                            mine, f);
+    };
+    if constexpr (HALVES == 2) {
+      // the blocks whose middle lies in the second half of [j0, j1) are the other wavefront's
+      constexpr int B = 4 * kWave * K;
+      __shared__ int count[S];
+      float *h = red + (S - 1) * 8 * kWave * K + wave * slots * B + lane;
+      const int twice = j0 + j1;
+      if (half == 0) {
+        segments([&](int p, int q) { return !shared || p + q < twice; }, fold);
+      } else {
+        int nb = 0;
+        segments([&](int p, int q) { return p + q >= twice; },
+                 [&](const float (&px)[K], const float (&py)[K], const float (&pz)[K],
+                     const float (&pg)[K]) {
+                   float *o = h + nb * B;
+#pragma unroll
+                   for (int k = 0; k < K; ++k) {
+                     o[(4 * k) * kWave] = px[k];
+                     o[(4 * k + 1) * kWave] = py[k];
+                     o[(4 * k + 2) * kWave] = pz[k];
+                     o[(4 * k + 3) * kWave] = pg[k];
+                   }
+                   ++nb;
+                 });
+        if (lane == 0) count[wave] = nb;
+      }
+      __syncthreads();
+      if (half == 0 && shared) {
+        const int nb = count[wave];
+        for (int t = 0; t < nb; ++t, h += B) {
+          float px[K], py[K], pz[K], pg[K];
+#pragma unroll
+          for (int k = 0; k < K; ++k) {
+            px[k] = h[(4 * k) * kWave];
+            py[k] = h[(4 * k + 1) * kWave];
+            pz[k] = h[(4 * k + 2) * kWave];
+            pg[k] = h[(4 * k + 3) * kWave];
+          }
+          fold(px, py, pz, pg);
+        }
+      }
+      if constexpr (S == 1) {
+        if (half != 0) return;
+      }
+    } else {
+      segments([](int, int) { return true; }, fold);
+    }
   }
 
   if constexpr (S > 1) {
     constexpr int L = kWave * K;
-    if (wave > 0) {
+    if (wave > 0 && half == 0) {
       float *r = red + (wave - 1) * 8 * L;
 #pragma unroll
       for (int c = 0; c < 4; ++c)
@@ -386,7 +445,7 @@ __device__ __forceinline__ void stage1_vjp_f32_block(
         }
     }
     __syncthreads();
-    if (wave != 0) return;
+    if (any != 0) return;
     for (int w = 1; w < S; ++w) {
       const float *r = red + (w - 1) * 8 * L;
 #pragma unroll
@@ -427,15 +486,17 @@ __device__ __forceinline__ void stage1_vjp_f32_block(
 }
 
 // Workgroup (blockIdx.x, blockIdx.y) of stage1_vjp_f32_block.
-template <int K, int S>
-__global__ __launch_bounds__(kWave *S) void k_stage1_vjp_f32(
+template <int K, int S, int HALVES>
+__global__ __launch_bounds__(kWave *S *HALVES) void k_stage1_vjp_f32(
     const float4 *__restrict__ posm, const float4 *__restrict__ mu4, double *__restrict__ rho,
     double *__restrict__ gamma, int n, int i0, int m, double hG, float eps2, int jblock,
-    const int4 *__restrict__ items, double *__restrict__ part, unsigned *__restrict__ eslot) {
-  extern __shared__ float red[];  // (S - 1) * 8 * (64 * K)
-  stage1_vjp_f32_block<K, S>(posm, mu4, rho, gamma, n, i0, m, hG, eps2, jblock, items, part,
-                             eslot, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y),
-                             static_cast<int>(gridDim.y), red);
+    const int4 *__restrict__ items, double *__restrict__ part, unsigned *__restrict__ eslot,
+    int slots) {
+  extern __shared__ float red[];  // (S - 1) * 8 * (64 * K), halves: and S * slots * 4 * (64 * K)
+  stage1_vjp_f32_block<K, S, HALVES>(posm, mu4, rho, gamma, n, i0, m, hG, eps2, jblock, items,
+                                     part, eslot, static_cast<int>(blockIdx.x),
+                                     static_cast<int>(blockIdx.y), static_cast<int>(gridDim.y),
+                                     red, slots);
 }
 
 // Component c of body i: rho[c][i] += hs * sum_p part[p][c][i] (c < 3) or gamma[i] -= hs * sum_p
@@ -586,15 +647,25 @@ __global__ __launch_bounds__(4 * kReduceBodies) void k_backward_pair_reduce(
 // i-tiles of the share [i0, i0 + m) (items == NULL) or the nitems items.
 template <int K, int S>
 int launch_vjp(const float4 *posm, const float4 *mu4, double *rho, double *gamma, int n, int i0,
-               int m, double hG, float eps2, const int4 *items, int nitems,
+               int m, double hG, float eps2, const int4 *items, int nitems, int max_bodies,
                hipStream_t stream) {
   const int per_block = kWave * K;
   const int grid = items ? nitems : (m + per_block - 1) / per_block;
   const size_t lds = (S > 1) ? sizeof(float) * (S - 1) * 8 * per_block : 0;
   if (grid == 0) return GRAV_OK;
-  hipLaunchKernelGGL((k_stage1_vjp_f32<K, S>), dim3(grid), dim3(kWave * S), lds, stream, posm,
+  if constexpr (K == 1) {
+    if (items != nullptr && nitems <= kHalvesVjpItems && halves_of(max_bodies, S)) {
+      const int slots = half_slots(max_bodies, S);
+      hipLaunchKernelGGL((k_stage1_vjp_f32<K, S, 2>), dim3(grid), dim3(2 * kWave * S),
+                         lds + sizeof(float) * S * slots * 4 * kWave, stream, posm, mu4, rho,
+                         gamma, n, i0, m, hG, eps2, 256, items, static_cast<double *>(nullptr),
+                         static_cast<unsigned *>(nullptr), slots);
+      return check_launch("k_stage1_vjp_f32 (halves)");
+    }
+  }
+  hipLaunchKernelGGL((k_stage1_vjp_f32<K, S, 1>), dim3(grid), dim3(kWave * S), lds, stream, posm,
                      mu4, rho, gamma, n, i0, m, hG, eps2, 256, items,
-                     static_cast<double *>(nullptr), static_cast<unsigned *>(nullptr));
+                     static_cast<double *>(nullptr), static_cast<unsigned *>(nullptr), 0);
   return check_launch("k_stage1_vjp_f32");
 }
 
@@ -605,10 +676,10 @@ int launch_vjp_split(const float4 *posm, const float4 *mu4, double *part, int n,
   const int per_block = kWave * K;
   const int tiles = (m + per_block - 1) / per_block;
   const size_t lds = (S > 1) ? sizeof(float) * (S - 1) * 8 * per_block : 0;
-  hipLaunchKernelGGL((k_stage1_vjp_f32<K, S>), dim3(tiles, splits), dim3(kWave * S), lds,
+  hipLaunchKernelGGL((k_stage1_vjp_f32<K, S, 1>), dim3(tiles, splits), dim3(kWave * S), lds,
                      stream, posm, mu4, static_cast<double *>(nullptr),
                      static_cast<double *>(nullptr), n, i0, m, 0.0, eps2, 256,
-                     static_cast<const int4 *>(nullptr), part, eslot);
+                     static_cast<const int4 *>(nullptr), part, eslot, 0);
   return check_launch("k_stage1_vjp_f32 (j-split)");
 }
 
@@ -623,10 +694,11 @@ int adjoint_mu_launch(const double *rho, double *nu, float4 *mu4, int n, double 
 
 int stage1_vjp_launch(const float4 *posm, const float4 *mu4, double *rho, double *gamma, int n,
                       double hG, float eps2, int K, int S, const int4 *items, int nitems,
-                      hipStream_t stream) {
+                      int max_bodies, hipStream_t stream) {
 #define GRAV_CASE(KK, SS)                                                                     \
   if (K == KK && S == SS)                                                                     \
-    return launch_vjp<KK, SS>(posm, mu4, rho, gamma, n, 0, n, hG, eps2, items, nitems, stream);
+    return launch_vjp<KK, SS>(posm, mu4, rho, gamma, n, 0, n, hG, eps2, items, nitems,        \
+                              max_bodies, stream);
   GRAV_CASE(1, 1) GRAV_CASE(1, 2) GRAV_CASE(1, 4) GRAV_CASE(1, 8)
   GRAV_CASE(2, 1) GRAV_CASE(2, 2) GRAV_CASE(2, 4) GRAV_CASE(2, 8)
   GRAV_CASE(4, 1) GRAV_CASE(4, 2) GRAV_CASE(4, 4)
@@ -670,7 +742,7 @@ int stage1_vjp_shard_launch(const float4 *posm, const float4 *mu4, double *rho, 
   if (splits == 1) {
 #define GRAV_CASE(KK, SS)                                                                   \
   if (K == KK && S == SS)                                                                   \
-    return launch_vjp<KK, SS>(posm, mu4, rho, gamma, n, i0, m, hG, eps2, nullptr, 0, stream);
+    return launch_vjp<KK, SS>(posm, mu4, rho, gamma, n, i0, m, hG, eps2, nullptr, 0, 0, stream);
     GRAV_CASE(1, 1) GRAV_CASE(1, 2) GRAV_CASE(1, 4) GRAV_CASE(1, 8)
     GRAV_CASE(2, 1) GRAV_CASE(2, 2) GRAV_CASE(2, 4) GRAV_CASE(2, 8)
     GRAV_CASE(4, 1) GRAV_CASE(4, 2) GRAV_CASE(4, 4)
@@ -822,7 +894,7 @@ int grav_stage1_vjp_f32(const void *posm, const void *mu4, void *rho64, void *ga
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int K = n >= (1 << 16) ? 4 : (n >= (1 << 13) ? 2 : 1);
   const int S = n >= (1 << 13) ? 4 : 8;
-  return stage1_vjp_launch(p, u, rho, gam, nn, dt * G, eps2, K, S, nullptr, 0, s);
+  return stage1_vjp_launch(p, u, rho, gam, nn, dt * G, eps2, K, S, nullptr, 0, 0, s);
 }
 
 int grav_stage1_vjp_f32_split(const void *posm, const void *mu4, void *rho64, void *gamma64,

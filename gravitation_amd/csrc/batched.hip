@@ -835,7 +835,8 @@ int grav_batched_step_items_f32(const grav_batched_plan *plan, const void *posm_
                                 static_cast<double *>(v64), static_cast<int>(plan->n_bodies),
                                 static_cast<float>(G), static_cast<float>(eps * eps),
                                 eps == 0.0 ? 1 : 0, dt, plan->kt, j_waves, plan->items,
-                                plan->nitems, static_cast<hipStream_t>(stream));
+                                plan->nitems, static_cast<int>(plan->max_universe),
+                                static_cast<hipStream_t>(stream));
 }
 
 int grav_batched_sym_prepare(grav_batched_plan *plan, int i_chunks_per_wave, int waves) {
@@ -985,7 +986,8 @@ int grav_batched_stage1_vjp_f32(const grav_batched_plan *plan, const void *posm,
                            static_cast<double *>(rho64), static_cast<double *>(gamma64),
                            static_cast<int>(plan->n_bodies), dt * G,
                            static_cast<float>(eps * eps), plan->kt, j_waves, plan->items,
-                           plan->nitems, static_cast<hipStream_t>(stream));
+                           plan->nitems, static_cast<int>(plan->max_universe),
+                           static_cast<hipStream_t>(stream));
 }
 
 int grav_batched_adjoint_f32(const grav_batched_plan *plan, const void *traj, void *rho64,

@@ -89,10 +89,11 @@ int stage1_f32_launch(const float4 *posm, float *acc, int n, float G, float eps2
 
 // One step of the items' bodies in one launch: stage1_f32_launch's accelerations, then the
 // FP64-master stage 2, bit for bit the two kernels'; the new positions go to out, which must not
-// overlap posm.  K in {1,2,4}, S in {1,2,4,8}.  (stage1.hip)
+// overlap posm.  K in {1,2,4}, S in {1,2,4,8}; max_bodies: the longest j-range of an item.
+// (stage1.hip)
 int step_items_f64m_launch(const float4 *posm, float4 *out, double *r64, double *v64, int n,
                            float G, float eps2, int mask, double dt, int K, int S,
-                           const int4 *items, int nitems, hipStream_t stream);
+                           const int4 *items, int nitems, int max_bodies, hipStream_t stream);
 
 // Unscaled FP32 sums of the bodies [i0, i0 + m) against their own blocks of diag_block bodies
 // (i0 and diag_block multiples of 256), into acc (3, m): the block-diagonal pass of the
@@ -106,10 +107,11 @@ int stage1_f32_diag_launch(const float4 *posm, float *acc, int n, int i0, int m,
 int adjoint_mu_launch(const double *rho, double *nu, float4 *mu4, int n, double dt,
                       const int64_t *offsets, int n_universes, hipStream_t stream);
 
-// VJP of stage 1 over an item list with the same convention (K in {1,2,4}). (adjoint.hip)
+// VJP of stage 1 over an item list with the same convention (K in {1,2,4}); max_bodies: the
+// longest j-range of an item. (adjoint.hip)
 int stage1_vjp_launch(const float4 *posm, const float4 *mu4, double *rho, double *gamma, int n,
                       double hG, float eps2, int K, int S, const int4 *items, int nitems,
-                      hipStream_t stream);
+                      int max_bodies, hipStream_t stream);
 
 // j-split form of the owner-computes stage 1 and of its VJP, for universes too small to fill
 // the GPU with i-tiles: a (tiles x splits) grid, each workgroup one i-tile of 64*K bodies

@@ -216,28 +216,42 @@ __global__ __launch_bounds__(kWave *S) void k_stage1_f64(const double4 *__restri
 // bytes per body, and, for a record, a copy of the positions.  MI355X, two launches and one: 1024
 // universes of 32-2048 bodies 0.136 and 0.130 ms per step, forward and backward of 128
 // universes over 12 steps 1.22 and 1.16 ms.
-template <int K, int S, int JB>
-__global__ __launch_bounds__(kWave *S) void k_step_items_f64m(const float4 *__restrict__ posm,
-                                                               int n, float G, float eps2,
-                                                               int mask_self,
-                                                               const int4 *__restrict__ items,
-                                                               StepIO io) {
-  extern __shared__ float red[];  // (S - 1) * 6 * (64 * K)
-  stage1_f32_block<K, S, JB, true>(posm, nullptr, n, 0, n, G, eps2, mask_self, 256, items, 0,
-                                   nullptr, static_cast<int>(blockIdx.x), 0, 1, red, io);
+template <int K, int S, int JB, int HALVES>
+__global__ __launch_bounds__(kWave *S *HALVES) void k_step_items_f64m(
+    const float4 *__restrict__ posm, int n, float G, float eps2, int mask_self,
+    const int4 *__restrict__ items, StepIO io, int slots) {
+  extern __shared__ float red[];  // (S - 1) * 6 * (64 * K), halves: and S * slots * 3 * (64 * K)
+  stage1_f32_block<K, S, JB, true, HALVES>(posm, nullptr, n, 0, n, G, eps2, mask_self, 256,
+                                           items, 0, nullptr, static_cast<int>(blockIdx.x), 0, 1,
+                                           red, io, slots);
 }
 
 template <int K, int S>
 int launch_step_items(const float4 *posm, int n, float G, float eps2, int mask,
-                      const int4 *items, int nitems, const StepIO &io, hipStream_t stream) {
+                      const int4 *items, int nitems, int max_bodies, const StepIO &io,
+                      hipStream_t stream) {
   const size_t lds = (S > 1) ? sizeof(float) * (S - 1) * 6 * kWave * K : 0;
   constexpr int kNarrow = K >= 4 ? 8 : K == 1 ? 4 : 2;   // pair_loop_width's other value
+  if constexpr (K == 1) {
+    if (nitems <= kHalvesStepItems && halves_of(max_bodies, S)) {
+      const int slots = half_slots(max_bodies, S);
+      const size_t more = sizeof(float) * S * slots * 3 * kWave;
+      if (pair_loop_width(nitems, K, false) == 8)
+        hipLaunchKernelGGL((k_step_items_f64m<K, S, 8, 2>), dim3(nitems), dim3(2 * kWave * S),
+                           lds + more, stream, posm, n, G, eps2, mask, items, io, slots);
+      else
+        hipLaunchKernelGGL((k_step_items_f64m<K, S, kNarrow, 2>), dim3(nitems),
+                           dim3(2 * kWave * S), lds + more, stream, posm, n, G, eps2, mask, items,
+                           io, slots);
+      return check_launch("k_step_items_f64m (halves)");
+    }
+  }
   if (pair_loop_width(nitems, K, false) == 8)
-    hipLaunchKernelGGL((k_step_items_f64m<K, S, 8>), dim3(nitems), dim3(kWave * S), lds, stream,
-                       posm, n, G, eps2, mask, items, io);
+    hipLaunchKernelGGL((k_step_items_f64m<K, S, 8, 1>), dim3(nitems), dim3(kWave * S), lds,
+                       stream, posm, n, G, eps2, mask, items, io, 0);
   else
-    hipLaunchKernelGGL((k_step_items_f64m<K, S, kNarrow>), dim3(nitems), dim3(kWave * S), lds,
-                       stream, posm, n, G, eps2, mask, items, io);
+    hipLaunchKernelGGL((k_step_items_f64m<K, S, kNarrow, 1>), dim3(nitems), dim3(kWave * S), lds,
+                       stream, posm, n, G, eps2, mask, items, io, 0);
   return check_launch("k_step_items_f64m");
 }
 
@@ -393,11 +407,13 @@ int launch_f32_ks(int K, int S, const float4 *posm, float *acc, int n, int i0, i
 
 int step_items_f64m_launch(const float4 *posm, float4 *out, double *r64, double *v64, int n,
                            float G, float eps2, int mask, double dt, int K, int S,
-                           const int4 *items, int nitems, hipStream_t stream) {
+                           const int4 *items, int nitems, int max_bodies,
+                           hipStream_t stream) {
   const StepIO io{out, r64, v64, dt};
 #define GRAV_STEP(KK, SS) \
   if (K == KK && S == SS)  \
-    return launch_step_items<KK, SS>(posm, n, G, eps2, mask, items, nitems, io, stream);
+    return launch_step_items<KK, SS>(posm, n, G, eps2, mask, items, nitems, max_bodies, io, \
+                                     stream);
   GRAV_STEP(1, 1) GRAV_STEP(1, 2) GRAV_STEP(1, 4) GRAV_STEP(1, 8)
   GRAV_STEP(2, 1) GRAV_STEP(2, 2) GRAV_STEP(2, 4) GRAV_STEP(2, 8)
   GRAV_STEP(4, 1) GRAV_STEP(4, 2) GRAV_STEP(4, 4) GRAV_STEP(4, 8)

@@ -130,14 +130,14 @@ __device__ __forceinline__ void pair_range_f32(const float4 *__restrict__ posm, 
 // workgroup's own i-range) run the self-masked pair routine.  That choice does not change a
 // pair's value for j != i, and the blocks start at j0 whatever [ma, mb) is, so a body's sum
 // does not depend on which i-tile holds it.
-template <int K, bool MASK, int JB>
+// fold(px, py, pz) takes each block's sums, in order.
+template <int K, bool MASK, int JB, typename Fold>
 __device__ __forceinline__ void sum_segment_f32(const float4 *__restrict__ posm, int j0, int j1,
                                                 int jblock, int ma, int mb,
                                                 const float (&xi)[K],
                                                 const float (&yi)[K], const float (&zi)[K],
                                                 const int (&ii)[K], const float eps2,
-                                                float (&hx)[K], float (&hy)[K], float (&hz)[K],
-                                                float (&lx)[K], float (&ly)[K], float (&lz)[K]) {
+                                                Fold &&fold) {
   for (int jb = j0, je; jb < j1; jb = je) {
     je = (j1 - jb > jblock) ? jb + jblock : j1;  // no overflow for jblock near INT_MAX
     float px[K], py[K], pz[K];
@@ -152,13 +152,40 @@ __device__ __forceinline__ void sum_segment_f32(const float4 *__restrict__ posm,
     } else {
       pair_range_f32<K, false, JB>(posm, jb, je, xi, yi, zi, ii, eps2, px, py, pz);
     }
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      two_sum_fold(hx[k], lx[k], px[k]);
-      two_sum_fold(hy[k], ly[k], py[k]);
-      two_sum_fold(hz[k], lz[k], pz[k]);
-    }
+    fold(px, py, pz);
   }
+}
+
+// Halves of the item-list forms (one body per lane).  A wavefront sums its j-range block after
+// block of 256 bodies, so a batch of few universes lasts as long as the blocks of its largest one:
+// 2048 bodies and four wavefronts, two blocks of 256 pairs that one wavefront alone issues at
+// half the rate of two.  In halves a workgroup has a second set of wavefronts: each takes over the
+// blocks of the second half of its counterpart's range and leaves their sums in LDS, and the
+// first folds them in after its own in the same order, so the bits are those of one wavefront.
+// A wavefront whose counterpart has one block or none ends at once.  Taken where there is a
+// second block (up to 1024 j-bodies per wavefront, for the sums' LDS) and the launch is
+// small: with wavefronts enough on every SIMD the second set gives nothing and costs its
+// workgroups' slots.  MI355X, without and with, forward and backward over 8 or 12 steps:
+// 30 universes of 64-2048 bodies (289 items) 0.728 and 0.501 ms, 60 of 32-1500 (392) 0.575
+// and 0.464, 100 of 100-1200 (743) 0.499 and 0.453, 128 of 64-2048 (1219) 1.131 and 1.090, 200
+// of 100-1200 (1482) 0.570 and 0.592; forward alone over 10 steps: 200 of 32-2048 (1619)
+// 0.366 and 0.332, 400 (3227) 0.550 and 0.572; over 20 steps 10 of 64-2048 (102) 0.631 and 0.370.
+constexpr int kHalvesStepItems = 2048;   // largest launches in halves, of steps
+constexpr int kHalvesVjpItems = 1280;    // and of VJPs
+constexpr int kHalvesChunk = 1024;
+
+// Whether the longest j-range of a wavefront has a second block and at most kHalvesChunk bodies.
+inline bool halves_of(int max_bodies, int S) {
+  const int chunk = ((max_bodies + S - 1) / S + 7) & ~7;
+  return chunk > 256 && chunk <= kHalvesChunk;
+}
+
+// Block sums that a wavefront of the second set leaves at most: the blocks whose middle lies in
+// the second half of a range of `chunk` bodies start in its last chunk / 2 + 128 bodies, and
+// the VJP's own-tile segment divides them into three segments, each with a rounded-up number.
+inline int half_slots(int max_bodies, int S) {
+  const int chunk = ((max_bodies + S - 1) / S + 7) & ~7;
+  return (chunk / 2 + 128) / 256 + 3;
 }
 
 // The FP64-master stage 2 of body i from its FP32 acceleration a, without contraction as
@@ -202,7 +229,9 @@ struct StepIO {
 // STEP (with items): instead of acc, the bodies' FP64-master stage 2 into io, bit for bit
 // k_stage1_f32 followed by k_stage2_f64m.  With one body per lane the masters are loaded before
 // the pair loop.
-template <int K, int S, int JB, bool STEP = false>
+// HALVES = 2: 2 S wavefronts, see halves_of; slots is half_slots, and red is larger by
+// S * slots * 3 * (64 * K) floats.
+template <int K, int S, int JB, bool STEP = false, int HALVES = 1>
 __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm,
                                                  float *__restrict__ acc, int n, int i0, int m,
                                                  float G, float eps2, int mask_self,
@@ -210,9 +239,11 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
                                                  const int4 *__restrict__ items,
                                                  int diag_block, double *__restrict__ part,
                                                  int bx, int by, int ny, float *red,
-                                                 const StepIO io = StepIO{}) {
+                                                 const StepIO io = StepIO{}, int slots = 0) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int any = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int half = HALVES == 2 && any >= S ? 1 : 0;
+  const int wave = any - half * S;
   int ibase, iend, jlo, jhi;
   if (items != nullptr) {
     const int4 it = items[bx];
@@ -234,6 +265,15 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
     }
   }
 
+  // This wave's j-range; with mask_self the pairs with j in the workgroup's own i-range
+  // [ibase, iend) are self-masked.
+  const int chunk = ((jhi - jlo + S - 1) / S + 7) & ~7;
+  const int j0 = min(jhi, jlo + wave * chunk);
+  const int j1 = min(jhi, j0 + chunk);
+  if constexpr (HALVES == 2) {
+    if (half != 0 && j1 - j0 <= jblock) return;   // one block or none: nothing to take over
+  }
+
   float xi[K], yi[K], zi[K];
   int ii[K];
 #pragma unroll
@@ -248,7 +288,7 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
 
   double mr[3], mv[3];
   if constexpr (STEP && K == 1) {
-    if (wave == 0) {
+    if (any == 0) {
       const int ic = min(ii[0], iend - 1);
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
@@ -262,24 +302,65 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
 #pragma unroll
   for (int k = 0; k < K; ++k) hx[k] = hy[k] = hz[k] = lx[k] = ly[k] = lz[k] = 0.0f;
 
-  // This wave's j-range; with mask_self the pairs with j in the workgroup's own i-range
-  // [ibase, iend) are self-masked.
-  const int chunk = ((jhi - jlo + S - 1) / S + 7) & ~7;
-  const int j0 = min(jhi, jlo + wave * chunk);
-  const int j1 = min(jhi, j0 + chunk);
   // eps2 in a VGPR, so that the first r2 FMA takes no SGPR operand (an SGPR operand adds
   // issue cycles to an FP32 instruction): 2^18 with (1, 16) 16.86 against 17.14 ms
   const float eps2v = in_vgpr(eps2);
-  if (mask_self)
-    sum_segment_f32<K, true, JB>(posm, j0, j1, jblock, ibase, iend, xi, yi, zi, ii, eps2v, hx,
-                                 hy, hz, lx, ly, lz);
-  else
-    sum_segment_f32<K, false, JB>(posm, j0, j1, jblock, 0, 0, xi, yi, zi, ii, eps2v, hx, hy,
-                                  hz, lx, ly, lz);
+  auto fold = [&](const float (&px)[K], const float (&py)[K], const float (&pz)[K]) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      two_sum_fold(hx[k], lx[k], px[k]);
+      two_sum_fold(hy[k], ly[k], py[k]);
+      two_sum_fold(hz[k], lz[k], pz[k]);
+    }
+  };
+  const int ma = mask_self ? ibase : 0, mb = mask_self ? iend : 0;
+  auto segment = [&](int a, int b, auto &&f) {
+    if (mask_self)
+      sum_segment_f32<K, true, JB>(posm, a, b, jblock, ma, mb, xi, yi, zi, ii, eps2v, f);
+    else
+      sum_segment_f32<K, false, JB>(posm, a, b, jblock, 0, 0, xi, yi, zi, ii, eps2v, f);
+  };
+  if constexpr (HALVES == 2) {
+    const int blocks = (j1 - j0 + jblock - 1) / jblock;
+    const int jm = min(j1, j0 + (blocks + 1) / 2 * jblock);
+    float *h = red + (S - 1) * 6 * kWave * K + wave * slots * 3 * kWave * K + lane;
+    if (half == 0) {
+      segment(j0, jm, fold);
+    } else {
+      float *o = h;
+      segment(jm, j1, [&](const float (&px)[K], const float (&py)[K], const float (&pz)[K]) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          o[(3 * k) * kWave] = px[k];
+          o[(3 * k + 1) * kWave] = py[k];
+          o[(3 * k + 2) * kWave] = pz[k];
+        }
+        o += 3 * kWave * K;
+      });
+    }
+    __syncthreads();
+    if (half == 0) {
+      for (int b = (blocks + 1) / 2; b < blocks; ++b, h += 3 * kWave * K) {
+        float px[K], py[K], pz[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          px[k] = h[(3 * k) * kWave];
+          py[k] = h[(3 * k + 1) * kWave];
+          pz[k] = h[(3 * k + 2) * kWave];
+        }
+        fold(px, py, pz);
+      }
+    }
+    if constexpr (S == 1) {
+      if (half != 0) return;
+    }
+  } else {
+    segment(j0, j1, fold);
+  }
 
   if constexpr (S > 1) {
     constexpr int L = kWave * K;
-    if (wave > 0) {
+    if (wave > 0 && half == 0) {
       float *r = red + (wave - 1) * 6 * L;
 #pragma unroll
       for (int k = 0; k < K; ++k) {
@@ -293,7 +374,7 @@ __device__ __forceinline__ void stage1_f32_block(const float4 *__restrict__ posm
       }
     }
     __syncthreads();
-    if (wave != 0) return;
+    if (any != 0) return;
     for (int w = 1; w < S; ++w) {
       const float *r = red + (w - 1) * 6 * L;
 #pragma unroll

@@ -346,3 +346,32 @@ def test_perstep_fused_step_is_bitwise_its_two_stages(cuda, sizes, kt, jw):
         _native.call('grav_batched_step_items_f32', b.plan.handle, b.posm.data_ptr(),
                      b.posm.data_ptr(), b.r64.data_ptr(), b.v64.data_ptr(), 1.0, 0.0, 1e-3, jw,
                      torch.cuda.current_stream().cuda_stream)
+
+
+@pytest.mark.parametrize('jw, sizes', [(4, [1100, 2050, 65, 1, 4096, 1024]),
+                                       (1, [300, 1024, 256, 513, 7]), (2, [600, 2048, 1000]),
+                                       (8, [2100, 64, 8192])])
+def test_perstep_in_halves_is_bitwise_a_large_launch(cuda, jw, sizes):
+    # few universes, the longest j-ranges of more than one block of 256: steps and VJP with a
+    # second set of wavefronts; beside 2100 universes of 3 bodies the launches are too large
+    # for it.  The same bits, with eps = 0 and > 0.
+    from gravitation_amd import adjoint
+    print('halves', jw, sizes, flush=True)
+    rng = np.random.default_rng(jw)
+    n = sum(sizes)
+    many = sizes + [3] * 2100
+    off = np.concatenate([[0], np.cumsum(many)])
+    r, v = rng.normal(size=(int(off[-1]), 3)), rng.normal(size=(int(off[-1]), 3))
+    m, w = rng.uniform(0.1, 1.0, int(off[-1])), rng.normal(size=(int(off[-1]), 3))
+    for eps in (0.0, 1e-2):
+        out = []
+        for k in (len(sizes), len(many)):
+            a = int(off[k])
+            eng = batched.Engine(off[:k + 1], ('perstep', 8, 1, 8, 0, jw), cuda)
+            leaves = [torch.from_numpy(x[:a]).to(cuda).requires_grad_(True) for x in (r, v, m)]
+            r1, v1 = adjoint.batched_trajectory(eng, *leaves, 2, G=1.0, eps=eps, dt=1e-3)
+            ((r1 + v1) * torch.from_numpy(w[:a]).to(cuda)).sum().backward()
+            out.append([x[:n].clone() for x in (r1.detach(), v1.detach(),
+                                                *[y.grad for y in leaves])])
+        for x, y in zip(*out):
+            assert torch.equal(x, y), eps
