@@ -44,6 +44,10 @@ SIGNATURES = {
     'grav_stage2_f64m': [_vp, _vp, _vp, _vp, _i64, _d, _vp],
     'grav_stage2_f64': [_vp, _vp, _vp, _i64, _d, _vp],
     'grav_stage2_f32_mirror': [_vp, _vp, _vp, _i64, _d, _vp, _vp],
+    'grav_stage2_f64m_io': [_vp, _vp, _vp, _vp, _vp, _i64, _d, _vp],
+    'grav_state_from_rows': [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp],
+    'grav_state_to_rows': [_vp, _vp, _vp, _vp, _i64, _vp],
+    'grav_cotangent_from_rows': [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp],
     'grav_stage2_f64m_mirror': [_vp, _vp, _vp, _vp, _i64, _d, _vp, _vp],
     'grav_stage2_f64_mirror': [_vp, _vp, _vp, _i64, _d, _vp, _vp],
     'grav_host_mirror_alloc': [_i64, ctypes.POINTER(_vp), ctypes.POINTER(_vp)],

@@ -231,6 +231,59 @@ def _check_state(r0, v0, m):
     return n
 
 
+def _rows(*tensors):
+    """Whether the kernels can read these (n, 3) or (n,) tensors as rows where they lie."""
+    return all(t.is_contiguous() and t.dtype == torch.float64 and not t.is_neg()
+               and t.numel() > 0 for t in tensors)
+
+
+def _load_state(r0, v0, m, posm, r64, v64):
+    """The state's buffers from r0, v0 (n, 3) and m (n,)."""
+    if _rows(r0, v0, m):
+        stages.same_device(r0, v0, m, posm)
+        with stages.on_device(posm):
+            _native.call('grav_state_from_rows', r0.data_ptr(), v0.data_ptr(), m.data_ptr(),
+                         posm.data_ptr(), r64.data_ptr(), v64.data_ptr(), r0.shape[0],
+                         stages.current_stream(posm.device))
+        return
+    r64.copy_(r0.detach().t())
+    v64.copy_(v0.detach().t())
+    posm[:, :3] = r0
+    posm[:, 3] = m
+
+
+def _state_rows(r64, v64):
+    """r64, v64 (3, n) as new (n, 3) tensors."""
+    n = r64.shape[1]
+    if n == 0:
+        return r64.t().contiguous(), v64.t().contiguous()
+    r, v = (torch.empty((n, 3), dtype=torch.float64, device=r64.device) for _ in range(2))
+    with stages.on_device(r64):
+        _native.call('grav_state_to_rows', r64.data_ptr(), v64.data_ptr(), r.data_ptr(),
+                     v.data_ptr(), n, stages.current_stream(r64.device))
+    return r, v
+
+
+def _load_cotangents(g_r, g_v, rho, nu, gamma, eslot=None):
+    """rho, nu (3, n) from the cotangents (n, 3) or None, with gamma and eslot cleared."""
+    if gamma.numel() and _rows(*[g for g in (g_r, g_v) if g is not None]):
+        with stages.on_device(rho):
+            _native.call('grav_cotangent_from_rows', None if g_r is None else g_r.data_ptr(),
+                         None if g_v is None else g_v.data_ptr(), rho.data_ptr(),
+                         nu.data_ptr(), gamma.data_ptr(),
+                         None if eslot is None else eslot.data_ptr(), gamma.shape[0],
+                         stages.current_stream(rho.device))
+        return
+    for g, x in ((g_r, rho), (g_v, nu)):
+        if g is not None:
+            x.copy_(g.t())
+        else:
+            x.zero_()
+    gamma.zero_()
+    if eslot is not None:
+        eslot.zero_()
+
+
 def _stage1_form(n, form):
     return stages.auto_form(n) if form == 'auto' else form
 
@@ -248,15 +301,16 @@ def _stage1(posm, acc, G, eps, form='auto', ws=None):
         stages.stage1_f32(posm, acc, G, eps, 'kahan')
 
 
-def _step(posm, acc, r64, v64, G, eps, dt, form='auto', ws=None):
+def _step(posm, acc, r64, v64, G, eps, dt, form='auto', ws=None, out=None):
     """One time step: stage 1 in the form for n, then the FP64-master stage 2; the j-split
     form as one fused step (``stages.step_split_f64m``, the same bits).  Every forward and
-    recomputed step goes through here, so they agree bit for bit."""
+    recomputed step goes through here, so they agree bit for bit.  ``out``: the buffer of the
+    new positions (default: posm)."""
     if _stage1_form(posm.shape[0], form) == 'split':
-        stages.step_split_f64m(posm, r64, v64, G, eps, dt, None, ws)
+        stages.step_split_f64m(posm, r64, v64, G, eps, dt, None, ws, out=out)
     else:
         _stage1(posm, acc, G, eps, form, ws)
-        stages.stage2_f64m(posm, r64, v64, acc, dt)
+        stages.stage2_f64m(posm, r64, v64, acc, dt, out=out)
 
 
 def _vjp_split(n, form):
@@ -309,7 +363,7 @@ class _SegmentGraphs:
         self.nu = torch.empty((3, n), dtype=f64, device=dev)
         self.gamma = torch.empty((n,), dtype=f64, device=dev)
         self.mu4 = torch.empty((n, 4), dtype=f32, device=dev)
-        self.eslot = torch.zeros((2,), dtype=torch.int32, device=dev)
+        self.eslot = torch.empty((2,), dtype=torch.int32, device=dev)
         s1 = _stage1_form(n, form)
         need = (stages.sym_workspace_size(n, device=dev) if s1 == 'symmetric'
                 else stages.split_workspace_bytes(n) if s1 == 'split' else 0)
@@ -374,12 +428,13 @@ class _SegmentGraphs:
             self.step()
             traj[t + 1].copy_(self.posm)
 
-    def begin_backward(self):
-        """The first backward step's cotangent (and a cleared exponent slot for the chain);
-        with the chain every later one comes from the previous step's reduce."""
+    def begin_backward(self, g_r, g_v):
+        """The adjoint state from the trajectory's cotangents, with a cleared exponent slot, and
+        with the chain the first backward step's cotangent; every later one comes from the
+        previous step's reduce."""
+        _load_cotangents(g_r, g_v, self.rho, self.nu, self.gamma, self.eslot)
         if self.chain:
             adjoint_mu(self.rho, self.nu, self.mu4, self.cfg[2], self.ws_adj)
-            self.eslot.zero_()
 
     def adjoint(self, k, last, traj):
         """Backward steps k-1 .. 0 over the record ``traj``; ``last``: the segment holds step
@@ -494,31 +549,20 @@ class _Single(torch.autograd.Function):
               if graph and not store else None)
         if sg is not None:
             posm, acc, r64, v64 = sg.posm, sg.acc, sg.r64, sg.v64
-            r64.copy_(r0.detach().t())
-            v64.copy_(v0.detach().t())
         else:
             posm = torch.empty((n, 4), dtype=torch.float32, device=dev)
             acc = torch.empty((3, n), dtype=torch.float32, device=dev)
-            r64 = r0.detach().t().contiguous()
-            v64 = v0.detach().t().contiguous()
-        posm[:, :3] = r0
-        posm[:, 3] = m
+            r64 = torch.empty((3, n), dtype=torch.float64, device=dev)
+            v64 = torch.empty((3, n), dtype=torch.float64, device=dev)
         traj = torch.empty((steps, n, 4), dtype=torch.float32, device=dev) if store else None
+        # a recorded step goes from one slot of the record to the next, the last one into posm
+        slots = [traj[t] for t in range(steps)] + [posm] if store else [posm]
+        _load_state(r0, v0, m, slots[0], r64, v64)
         checkpoints = []
-        t = 0
-        if store and steps > 0 and _stage1_form(n, form) == 'split':
-            # a step goes from one slot of the record to the next, the last one back into posm
-            traj[0].copy_(posm)
-            for t in range(steps):
-                stages.step_split_f64m(traj[t], r64, v64, G, eps, dt,
-                                       out=traj[t + 1] if t + 1 < steps else posm)
-            t = steps
+        for p, q in zip(slots, slots[1:]):
+            _step(p, acc, r64, v64, G, eps, dt, form, out=q)
+        t = steps if store else 0
         while t < steps:
-            if store:
-                traj[t].copy_(posm)
-                _step(posm, acc, r64, v64, G, eps, dt, form)
-                t += 1
-                continue
             checkpoints.append((r64.clone(), v64.clone()))
             k = min(interval, steps - t)
             if sg is not None and sg.paired and t + k == steps:
@@ -534,8 +578,8 @@ class _Single(torch.autograd.Function):
         ctx.cfg = (G, eps, dt, steps, interval, store, form, graph)
         ctx.traj = traj
         ctx.checkpoints = checkpoints
-        ctx.mass = posm[:, 3].clone()
-        return r64.t().contiguous(), v64.t().contiguous()
+        ctx.mass = posm[:, 3] if store else posm[:, 3].clone()
+        return _state_rows(r64, v64)
 
     @staticmethod
     def backward(ctx, g_r, g_v):
@@ -548,16 +592,7 @@ class _Single(torch.autograd.Function):
             sg = _SegmentGraphs(n, dev, G, eps, dt, interval, form, 2 if OVERLAP else 1)
         else:
             sg = _segment_graphs(n, dev, G, eps, dt, interval, form)
-        if g_r is not None:
-            sg.rho.copy_(g_r.t())
-        else:
-            sg.rho.zero_()
-        if g_v is not None:
-            sg.nu.copy_(g_v.t())
-        else:
-            sg.nu.zero_()
-        sg.gamma.zero_()
-        sg.begin_backward()
+        sg.begin_backward(g_r, g_v)
         if store:
             sg.adjoint(steps, True, ctx.traj)
         else:
@@ -565,8 +600,10 @@ class _Single(torch.autograd.Function):
                                recorded=sg.recorded is getattr(ctx, 'rec_token', 0))
         ctx.traj = None
         ctx.checkpoints = None
-        return (sg.rho.t().clone(), sg.nu.t().clone(), sg.gamma.clone(), None, None, None, None,
-                None, None, None, None)
+        grads = sg.rho.t(), sg.nu.t(), sg.gamma
+        if graph and not store:   # sg outlives this pass
+            grads = [g.clone() for g in grads]
+        return (*grads, None, None, None, None, None, None, None, None)
 
 
 def trajectory(r0, v0, m, steps, G=1.0, eps=0.0, dt=1e-3, interval=None, budget=None,
@@ -600,10 +637,9 @@ class _Batched(torch.autograd.Function):
         n = r0.shape[0]
         dev = r0.device
         posm = torch.empty((n, 4), dtype=torch.float32, device=dev)
-        posm[:, :3] = r0
-        posm[:, 3] = m
-        r64 = r0.detach().t().contiguous()
-        v64 = v0.detach().t().contiguous()
+        r64 = torch.empty((3, n), dtype=torch.float64, device=dev)
+        v64 = torch.empty((3, n), dtype=torch.float64, device=dev)
+        _load_state(r0, v0, m, posm, r64, v64)
         traj = None
         checkpoints = []
         if store:
@@ -616,19 +652,18 @@ class _Batched(torch.autograd.Function):
         ctx.cfg = (engine, G, eps, dt, steps, interval, store)
         ctx.traj = traj
         ctx.checkpoints = checkpoints
-        ctx.mass = posm[:, 3].clone()
-        return r64.t().contiguous(), v64.t().contiguous()
+        ctx.mass = posm[:, 3] if store else posm[:, 3].clone()
+        return _state_rows(r64, v64)
 
     @staticmethod
     def backward(ctx, g_r, g_v):
         engine, G, eps, dt, steps, interval, store = ctx.cfg
         n = ctx.mass.shape[0]
         dev = ctx.mass.device
-        rho = (g_r.t().contiguous().double() if g_r is not None
-               else torch.zeros((3, n), dtype=torch.float64, device=dev))
-        nu = (g_v.t().contiguous().double() if g_v is not None
-              else torch.zeros((3, n), dtype=torch.float64, device=dev))
-        gamma = torch.zeros((n,), dtype=torch.float64, device=dev)
+        rho = torch.empty((3, n), dtype=torch.float64, device=dev)
+        nu = torch.empty((3, n), dtype=torch.float64, device=dev)
+        gamma = torch.empty((n,), dtype=torch.float64, device=dev)
+        _load_cotangents(g_r, g_v, rho, nu, gamma)
         if store:
             engine.adjoint(ctx.traj, rho, nu, gamma, G, eps, dt, steps)
         else:

@@ -45,8 +45,11 @@ __global__ __launch_bounds__(kBlock) void k_stage2_f32(float4 *__restrict__ posm
 }
 
 // FP64 masters advanced with FP32 accelerations; the FP32 stage-1 copy gets x, y, z only
-// (a 12-byte store, so m is neither read nor written).
-__global__ __launch_bounds__(kBlock) void k_stage2_f64m(float *__restrict__ posm,
+// (a 12-byte store, so m is neither read nor written), and m from `from` when that is not NULL
+// (the positions go to a buffer of their own: a recorded step without a copy of the record's
+// slot, 4.3 us of a step of 20000 bodies).
+__global__ __launch_bounds__(kBlock) void k_stage2_f64m(const float4 *__restrict__ from,
+                                                        float *__restrict__ posm,
                                                         double *__restrict__ r64,
                                                         double *__restrict__ v64,
                                                         const float *__restrict__ acc, int n,
@@ -70,6 +73,7 @@ __global__ __launch_bounds__(kBlock) void k_stage2_f64m(float *__restrict__ posm
   p[0] = static_cast<float>(r[0]);
   p[1] = static_cast<float>(r[1]);
   p[2] = static_cast<float>(r[2]);
+  if (from != nullptr) p[3] = from[i].w;
   if (mirror != nullptr) {   // [r64 (3, n) | v64 (3, n)]
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
@@ -99,6 +103,49 @@ __global__ __launch_bounds__(kBlock) void k_stage2_f64(double *__restrict__ posm
     }
   }
   if (mirror != nullptr) mirror[4 * static_cast<size_t>(i) + 3] = p[3];
+}
+
+// Body i's rows r[i], v[i] (NULL: zeros) into the columns of r64, v64 (3, n); with posm also
+// its FP32 position and mass, with zero its element of a cleared vector and with slot two
+// cleared words.  Bound by launches: a universe's state was four torch kernels and an adjoint's
+// start four, 4 to 5 us each at 20000 bodies, where the bytes (88 per body) take 0.4 us.  A
+// thread per body: the rows' 24-byte strides cost less than a pass through LDS would.
+__global__ __launch_bounds__(kBlock) void k_columns_of_rows(
+    const double *__restrict__ r, const double *__restrict__ v, const double *__restrict__ m,
+    float4 *__restrict__ posm, double *__restrict__ r64, double *__restrict__ v64,
+    double *__restrict__ zero, unsigned *__restrict__ slot, int n) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (slot != nullptr && i < 2) slot[i] = 0u;
+  if (i >= n) return;
+  double x[3], u[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    x[c] = r != nullptr ? r[3 * static_cast<size_t>(i) + c] : 0.0;
+    u[c] = v != nullptr ? v[3 * static_cast<size_t>(i) + c] : 0.0;
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    r64[c * static_cast<size_t>(n) + i] = x[c];
+    v64[c * static_cast<size_t>(n) + i] = u[c];
+  }
+  if (posm != nullptr)
+    posm[i] = make_float4(static_cast<float>(x[0]), static_cast<float>(x[1]),
+                          static_cast<float>(x[2]), static_cast<float>(m[i]));
+  if (zero != nullptr) zero[i] = 0.0;
+}
+
+// The columns of r64, v64 (3, n) back into rows r, v (n, 3).
+__global__ __launch_bounds__(kBlock) void k_rows_of_columns(const double *__restrict__ r64,
+                                                            const double *__restrict__ v64,
+                                                            double *__restrict__ r,
+                                                            double *__restrict__ v, int n) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    r[3 * static_cast<size_t>(i) + c] = r64[c * static_cast<size_t>(n) + i];
+    v[3 * static_cast<size_t>(i) + c] = v64[c * static_cast<size_t>(n) + i];
+  }
 }
 
 int validate(const char *fn, const void *a, const void *b, const void *c, int64_t n, double dt) {
@@ -131,8 +178,8 @@ int stage2_f32(const char *fn, void *posm, void *vel, const void *acc, int64_t n
   return check_launch("k_stage2_f32");
 }
 
-int stage2_f64m(const char *fn, void *posm, void *r64, void *v64, const void *acc, int64_t n,
-                double dt, void *mirror, void *stream) {
+int stage2_f64m(const char *fn, const void *from, void *posm, void *r64, void *v64,
+                const void *acc, int64_t n, double dt, void *mirror, void *stream) {
   int rc = validate(fn, posm, r64, v64, n, dt);
   if (rc != GRAV_OK) return rc;
   GRAV_REQUIRE(acc != nullptr, "%s: acc is NULL", fn);
@@ -141,9 +188,10 @@ int stage2_f64m(const char *fn, void *posm, void *r64, void *v64, const void *ac
                "%s: r64/v64/acc misaligned", fn);
   const int nn = static_cast<int>(n);
   hipLaunchKernelGGL(k_stage2_f64m, dim3((nn + kBlock - 1) / kBlock), dim3(kBlock), 0,
-                     static_cast<hipStream_t>(stream), static_cast<float *>(posm),
-                     static_cast<double *>(r64), static_cast<double *>(v64),
-                     static_cast<const float *>(acc), nn, dt, static_cast<double *>(mirror));
+                     static_cast<hipStream_t>(stream), static_cast<const float4 *>(from),
+                     static_cast<float *>(posm), static_cast<double *>(r64),
+                     static_cast<double *>(v64), static_cast<const float *>(acc), nn, dt,
+                     static_cast<double *>(mirror));
   return check_launch("k_stage2_f64m");
 }
 
@@ -178,7 +226,77 @@ int grav_stage2_f32(void *posm, void *vel, const void *acc, int64_t n, double dt
 int grav_stage2_f64m(void *posm, void *r64, void *v64, const void *acc, int64_t n, double dt,
                      void *stream) {
   clear_error();
-  return stage2_f64m("grav_stage2_f64m", posm, r64, v64, acc, n, dt, nullptr, stream);
+  return stage2_f64m("grav_stage2_f64m", nullptr, posm, r64, v64, acc, n, dt, nullptr, stream);
+}
+
+int grav_stage2_f64m_io(const void *posm_in, void *posm_out, void *r64, void *v64,
+                        const void *acc, int64_t n, double dt, void *stream) {
+  clear_error();
+  const char *fn = "grav_stage2_f64m_io";
+  GRAV_REQUIRE(posm_in != nullptr && aligned(posm_in, 16),
+               "%s: posm_in must be a 16-byte aligned buffer", fn);
+  GRAV_REQUIRE(n >= 1 && n <= kMaxBodies, "%s: n must be in [1, 2^29] (got %lld)", fn,
+               (long long)n);
+  const char *a = static_cast<const char *>(posm_in);
+  const char *b = static_cast<const char *>(posm_out);
+  GRAV_REQUIRE(a + 16 * n <= b || b + 16 * n <= a, "%s: posm_out overlaps posm_in", fn);
+  return stage2_f64m(fn, posm_in, posm_out, r64, v64, acc, n, dt, nullptr, stream);
+}
+
+int grav_state_from_rows(const void *r, const void *v, const void *m, void *posm, void *r64,
+                         void *v64, int64_t n, void *stream) {
+  clear_error();
+  const char *fn = "grav_state_from_rows";
+  const int rc = validate(fn, r, v, m, n, 0.0);
+  if (rc != GRAV_OK) return rc;
+  GRAV_REQUIRE(posm != nullptr && r64 != nullptr && v64 != nullptr, "%s: NULL buffer", fn);
+  GRAV_REQUIRE(aligned(r, 8) && aligned(v, 8) && aligned(m, 8) && aligned(posm, 16) &&
+                   aligned(r64, 8) && aligned(v64, 8),
+               "%s: misaligned buffer", fn);
+  const int nn = static_cast<int>(n);
+  hipLaunchKernelGGL(k_columns_of_rows, dim3((nn + kBlock - 1) / kBlock), dim3(kBlock), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const double *>(r),
+                     static_cast<const double *>(v), static_cast<const double *>(m),
+                     static_cast<float4 *>(posm), static_cast<double *>(r64),
+                     static_cast<double *>(v64), static_cast<double *>(nullptr),
+                     static_cast<unsigned *>(nullptr), nn);
+  return check_launch("k_columns_of_rows");
+}
+
+int grav_cotangent_from_rows(const void *g_r, const void *g_v, void *rho64, void *nu64,
+                             void *gamma64, void *eslot, int64_t n, void *stream) {
+  clear_error();
+  const char *fn = "grav_cotangent_from_rows";
+  const int rc = validate(fn, rho64, nu64, gamma64, n, 0.0);
+  if (rc != GRAV_OK) return rc;
+  GRAV_REQUIRE(aligned(g_r, 8) && aligned(g_v, 8) && aligned(rho64, 8) && aligned(nu64, 8) &&
+                   aligned(gamma64, 8) && aligned(eslot, 4),
+               "%s: misaligned buffer", fn);
+  const int nn = static_cast<int>(n);
+  hipLaunchKernelGGL(k_columns_of_rows, dim3((nn + kBlock - 1) / kBlock), dim3(kBlock), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const double *>(g_r),
+                     static_cast<const double *>(g_v), static_cast<const double *>(nullptr),
+                     static_cast<float4 *>(nullptr), static_cast<double *>(rho64),
+                     static_cast<double *>(nu64), static_cast<double *>(gamma64),
+                     static_cast<unsigned *>(eslot), nn);
+  return check_launch("k_columns_of_rows");
+}
+
+int grav_state_to_rows(const void *r64, const void *v64, void *r, void *v, int64_t n,
+                       void *stream) {
+  clear_error();
+  const char *fn = "grav_state_to_rows";
+  const int rc = validate(fn, r64, v64, r, n, 0.0);
+  if (rc != GRAV_OK) return rc;
+  GRAV_REQUIRE(v != nullptr, "%s: NULL buffer", fn);
+  GRAV_REQUIRE(aligned(r64, 8) && aligned(v64, 8) && aligned(r, 8) && aligned(v, 8),
+               "%s: misaligned buffer", fn);
+  const int nn = static_cast<int>(n);
+  hipLaunchKernelGGL(k_rows_of_columns, dim3((nn + kBlock - 1) / kBlock), dim3(kBlock), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const double *>(r64),
+                     static_cast<const double *>(v64), static_cast<double *>(r),
+                     static_cast<double *>(v), nn);
+  return check_launch("k_rows_of_columns");
 }
 
 int grav_stage2_f64(void *posm64, void *v64, const void *acc64, int64_t n, double dt,
@@ -200,7 +318,8 @@ int grav_stage2_f64m_mirror(void *posm, void *r64, void *v64, const void *acc, i
   clear_error();
   const int rc = mirror_ok("grav_stage2_f64m_mirror", mirror, 8);
   if (rc != GRAV_OK) return rc;
-  return stage2_f64m("grav_stage2_f64m_mirror", posm, r64, v64, acc, n, dt, mirror, stream);
+  return stage2_f64m("grav_stage2_f64m_mirror", nullptr, posm, r64, v64, acc, n, dt, mirror,
+                     stream);
 }
 
 int grav_stage2_f64_mirror(void *posm64, void *v64, const void *acc64, int64_t n, double dt,

@@ -462,16 +462,25 @@ def stage2_f32(posm, vel, acc, dt):
                      float(dt), _stream(posm))
 
 
-def stage2_f64m(posm, r64, v64, acc, dt):
+def stage2_f64m(posm, r64, v64, acc, dt, out=None):
+    """The FP64-master stage 2, in place, or (``out``) with the new positions and posm's masses
+    in a position buffer of their own."""
     n = posm.shape[0]
     _check(posm, 'posm', torch.float32, (n, 4))
     _check(r64, 'r64', torch.float64, (3, n))
     _check(v64, 'v64', torch.float64, (3, n))
     _check(acc, 'acc', torch.float32, (3, n))
     same_device(posm, r64, v64, acc)
+    if out is not None:
+        _check(out, 'out', torch.float32, (n, 4))
+        same_device(posm, out)
     with on_device(posm):
-        _native.call('grav_stage2_f64m', posm.data_ptr(), r64.data_ptr(), v64.data_ptr(),
-                     acc.data_ptr(), n, float(dt), _stream(posm))
+        if out is not None:
+            _native.call('grav_stage2_f64m_io', posm.data_ptr(), out.data_ptr(), r64.data_ptr(),
+                         v64.data_ptr(), acc.data_ptr(), n, float(dt), _stream(posm))
+        else:
+            _native.call('grav_stage2_f64m', posm.data_ptr(), r64.data_ptr(), v64.data_ptr(),
+                         acc.data_ptr(), n, float(dt), _stream(posm))
 
 
 def stage2_f64(posm64, v64, acc64, dt):

@@ -163,6 +163,24 @@ int grav_stage2_f32(void *posm, void *vel, const void *acc, int64_t n, double dt
 int grav_stage2_f64m(void *posm, void *r64, void *v64, const void *acc, int64_t n,
                      double dt, void *stream);
 
+/* grav_stage2_f64m from one position buffer to another: reads the masses of posm_in and writes
+ * posm_out float4[n], which must not overlap it. */
+int grav_stage2_f64m_io(const void *posm_in, void *posm_out, void *r64, void *v64,
+                        const void *acc, int64_t n, double dt, void *stream);
+
+/* A universe's state from rows: r, v double[n][3] and m double[n] to posm float4[n] (rounded)
+ * and r64, v64 double[3][n]; and the state's r64, v64 back to rows. */
+int grav_state_from_rows(const void *r, const void *v, const void *m, void *posm, void *r64,
+                         void *v64, int64_t n, void *stream);
+int grav_state_to_rows(const void *r64, const void *v64, void *r, void *v, int64_t n,
+                       void *stream);
+
+/* The start of an adjoint pass: cotangent rows g_r, g_v double[n][3] (NULL: zeros) to rho64,
+ * nu64 double[3][n], with gamma64 double[n] and, when not NULL, the two words of eslot
+ * (grav_stage1_vjp_f32_split_chain) cleared. */
+int grav_cotangent_from_rows(const void *g_r, const void *g_v, void *rho64, void *nu64,
+                             void *gamma64, void *eslot, int64_t n, void *stream);
+
 /* Stage 2, all-FP64: posm64.xyz and v64 advanced with acc64. */
 int grav_stage2_f64(void *posm64, void *v64, const void *acc64, int64_t n, double dt,
                     void *stream);

@@ -753,3 +753,54 @@ def test_vjp_shard_rows_equal_whole_universe(cuda, n, eps):
     adjoint.stage1_vjp_shard_f32(posm, mu4, rs, gs, 0, 0.9, eps, 1e-3)
     assert torch.isfinite(rs).all() and not torch.equal(rs, rho0[:, :n // 2])
     stages.release_workspaces()
+
+
+@pytest.mark.parametrize('n', [1, 63, 256, 257, 1300])
+def test_contiguous_rows_equal_the_general_path(cuda, n):
+    # contiguous float64 rows go through one kernel each way, any other layout through torch:
+    # the same trajectories and gradients, bit for bit, recorded and checkpointed, for one
+    # universe and a batch, with one cotangent missing too; and a stage 2 into another buffer
+    # is the one in place
+    from gravitation_amd import batched, stages
+    print('rows', n, flush=True)
+    rng = np.random.default_rng(n)
+    r, v, w = (torch.from_numpy(rng.normal(size=(n, 3))).to(cuda) for _ in range(3))
+    m = torch.from_numpy(rng.uniform(0.1, 1.0, n)).to(cuda)
+    eng = batched.Engine(np.array([0, n // 2, n] if n > 1 else [0, n]))
+
+    def strided(x):
+        y = torch.empty((*x.shape, 2), dtype=x.dtype, device=cuda)[..., 1]
+        y.copy_(x)
+        return y
+
+    def negated(x):
+        y = torch._neg_view(-x)
+        assert y.is_neg() and y.is_contiguous()
+        return y
+
+    kw = dict(G=1.0, eps=1e-2, dt=1e-3)
+    runs = [lambda *x: adjoint.trajectory(*x, 4, **kw),
+            lambda *x: adjoint.trajectory(*x, 4, interval=2, **kw),
+            lambda *x: adjoint.batched_trajectory(eng, *x, 4, **kw)]
+    for run in runs:
+        for both in (True, False):
+            got = []
+            for of in (lambda x: x.clone(), strided, negated):
+                leaves = [of(x).requires_grad_(True) for x in (r, v, m)]
+                out = run(*leaves)
+                cots = [of(w), of(w + 1.0)]
+                k = 2 if both else 1
+                got.append([x.detach() for x in out] +
+                           list(torch.autograd.grad(out[:k], leaves, cots[:k])))
+            for other in got[1:]:
+                for x, y in zip(got[0], other):
+                    assert torch.equal(x, y)
+    p = torch.empty((n, 4), dtype=torch.float32, device=cuda)
+    p[:, :3], p[:, 3] = r, m
+    acc = torch.randn((3, n), device=cuda)
+    q = torch.full_like(p, 7.0)
+    a, b = ([r.t().contiguous().clone(), v.t().contiguous().clone()] for _ in range(2))
+    stages.stage2_f64m(p, *a, acc, 1e-2, out=q)
+    stages.stage2_f64m(p, *b, acc, 1e-2)
+    for x, y in zip((q, *a), (p, *b)):
+        assert torch.equal(x, y)
