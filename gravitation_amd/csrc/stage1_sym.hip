@@ -73,8 +73,9 @@ __device__ __forceinline__ float4 load_or_far(const float4 *__restrict__ posm, i
 // takes 11.19 ms.  Measured and not kept: the j-bodies read from LDS instead of rotated (3 DPP
 // moves per step instead of 7) is no faster once the moves have priority (2.95 against 2.86 ms
 // at 2^17), and temporaries pinned to registers of alternating parity (an FMA whose three
-// operands have register numbers of one parity issues alone) gain 1 %.
-template <int K, bool OWN>
+// operands have register numbers of one parity issues alone) gain 1 %.  Without PRIO no priority
+// is raised, for launches that leave a SIMD to one wavefront (sym_prio).
+template <int K, bool OWN, bool PRIO = true>
 __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const float eps2,
                                           const float (&xi)[K], const float (&yi)[K],
                                           const float (&zi)[K], const float (&mn)[K],
@@ -99,10 +100,10 @@ __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const
         r2 = __builtin_fmaf(dy[g], dy[g], r2);
         inv[g] = __builtin_fmaf(dz[g], dz[g], r2);
       }
-      prio_up();
+      if constexpr (PRIO) prio_up();
 #pragma unroll
       for (int g = 0; g < G; ++g) inv[g] = __builtin_amdgcn_rsqf(inv[g]);
-      prio_down();
+      if constexpr (PRIO) prio_down();
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         if (OWN && t == 0 && k + g == kself) inv[g] = 0.0f;
@@ -119,7 +120,7 @@ __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const
         }
       }
     }
-    prio_up();
+    if constexpr (PRIO) prio_up();
     if constexpr (!OWN) {
       // the sums so far come from the lane that held this j-body in the step before
       ajx = rot1(ajx) + tx;
@@ -130,7 +131,7 @@ __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const
     yj = rot1(yj);
     zj = rot1(zj);
     mj = rot1(mj);
-    prio_down();
+    if constexpr (PRIO) prio_down();
   }
   if constexpr (!OWN) {   // home
     ajx = rot1(ajx);
@@ -145,7 +146,7 @@ __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const
 // pairs (hx, lx) .. (hz, lz), which the caller may carry over several gamma blocks; the j-side
 // sums of a chunk, added over the W wavefronts through the double-buffered LDS `red` (buffer
 // chunk & 1, chunk counting on across calls), go to pj[c * IB + jc * 64 + l], 3 * IB floats.
-template <int K, int W>
+template <int K, int W, bool PRIO>
 __device__ __forceinline__ void sym_block_pair(const float4 *__restrict__ posm, int jb0,
                                                int jend, float eps2, const float (&xi)[K],
                                                const float (&yi)[K], const float (&zi)[K],
@@ -162,7 +163,7 @@ __device__ __forceinline__ void sym_block_pair(const float4 *__restrict__ posm, 
     float px[K], py[K], pz[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) px[k] = py[k] = pz[k] = 0.0f;
-    sym_chunk<K, false>(q, -1, eps2, xi, yi, zi, mn, px, py, pz, ajx, ajy, ajz);
+    sym_chunk<K, false, PRIO>(q, -1, eps2, xi, yi, zi, mn, px, py, pz, ajx, ajy, ajz);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       two_sum_sym(hx[k], lx[k], px[k]);
@@ -190,7 +191,7 @@ __device__ __forceinline__ void sym_block_pair(const float4 *__restrict__ posm, 
 // block gamma, end of block beta, end of block gamma} of one universe.  Block beta is never
 // its universe's last block, so only block gamma can be short.  Writes the i-side partial to
 // p_i and the j-side partial to p_j at item * 3 * IB.
-template <int K, int W>
+template <int K, int W, bool PRIO>
 __global__ __launch_bounds__(kWave *W) void k_sym_pairs(const float4 *__restrict__ posm,
                                                          float eps2, float *__restrict__ p_i,
                                                          float *__restrict__ p_j,
@@ -216,7 +217,7 @@ __global__ __launch_bounds__(kWave *W) void k_sym_pairs(const float4 *__restrict
   }
   int chunk = 0;
   const float eps2v = in_vgpr(eps2);
-  sym_block_pair<K, W>(posm, it.y, it.w, eps2v, xi, yi, zi, mn, hx, hy, hz, lx, ly, lz,
+  sym_block_pair<K, W, PRIO>(posm, it.y, it.w, eps2v, xi, yi, zi, mn, hx, hy, hz, lx, ly, lz,
                        p_j + base, red, chunk, lane, wave);
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -282,7 +283,7 @@ __device__ __forceinline__ void span_segment(const SegSpan &sp, int b, int nb, i
 
 // blockIdx.x: the blockIdx.x-th segment of the span; its partials go to p_i / p_j at the
 // slab-local index blockIdx.x.
-template <int K, int W>
+template <int K, int W, bool PRIO>
 __global__ __launch_bounds__(kWave *W) void k_sym_segments(const float4 *__restrict__ posm,
                                                             int n, int nb, int lg,
                                                             SegSpan span, float eps2,
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(kWave *W) void k_sym_segments(const float4 *__restr
   const float eps2v = in_vgpr(eps2);
   for (int gamma = g0; gamma < g1; ++gamma) {
     float *pj = p_j + ((local << lg) + (gamma - g0)) * (3 * IB);
-    sym_block_pair<K, W>(posm, gamma * IB, n, eps2v, xi, yi, zi, mn, hx, hy, hz, lx, ly, lz,
+    sym_block_pair<K, W, PRIO>(posm, gamma * IB, n, eps2v, xi, yi, zi, mn, hx, hy, hz, lx, ly, lz,
                          pj, red, chunk, lane, wave);
   }
   const size_t base = local * 3 * IB;
@@ -1084,11 +1085,24 @@ bool sym_units_shape(int64_t n, int K, int W) {
   return K == K0 && W == W0 && n >= kUnitsFrom && n < kUnitsTo;
 }
 
+// Whether a launch of workgroups of W wavefronts raises the priority of its rsq and DPP moves:
+// where it does not give some SIMD two wavefronts, s_setprio only keeps the compiler from
+// mixing one pair's instructions into the next one's.  MI355X, one universe, without and with:
+// (4, 2) 8192 bodies (120 workgroups) 106 and 113 us, 12288 (276) 159 and 121; (4, 4) 18000 (153)
+// 204 and 220, 24576 (276) 312 and 232; (8, 2) 16384 (120) 327 and 349, 24576 (276) 542 and 403.
+// Batched, W = 1: (8, 1) 420 block pairs 185 and 201, 945 346 and 275, (4, 1) 980 95 and 77; (4, 2)
+// 205 120 and 134, 420 173 and 142.
+bool sym_prio(int64_t workgroups, int W) { return workgroups > kCus * (W == 1 ? 2 : 1); }
+
 template <int K, int W>
 int launch_segments(const float4 *posm, int n, const SymPlan &P, const SegSpan &sp, int nseg,
                     float eps2, float *pi, float *pj, hipStream_t s) {
-  hipLaunchKernelGGL((k_sym_segments<K, W>), dim3(static_cast<unsigned>(nseg)),
-                     dim3(kWave * W), 0, s, posm, n, P.nb, P.lg, sp, eps2, pi, pj);
+  if (sym_prio(nseg, W))
+    hipLaunchKernelGGL((k_sym_segments<K, W, true>), dim3(static_cast<unsigned>(nseg)),
+                       dim3(kWave * W), 0, s, posm, n, P.nb, P.lg, sp, eps2, pi, pj);
+  else
+    hipLaunchKernelGGL((k_sym_segments<K, W, false>), dim3(static_cast<unsigned>(nseg)),
+                       dim3(kWave * W), 0, s, posm, n, P.nb, P.lg, sp, eps2, pi, pj);
   return check_launch("k_sym_segments");
 }
 
@@ -1124,8 +1138,12 @@ template <int K, int W>
 int launch_pairs_items(const float4 *posm, float eps2, float *pi, float *pj, const int4 *items,
                        int nitems, hipStream_t s) {
   if (nitems == 0) return GRAV_OK;
-  hipLaunchKernelGGL((k_sym_pairs<K, W>), dim3(static_cast<unsigned>(nitems)), dim3(kWave * W),
-                     0, s, posm, eps2, pi, pj, items);
+  if (sym_prio(nitems, W))
+    hipLaunchKernelGGL((k_sym_pairs<K, W, true>), dim3(static_cast<unsigned>(nitems)),
+                       dim3(kWave * W), 0, s, posm, eps2, pi, pj, items);
+  else
+    hipLaunchKernelGGL((k_sym_pairs<K, W, false>), dim3(static_cast<unsigned>(nitems)),
+                       dim3(kWave * W), 0, s, posm, eps2, pi, pj, items);
   return check_launch("k_sym_pairs");
 }
 

@@ -375,3 +375,22 @@ def test_perstep_in_halves_is_bitwise_a_large_launch(cuda, jw, sizes):
                                                 *[y.grad for y in leaves])])
         for x, y in zip(*out):
             assert torch.equal(x, y), eps
+
+
+@pytest.mark.parametrize('sym', [(4, 1), (8, 1), (4, 2), (8, 2), (4, 4)])
+def test_sym_pairs_of_small_and_large_launches_are_bitwise_equal(cuda, sym):
+    # the block pairs of one universe alone leave SIMDs with one wavefront, those of 300 copies
+    # do not: the pair loops without and with the raised priority, the same sums
+    print('sym launches', sym, flush=True)
+    s = 1100
+    rng = np.random.default_rng(7)
+    one = np.concatenate([rng.normal(size=(s, 3)), rng.uniform(0.1, 1.0, (s, 1))], axis=1)
+    got = []
+    for copies in (1, 300):
+        eng = batched.Engine(np.arange(copies + 1) * s, ('perstep-sym', 8, 1, 8, 0, 4, sym), cuda)
+        posm = torch.from_numpy(np.tile(one, (copies, 1)).astype(np.float32)).to(cuda)
+        got.append(_sym_acc(eng, posm, 0.7, 1e-2))
+    few, many = got
+    assert torch.isfinite(few).all()
+    for k in (0, 150, 299):
+        assert torch.equal(many[:, k * s:(k + 1) * s], few)
