@@ -67,8 +67,8 @@ __device__ __forceinline__ float4 load_or_far(const float4 *__restrict__ posm, i
 // raised priority (prio_up), eps2 sits in a VGPR and the masses come negated, so that the j side
 // needs no negating (8-byte) FMA.  Adding the step's j-side sum in the move itself leaves the time
 // as it was (2^18 11.36 against 11.43 ms on one box) and about halves the error against 64 bits
-// (Plummer, eps 1e-3: 20000 bodies 1.5e-7 to 7e-8, 65536 9.3e-8 to 5.7e-8).  MI355X, (8, 2), before and after: 2^18 bodies 13.40 and
-// 11.13 ms (65.7 to 54 cycles per pair of bodies and wavefront), 2^17 3.44 and 2.87 ms; (4, 2) at
+// (Plummer, eps 1e-3: 20000 bodies 1.5e-7 to 7e-8, 65536 9.3e-8 to 5.7e-8).  MI355X, (8, 2),
+// before and after: 2^18 bodies 13.40 and 11.13 ms (59 to 49 cycles per pair and SIMD), 2^17 3.44 and 2.87 ms; (4, 2) at
 // 49999 bodies 0.652 and 0.496 ms.  G = 4 pairs need 138 VGPRs with K = 8 for 11.05 ms, G = 1
 // takes 11.19 ms.  Measured and not kept: the j-bodies read from LDS instead of rotated (3 DPP
 // moves per step instead of 7) is no faster once the moves have priority (2.95 against 2.86 ms
