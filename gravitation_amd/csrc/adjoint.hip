@@ -43,16 +43,22 @@ __global__ __launch_bounds__(kMuBlock) void k_adjoint_mu(const double *__restric
   const int b0 = offsets ? static_cast<int>(offsets[u]) : 0;
   const int b1 = offsets ? static_cast<int>(offsets[u + 1]) : n;
   // Bodies are taken U at a time per thread with all their loads issued before any store
-  // (nu is read and written, so the compiler would otherwise keep one body in flight).
+  // (nu is read and written, so the compiler would otherwise keep one body in flight).  A
+  // universe of at most U * kMuBlock bodies stays in registers between the two passes: bound by
+  // latency, so the second reading of nu showed.  MI355X, reading it again and held: 128
+  // universes of 64-2048 bodies 5.6 and 4.8 us, 512 of 64-4096 13.0 and 11.1, one of 2000 4.9 and
+  // 4.2; 512 of 32-256 4.4 both.
   constexpr int U = 4;
+  const bool resident = b1 - b0 <= U * kMuBlock;
+  double held[U][3];
   int e = INT_MIN;
-  auto body = [&](int i, const double (&nv)[3], const double (&rv)[3]) {
+  auto body = [&](int i, const double (&nv)[3], const double (&rv)[3], double (&mu)[3]) {
     double a = 0.0;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const double mu = nv[c] + dt * rv[c];
-      nu[c * n + i] = mu;
-      a = fmax(a, fabs(mu));  // NaN components drop out here
+      mu[c] = nv[c] + dt * rv[c];
+      nu[c * n + i] = mu[c];
+      a = fmax(a, fabs(mu[c]));  // NaN components drop out here
     }
     if (a > 0.0 && a <= DBL_MAX) {
       int x;
@@ -60,7 +66,27 @@ __global__ __launch_bounds__(kMuBlock) void k_adjoint_mu(const double *__restric
       e = max(e, x);
     }
   };
-  int i0 = b0 + static_cast<int>(threadIdx.x);
+  if (resident) {
+    double rv[U][3];
+#pragma unroll
+    for (int t = 0; t < U; ++t) {
+      const int i = b0 + static_cast<int>(threadIdx.x) + t * kMuBlock;
+      if (i < b1) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          held[t][c] = nu[c * n + i];
+          rv[t][c] = rho[c * n + i];
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < U; ++t) {
+      const int i = b0 + static_cast<int>(threadIdx.x) + t * kMuBlock;
+      if (i < b1) body(i, held[t], rv[t], held[t]);
+    }
+  }
+  double mu[3];
+  int i0 = resident ? b1 : b0 + static_cast<int>(threadIdx.x);
   for (; i0 + (U - 1) * kMuBlock < b1; i0 += U * kMuBlock) {
     double nv[U][3], rv[U][3];
 #pragma unroll
@@ -71,7 +97,7 @@ __global__ __launch_bounds__(kMuBlock) void k_adjoint_mu(const double *__restric
         rv[t][c] = rho[c * n + i0 + t * kMuBlock];
       }
 #pragma unroll
-    for (int t = 0; t < U; ++t) body(i0 + t * kMuBlock, nv[t], rv[t]);
+    for (int t = 0; t < U; ++t) body(i0 + t * kMuBlock, nv[t], rv[t], mu);
   }
   for (; i0 < b1; i0 += kMuBlock) {
     double nv[3], rv[3];
@@ -80,7 +106,7 @@ __global__ __launch_bounds__(kMuBlock) void k_adjoint_mu(const double *__restric
       nv[c] = nu[c * n + i0];
       rv[c] = rho[c * n + i0];
     }
-    body(i0, nv, rv);
+    body(i0, nv, rv, mu);
   }
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) e = max(e, __shfl_xor(e, off));
@@ -90,11 +116,19 @@ __global__ __launch_bounds__(kMuBlock) void k_adjoint_mu(const double *__restric
 #pragma unroll
   for (int w = 1; w < kMuBlock / kWave; ++w) E = max(E, wmax[w]);
   if (E == INT_MIN) E = 0;
-  // Each thread reads back only the nu entries it wrote above.
   auto scaled = [&](int i, const double (&m)[3]) {
     mu4[i] = make_float4(static_cast<float>(ldexp(m[0], -E)), static_cast<float>(ldexp(m[1], -E)),
                          static_cast<float>(ldexp(m[2], -E)), __int_as_float(E));
   };
+  if (resident) {
+#pragma unroll
+    for (int t = 0; t < U; ++t) {
+      const int i = b0 + static_cast<int>(threadIdx.x) + t * kMuBlock;
+      if (i < b1) scaled(i, held[t]);
+    }
+    return;
+  }
+  // Each thread reads back only the nu entries it wrote above.
   i0 = b0 + static_cast<int>(threadIdx.x);
   for (; i0 + (U - 1) * kMuBlock < b1; i0 += U * kMuBlock) {
     double m[U][3];

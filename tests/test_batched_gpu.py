@@ -394,3 +394,33 @@ def test_sym_pairs_of_small_and_large_launches_are_bitwise_equal(cuda, sym):
     assert torch.isfinite(few).all()
     for k in (0, 150, 299):
         assert torch.equal(many[:, k * s:(k + 1) * s], few)
+
+
+@pytest.mark.parametrize('sizes', [[1, 64, 1023, 1024, 1025], [4095, 4096, 4097, 2], [9000, 5, 3000]])
+def test_batched_mu_is_exact_at_the_register_limit(cuda, sizes):
+    # universes of up to 4096 bodies are held in registers between the two passes, larger ones
+    # read again: mu = nu + h rho rounded twice, and its copy scaled by the exponent of the
+    # universe's largest finite component, exactly
+    print('mu', sizes, flush=True)
+    rng = np.random.default_rng(sum(sizes))
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    n, dt = int(off[-1]), 1e-3
+    rho, nu = (rng.normal(size=(3, n)) * np.exp(rng.uniform(-20, 20, (3, n))) for _ in range(2))
+    nu[1, 0], nu[2, n - 1] = np.inf, np.nan
+    plan = batched.BatchedPlan(off)
+    d_rho, d_nu = torch.from_numpy(rho).to(cuda), torch.from_numpy(nu).to(cuda)
+    mu4 = torch.empty((n, 4), dtype=torch.float32, device=cuda)
+    _native.call('grav_batched_adjoint_mu', plan.handle, d_rho.data_ptr(), d_nu.data_ptr(),
+                 mu4.data_ptr(), dt, torch.cuda.current_stream().cuda_stream)
+    got = mu4.cpu()
+    want = nu + dt * rho
+    assert np.array_equal(d_nu.cpu().numpy(), want, equal_nan=True)
+    for u in range(len(sizes)):
+        a, b = int(off[u]), int(off[u + 1])
+        big = np.fmax.reduce(np.abs(want[:, a:b]), axis=0)   # a body with an infinity has no say
+        big = big[np.isfinite(big) & (big > 0)]
+        e = int(np.frexp(big.max())[1]) if big.size else 0
+        assert torch.all(got[a:b, 3].contiguous().view(torch.int32) == e)
+        with np.errstate(over='ignore', invalid='ignore'):
+            w = np.ldexp(want[:, a:b], -e).astype(np.float32).T
+        assert np.array_equal(got[a:b, :3].numpy(), w, equal_nan=True)
