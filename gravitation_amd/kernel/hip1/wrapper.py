@@ -16,9 +16,9 @@ Options (keyword arguments of the constructor; they travel through ``**kwargs`` 
   pair terms are FP32 and r, v accumulate in FP64.
 * ``graph`` (bool, default False): replay the two stages as HIP graphs captured at start();
   the results are those of the eager path, bit for bit.  Off by
-  default: on ROCm 7 one graph replay costs about 20 us against about 10 us for the direct
-  launch of the same kernel, so small universes step slower with graphs (57 against 46 us at
-  256 bodies) and large ones gain 1-8 %.
+  default: on ROCm 7 one graph replay costs about 17 us against about 5 us for the direct
+  launch of the same kernel, so universes step slower with graphs (45 against 18 us at 256
+  bodies, 107 against 96 us at 16384).
 * ``sync_host`` (bool, default True): refresh the host views after every step, so that
   ``pm._r`` / ``pm._v`` hold the new state when ``step()`` returns (README.md:50 of the
   reference requires it): the stage-2 kernel stores the new state into the mapped host mirror

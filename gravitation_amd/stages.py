@@ -110,12 +110,13 @@ _workspaces = {}
 
 
 # Form thresholds, from times on an MI355X.  FP32: one launch (owner-computes) beats the two of
-# the j-split form below 1088 bodies (a hip1 step of the galaxy, us, owner-computes against
-# j-split: 512 24.8 and 27.5, 1000 28.2 and 27.2, 1500 31.6 and 27.4, 2000 35.7 and 27.7).  The
-# j-split form beats the symmetric one below 19456, where few groups of its balanced form fit
-# its workspace (stage 1, Plummer, us, j-split against symmetric: 17000 76 against 114, 18500 92
-# against 128, 19456 95 against 82, 24576 146 against 132, 32768 251 against 200, 49999 577
-# against 450).  FP64: j-split from 448 bodies (a hip1 step of the galaxy, us, owner-computes
+# the j-split form below 1088 bodies while the state stays on the device (a hip1 step of the
+# galaxy, us, owner-computes against j-split: 512 10.3 and 13.5, 900 12.3 and 13.3, 1080 13.4 and
+# 13.4; with the host views refreshed, where the wait hides the launches, 512 21.3 and 21.4, 1000
+# 25.4 and 22.2, 2000 32.9 and 22.4).  The j-split form beats the symmetric one below 19456,
+# where few groups of its balanced form fit its workspace (stage 1, Plummer, us, j-split against
+# symmetric: 17000 76 against 114, 18500 92 against 128, 19456 95 against 82, 24576 146 against
+# 132, 32768 251 against 200, 49999 577 against 450).  FP64: j-split from 448 bodies (a hip1 step of the galaxy, us, owner-computes
 # against j-split, on the device and with the host views refreshed: 384 12.0 and 13.3, 25.1 and
 # 22.5; 448 14.0 and 13.2, 26.3 and 22.4; 640 17.0 and 13.3, 30.7 and 22.7; 1000 26.0 and 13.2,
 # 38.3 and 23.5), symmetric from 10500 (us, j-split against symmetric: 9000 52 against 50, 10000
