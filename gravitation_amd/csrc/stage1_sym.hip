@@ -25,6 +25,7 @@
 //   * batched universes list their block pairs as items, and one reduction kernel adds every
 //     body's diagonal-block sum and partials in a fixed order in FP64.
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -75,7 +76,12 @@ __device__ __forceinline__ float4 load_or_far(const float4 *__restrict__ posm, i
 // at 2^17), and temporaries pinned to registers of alternating parity (an FMA whose three
 // operands have register numbers of one parity issues alone) gain 1 %.  Without PRIO no priority
 // is raised, for launches that leave a SIMD to one wavefront (sym_prio).
-template <int K, bool OWN, bool PRIO = true>
+//
+// WIDE: the weights are (m/r) (1/r^2), as in the owner-computes and j-split forms, and hold for
+// every r whose square is an FP32 number (1e-19 to 1e19).  Otherwise both bodies share 1/r^3,
+// one multiplication less per pair (5 % of the time: 32768 bodies 240 against 253 us, 65536 846
+// against 886), which overflows below r = 1.4e-13 and loses its bits above 4.4e12.
+template <int K, bool OWN, bool PRIO = true, bool WIDE = false>
 __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const float eps2,
                                           const float (&xi)[K], const float (&yi)[K],
                                           const float (&zi)[K], const float (&mn)[K],
@@ -107,13 +113,14 @@ __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         if (OWN && t == 0 && k + g == kself) inv[g] = 0.0f;
-        const float inv3 = inv[g] * (inv[g] * inv[g]);
-        const float si = mj * inv3;
+        const float inv2 = inv[g] * inv[g];
+        const float inv3 = WIDE ? inv2 : inv[g] * inv2;
+        const float si = (WIDE ? mj * inv[g] : mj) * inv3;
         px[k + g] = __builtin_fmaf(dx[g], si, px[k + g]);
         py[k + g] = __builtin_fmaf(dy[g], si, py[k + g]);
         pz[k + g] = __builtin_fmaf(dz[g], si, pz[k + g]);
         if constexpr (!OWN) {
-          const float sj = mn[k + g] * inv3;
+          const float sj = (WIDE ? mn[k + g] * inv[g] : mn[k + g]) * inv3;
           tx = k + g == 0 ? dx[g] * sj : __builtin_fmaf(dx[g], sj, tx);
           ty = k + g == 0 ? dy[g] * sj : __builtin_fmaf(dy[g], sj, ty);
           tz = k + g == 0 ? dz[g] * sj : __builtin_fmaf(dz[g], sj, tz);
@@ -478,10 +485,10 @@ __host__ __device__ inline int64_t pair_row(int64_t beta, int64_t nb) {
 }
 
 // The i-side sums of K bodies per lane: FP32 chunk sums folded into TwoSum pairs, FP64 as is.
-template <typename T, int K>
+template <typename T, int K, bool WIDE>
 struct ISum;
-template <int K>
-struct ISum<float, K> {
+template <int K, bool WIDE>
+struct ISum<float, K, WIDE> {
   float h[3][K], l[3][K];
   __device__ __forceinline__ void clear() {
 #pragma unroll
@@ -495,7 +502,8 @@ struct ISum<float, K> {
     float px[K], py[K], pz[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) px[k] = py[k] = pz[k] = 0.0f;
-    sym_chunk<K, OWN>(q, kself, eps2, x[0], x[1], x[2], x[3], px, py, pz, aj[0], aj[1], aj[2]);
+    sym_chunk<K, OWN, true, WIDE>(q, kself, eps2, x[0], x[1], x[2], x[3], px, py, pz, aj[0],
+                                  aj[1], aj[2]);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       two_sum_sym(h[0][k], l[0][k], px[k]);
@@ -505,8 +513,8 @@ struct ISum<float, K> {
   }
   __device__ __forceinline__ float get(int c, int k) const { return h[c][k] + l[c][k]; }
 };
-template <int K>
-struct ISum<double, K> {
+template <int K, bool WIDE>
+struct ISum<double, K, WIDE> {
   double p[3][K];
   __device__ __forceinline__ void clear() {
 #pragma unroll
@@ -539,7 +547,7 @@ constexpr T kMassSign = sizeof(T) == 4 ? T(-1) : T(1);
 // (FP64, 40000 bodies: 23 of 690 us), no last round of workgroups that leaves half the compute
 // units idle, i-side partials once per group and row.  FP32 65536 bodies: 744 us = 55 cycles per
 // unordered pair and SIMD, of 50 that the loop can reach; 32768: 200 us, 59 cycles.
-template <typename T, typename T4, int K, int W>
+template <typename T, typename T4, int K, int W, bool WIDE>
 __global__ __launch_bounds__(kWave *W) void k_sym_units(const T4 *__restrict__ posm, int n,
                                                          int nb, int nc, int64_t units, T eps2,
                                                          T *__restrict__ p_i,
@@ -576,7 +584,7 @@ __global__ __launch_bounds__(kWave *W) void k_sym_units(const T4 *__restrict__ p
     const int c_end = beta * KW + static_cast<int>((u_end < r1 ? u_end : r1) - r0);
     u += c_end - c;
     T x[4][K];
-    ISum<T, K> sum;
+    ISum<T, K, WIDE> sum;
     sum.clear();
     const int i0 = beta * IB + wave * (K * kWave);
 #pragma unroll
@@ -974,6 +982,10 @@ constexpr int64_t kUnitGroups = 10 * kCus;
 // 2854 and 2862; FP64 9000 74 and 50 (52), 12288 100 and 77 (88), 20000 202 and 168 (227), 40000
 // 690 and 592 (876), 60000 1332 and 1297.
 constexpr int64_t kUnitsFrom = 18945, kUnitsTo = 114688;
+// FP32 sizes whose weights are WIDE (sym_chunk).  Below this size the form stands beside the
+// j-split form, whose range of distances it has to have, and is faster than it with the wider
+// weights too; from here on it stands beside the row segments, which share 1/r^3.
+constexpr int64_t kUnitsWideTo = 65536;
 constexpr int64_t kUnitsFromF64 = 8961, kUnitsToF64 = 65536;
 
 // groups: kUnitGroups, or the multiple of kCus below it whose i-side slots fit the workspace;
@@ -997,8 +1009,15 @@ int sym_units_run(const T4 *posm, T *acc, double *sums, int n, const UnitPlan &P
                   T eps2, void *ws, hipStream_t s) {
   T *p_j = static_cast<T *>(ws);
   T *p_i = reinterpret_cast<T *>(static_cast<char *>(ws) + P.j_bytes);
-  hipLaunchKernelGGL((k_sym_units<T, T4, K, W>), dim3(static_cast<unsigned>(P.groups)),
-                     dim3(kWave * W), 0, s, posm, n, P.nb, P.nc, P.units, eps2, p_i, p_j);
+  auto launch = [&](auto wide) {
+    hipLaunchKernelGGL((k_sym_units<T, T4, K, W, decltype(wide)::value>),
+                       dim3(static_cast<unsigned>(P.groups)), dim3(kWave * W), 0, s, posm, n, P.nb,
+                       P.nc, P.units, eps2, p_i, p_j);
+  };
+  if (sizeof(T) == 4 && n < kUnitsWideTo)
+    launch(std::integral_constant<bool, sizeof(T) == 4>());
+  else
+    launch(std::false_type());
   const int rc = check_launch("k_sym_units");
   if (rc != GRAV_OK) return rc;
   hipLaunchKernelGGL((k_sym_units_fold<T>), dim3(static_cast<unsigned>(P.nc)),

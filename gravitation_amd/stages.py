@@ -127,6 +127,10 @@ SYMMETRIC_FROM = 19456
 SPLIT_F64_FROM = 448
 SYMMETRIC_F64_FROM = 10500
 VJP_SPLIT_FROM = 1024
+# Below this size the symmetric form, given its one-slab workspace, weighs a pair as the owner and
+# j-split forms do, for distances r from 1e-19 to 1e19; from here on it shares 1/r^3 between the
+# two bodies of a pair and needs r between 1.4e-13 and 4.4e12 (or eps above the lower limit).
+SYMMETRIC_WIDE_TO = 65536
 
 
 def auto_form(n, accum='kahan', free_bytes=None, dtype='float32'):
@@ -168,9 +172,13 @@ def sym_workspace_size(n, cfg=None, free_bytes=None, dtype='float32', device=Non
     """The workspace to allocate for the symmetric form: its one-slab size when that fits a
     quarter of the free device memory (``free_bytes``, default: measured on ``device``), else
     that quarter (at least the form's minimum).  Any size from the minimum up gives the same
-    accelerations to rounding; fewer slabs save a few launches and fold passes."""
+    accelerations to rounding; fewer slabs save a few launches and fold passes.  In FP32 below
+    SYMMETRIC_WIDE_TO bodies always the one-slab size (at most 77 MB): less would take the
+    library to row segments, which do not have the j-split form's range of distances."""
     of = sym_f64_workspace_bytes if dtype == 'float64' else sym_workspace_bytes
     full = of(n, cfg)
+    if cfg is None and dtype == 'float32' and n < SYMMETRIC_WIDE_TO:
+        return full
     if free_bytes is None:
         import torch
         free_bytes, _ = torch.cuda.mem_get_info(device)

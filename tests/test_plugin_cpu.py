@@ -82,6 +82,18 @@ def test_auto_form_needs_the_workspace_to_fit():
     assert stages.sym_workspace_size(n, free_bytes=least) == least
 
 
+def test_symmetric_sizes_of_the_split_forms_range_get_the_whole_workspace():
+    # below SYMMETRIC_WIDE_TO a smaller workspace would take the library to row segments, whose
+    # range of distances is narrower than that of the form that served these sizes before
+    from gravitation_amd import stages
+    for n in (stages.SYMMETRIC_FROM, 57343, stages.SYMMETRIC_WIDE_TO - 1):
+        full = stages.sym_workspace_bytes(n)
+        assert stages.sym_workspace_size(n, free_bytes=full) == full
+    n = stages.SYMMETRIC_WIDE_TO
+    assert stages.sym_workspace_size(n, free_bytes=stages.sym_workspace_bytes(n)) < \
+        stages.sym_workspace_bytes(n)
+
+
 def test_auto_form_f64_threshold():
     from gravitation_amd import stages
     assert stages.auto_form(stages.SPLIT_F64_FROM - 1, dtype='float64') == 'owner'

@@ -565,6 +565,27 @@ def test_symmetric_default_shape_at_its_size_limits(cuda, n, dtype):
     stages.release_workspaces()
 
 
+@pytest.mark.parametrize('n', [19456, 57344, 65535])
+@pytest.mark.parametrize('size, mass', [(1e15, 1e20), (1e-10, 1e-12), (1.0, 1.0)])
+def test_symmetric_middle_sizes_have_the_range_of_the_split_form(cuda, n, size, mass):
+    # Sizes that the j-split form served before the symmetric one took them over: universes in
+    # metres (1/r^3 below FP32's smallest number) and of tiny units (above its largest at close
+    # pairs), where m/r and 1/r^2 are ordinary numbers, to the bar of every other size.
+    print('sym range n=%d size=%g' % (n, size), flush=True)
+    rng = np.random.default_rng(n)
+    posm = _posm(rng.uniform(0.0, size, (n, 3)),
+                 mass * np.exp(rng.uniform(np.log(1e-4), np.log(1e-2), n)), cuda)
+    pos, m = _inputs(posm)
+    rows = np.unique(np.concatenate([rng.choice(n, 200, replace=False), [0, n - 1]]))
+    ref = oracle_rows(pos, m, 1.0, 0.0, rows)
+    for run in (stages.stage1_split_f32, stages.stage1_sym_f32):
+        acc = torch.full((3, n), float('nan'), dtype=torch.float32, device=cuda)
+        run(posm, acc, 1.0, 0.0)
+        a = acc.cpu().numpy().T.astype(np.float64)
+        assert np.all(np.isfinite(a)), run
+        assert O.rel_err(a[rows], ref) < TOL32, run
+
+
 @pytest.mark.parametrize('n', [65, 4096, 5000, 20000])
 def test_split_step_io_is_bitwise_in_place(cuda, n):
     # grav_step_split_f64m_io (new positions to another buffer, as the recomputed segments of
