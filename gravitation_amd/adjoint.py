@@ -288,10 +288,17 @@ def _stage1_form(n, form):
     return stages.auto_form(n) if form == 'auto' else form
 
 
+def _stage1_workspace(n, dev, form):
+    """A workspace of the stage-1 form for n."""
+    form = _stage1_form(n, form)
+    return stages.scratch(stages.sym_workspace_size(n, device=dev) if form == 'symmetric'
+                          else stages.split_workspace_bytes(n) if form == 'split' else 0, dev)
+
+
 def _stage1(posm, acc, G, eps, form='auto', ws=None):
     """FP32 compensated stage 1 in the faster form for n, or owner-computes with
     form='owner' (forward and recompute use the same one, so a recomputed segment equals the
-    recorded one bit for bit).  ``ws``: the form's workspace (default: the shared one)."""
+    recorded one bit for bit).  ``ws``: the form's workspace (default: the call's own)."""
     form = _stage1_form(posm.shape[0], form)
     if form == 'symmetric':
         stages.stage1_sym_f32(posm, acc, G, eps, None, ws)
@@ -319,8 +326,8 @@ def _vjp_split(n, form):
 
 def _vjp(posm, mu4, rho, gamma, G, eps, dt, form='auto', ws=None):
     """The VJP in the faster form for n (j-split from VJP_SPLIT_FROM bodies), or
-    owner-computes with form='owner'.  ``ws``: the j-split workspace (default: the shared
-    one)."""
+    owner-computes with form='owner'.  ``ws``: the j-split workspace (default: the call's
+    own)."""
     if _vjp_split(posm.shape[0], form):
         stage1_vjp_split_f32(posm, mu4, rho, gamma, G, eps, dt, None, ws)
     else:
@@ -365,9 +372,7 @@ class _SegmentGraphs:
         self.mu4 = torch.empty((n, 4), dtype=f32, device=dev)
         self.eslot = torch.empty((2,), dtype=torch.int32, device=dev)
         s1 = _stage1_form(n, form)
-        need = (stages.sym_workspace_size(n, device=dev) if s1 == 'symmetric'
-                else stages.split_workspace_bytes(n) if s1 == 'split' else 0)
-        self.ws = torch.empty((max(need, 256),), dtype=torch.uint8, device=dev)
+        self.ws = _stage1_workspace(n, dev, form)
         self.io = s1 == 'split'
         self.chain = CHAIN and _vjp_split(n, form)
         self.paired = OVERLAP and self.io and self.chain and records == 2
@@ -378,7 +383,7 @@ class _SegmentGraphs:
         if self.paired:
             need = max(need, backward_pair_workspace_bytes(n))
         need = max(need, 4 * ((n + 1023) // 1024))
-        self.ws_adj = torch.empty((max(need, 256),), dtype=torch.uint8, device=dev)
+        self.ws_adj = stages.scratch(need, dev)
         self.graphs = {}
         # the token of the forward pass whose last segment the record buffers hold (the
         # backward of that pass need not recompute it); any other use of them clears it
@@ -550,6 +555,7 @@ class _Single(torch.autograd.Function):
         if sg is not None:
             posm, acc, r64, v64 = sg.posm, sg.acc, sg.r64, sg.v64
         else:
+            ws = _stage1_workspace(n, dev, form)
             posm = torch.empty((n, 4), dtype=torch.float32, device=dev)
             acc = torch.empty((3, n), dtype=torch.float32, device=dev)
             r64 = torch.empty((3, n), dtype=torch.float64, device=dev)
@@ -560,7 +566,7 @@ class _Single(torch.autograd.Function):
         _load_state(r0, v0, m, slots[0], r64, v64)
         checkpoints = []
         for p, q in zip(slots, slots[1:]):
-            _step(p, acc, r64, v64, G, eps, dt, form, out=q)
+            _step(p, acc, r64, v64, G, eps, dt, form, ws, out=q)
         t = steps if store else 0
         while t < steps:
             checkpoints.append((r64.clone(), v64.clone()))
@@ -573,7 +579,7 @@ class _Single(torch.autograd.Function):
                 sg.run('fwd', k)
             else:
                 for _ in range(k):
-                    _step(posm, acc, r64, v64, G, eps, dt, form)
+                    _step(posm, acc, r64, v64, G, eps, dt, form, ws)
             t += k
         ctx.cfg = (G, eps, dt, steps, interval, store, form, graph)
         ctx.traj = traj

@@ -167,7 +167,9 @@ def _slots_of(traj, posm, steps, n):
 
 class Engine:
     """A plan plus a schedule ('fused', 'perstep' or 'perstep-sym'); advances and
-    differentiates the concatenated state of all universes on the current stream."""
+    differentiates the concatenated state of all universes on the current stream.  Calls on
+    different states may run on several streams or threads at once, except the forward ones of
+    'perstep-sym', which share the engine's workspace."""
 
     def __init__(self, offsets, config=DEFAULT_CONFIG, device=None):
         if len(config) not in (6, 7):
@@ -193,9 +195,6 @@ class Engine:
         self.mode = mode
         self.j_waves = int(jw)
         self.config = (mode,) + self.plan.config + (int(jw),)
-        self._acc = None
-        self._pos2 = None
-        self._mu4 = None
         self._ws = None
         if mode == 'perstep-sym':
             self.config += (sym,)
@@ -221,13 +220,6 @@ class Engine:
                                  % (t.device, self.plan.device))
         return stages.on_device(self.plan.device)
 
-    def _buf(self, name, shape, dtype, dev):
-        b = getattr(self, name)
-        if b is None or b.device != dev or tuple(b.shape) != shape:
-            b = torch.empty(shape, dtype=dtype, device=dev)
-            setattr(self, name, b)
-        return b
-
     def forward(self, posm, r64, v64, G, eps, dt, steps, traj=None):
         """``steps`` steps of every universe; traj (steps, n, 4) float32 or None receives posm
         at the start of every step."""
@@ -241,7 +233,7 @@ class Engine:
             if self._ws is None:
                 self._forward_items(posm, r64, v64, G, eps, dt, steps, traj)
                 return
-            acc = self._buf('_acc', (3, self.n), torch.float32, dev)
+            acc = torch.empty((3, self.n), dtype=torch.float32, device=dev)
             for t in range(steps):
                 if traj is not None:
                     traj[t].copy_(posm)
@@ -253,7 +245,7 @@ class Engine:
     def _forward_items(self, posm, r64, v64, G, eps, dt, steps, traj):
         """``forward`` of the 'perstep' schedule: a step is one launch from one position buffer
         to another, through the record's slots or back and forth between posm and a buffer of
-        the engine's.  A single step without a record, and steps into a record whose slots are
+        the call's own.  A single step without a record, and steps into a record whose slots are
         no float32 position buffers of their own, run their two stages in place."""
         n = self.n
         for t, name, dtype, shape in ((posm, 'posm', torch.float32, (n, 4)),
@@ -265,7 +257,7 @@ class Engine:
         bufs, in_place = [posm], steps % 2
         if traj is None:
             if steps > 1:
-                other = self._buf('_pos2', (n, 4), torch.float32, dev)
+                other = torch.empty((n, 4), dtype=torch.float32, device=dev)
                 bufs = [posm, other] * (steps // 2) + [posm]
         elif steps and _slots_of(traj, posm, steps, n):
             in_place = 0
@@ -273,8 +265,9 @@ class Engine:
             bufs = [traj[t] for t in range(steps)] + [posm]
         else:
             in_place = steps
+        if in_place:
+            acc = torch.empty((3, n), dtype=torch.float32, device=dev)
         for t in range(in_place):
-            acc = self._buf('_acc', (3, n), torch.float32, dev)
             if traj is not None:
                 traj[t].copy_(posm)
             _native.call('grav_batched_stage1_f32', self.plan.handle, posm.data_ptr(),
@@ -294,7 +287,7 @@ class Engine:
                              rho.data_ptr(), nu.data_ptr(), gamma.data_ptr(), G, eps, dt,
                              int(steps), _stream(dev))
                 return
-            mu4 = self._buf('_mu4', (self.n, 4), torch.float32, dev)
+            mu4 = torch.empty((self.n, 4), dtype=torch.float32, device=dev)
             for t in range(steps - 1, -1, -1):
                 _native.call('grav_batched_adjoint_mu', self.plan.handle, rho.data_ptr(),
                              nu.data_ptr(), mu4.data_ptr(), dt, _stream(dev))
@@ -361,9 +354,6 @@ class Batch:
         s = torch.cuda.Stream(self.device)
         s.wait_stream(torch.cuda.current_stream(self.device))
         with torch.cuda.stream(s):
-            if self.engine.mode != 'fused':
-                self.engine._buf('_acc', (3, self.n), torch.float32, self.device)
-                self.engine._buf('_pos2', (self.n, 4), torch.float32, self.device)
             with torch.cuda.graph(g, stream=s):
                 self.step(steps)
         torch.cuda.current_stream(self.device).wait_stream(s)

@@ -12,6 +12,7 @@ torch's current HIP stream to libgravhip.  Layouts:
 
 import contextlib
 import ctypes
+import functools
 
 import torch
 
@@ -106,9 +107,6 @@ def stage1_f32(posm, acc, G, eps=0.0, accum='kahan', cfg=None):
     return acc
 
 
-_workspaces = {}
-
-
 # Form thresholds, from times on an MI355X.  FP32: one launch (owner-computes) beats the two of
 # the j-split form below 1088 bodies while the state stays on the device (a hip1 step of the
 # galaxy, us, owner-computes against j-split: 512 10.3 and 13.5, 900 12.3 and 13.3, 1080 13.4 and
@@ -180,7 +178,6 @@ def sym_workspace_size(n, cfg=None, free_bytes=None, dtype='float32', device=Non
     if cfg is None and dtype == 'float32' and n < SYMMETRIC_WIDE_TO:
         return full
     if free_bytes is None:
-        import torch
         free_bytes, _ = torch.cuda.mem_get_info(device)
     cap = free_bytes // 4
     if full <= cap:
@@ -188,23 +185,40 @@ def sym_workspace_size(n, cfg=None, free_bytes=None, dtype='float32', device=Non
     return max(of(n, cfg, minimum=True), cap & ~255)
 
 
+def scratch(nbytes, device):
+    """Device scratch of one call or object.  From torch's allocator on each call rather than kept
+    here: two calls on different streams or threads, whose launches may interleave, never get
+    the same memory while either needs it, and nothing outlives its use (about 2 us of host)."""
+    return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
+
+
+_sym_sizes = {}   # workspace bytes per (precision, device, n, cfg), so that repeated calls agree
+
+
+def _sym_workspace(t, n, cfg, dtype):
+    key = (dtype, t.device, n, None if cfg is None else tuple(cfg))
+    size = _sym_sizes.get(key)
+    if size is None:
+        size = _sym_sizes[key] = sym_workspace_size(n, cfg, dtype=dtype, device=t.device)
+    try:
+        return scratch(size, t.device)
+    except torch.cuda.OutOfMemoryError:   # the memory was free when the size was chosen
+        size = _sym_sizes[key] = sym_workspace_size(n, cfg, dtype=dtype, device=t.device)
+        return scratch(size, t.device)
+
+
 def stage1_sym_f32(posm, acc, G, eps=0.0, cfg=None, workspace=None):
     """acc (3, n) <- FP32 accelerations of posm (n, 4), symmetric form (each pair once).
     cfg = (i_chunks_per_wave, waves), None for the library's shape for n.  ``workspace``: a
     uint8 device tensor of at least ``sym_workspace_bytes(n, cfg, minimum=True)`` bytes (the
     form runs in slabs of rows below ``sym_workspace_bytes(n, cfg)``); by default one of
-    ``sym_workspace_size`` bytes is kept per (device, n, cfg)."""
+    ``sym_workspace_size`` bytes, the call's own."""
     n = posm.shape[0]
     _check(posm, 'posm', torch.float32, (n, 4))
     _check(acc, 'acc', torch.float32, (3, n))
     same_device(posm, acc)
     if workspace is None:
-        key = (posm.device, n, None if cfg is None else tuple(cfg))
-        workspace = _workspaces.get(key)
-        if workspace is None:
-            size = sym_workspace_size(n, cfg, device=posm.device)
-            workspace = torch.empty((max(size, 256),), dtype=torch.uint8, device=posm.device)
-            _workspaces[key] = workspace
+        workspace = _sym_workspace(posm, n, cfg, 'float32')
     same_device(posm, workspace)
     need = sym_workspace_bytes(n, cfg, minimum=True)
     if workspace.numel() < need:
@@ -237,12 +251,7 @@ def stage1_sym_f64(posm64, acc64, G, eps=0.0, cfg=None, workspace=None):
     _check(acc64, 'acc64', torch.float64, (3, n))
     same_device(posm64, acc64)
     if workspace is None:
-        key = ('f64', posm64.device, n, None if cfg is None else tuple(cfg))
-        workspace = _workspaces.get(key)
-        if workspace is None:
-            size = sym_workspace_size(n, cfg, dtype='float64', device=posm64.device)
-            workspace = torch.empty((max(size, 256),), dtype=torch.uint8, device=posm64.device)
-            _workspaces[key] = workspace
+        workspace = _sym_workspace(posm64, n, cfg, 'float64')
     same_device(posm64, workspace)
     need = sym_f64_workspace_bytes(n, cfg, minimum=True)
     if workspace.numel() < need:
@@ -271,29 +280,27 @@ def check_split_cfg(cfg, dtype='float32'):
 def split_workspace_bytes(n, cfg=None):
     """Workspace bytes of the j-split forms (stage 1 and its VJP share the size); cfg =
     (i_per_lane, j_waves, splits), None for the library's shape for n."""
-    p = int(cfg[2]) if cfg is not None else 0
+    return _split_bytes(int(n), int(cfg[2]) if cfg is not None else 0)
+
+
+@functools.lru_cache(maxsize=256)
+def _split_bytes(n, splits):
     b = ctypes.c_int64(0)
-    _native.call('grav_stage1_split_workspace', int(n), p, ctypes.byref(b))
+    _native.call('grav_stage1_split_workspace', n, splits, ctypes.byref(b))
     return b.value
 
 
 def split_workspace(t, n, cfg=None):
-    """A cached uint8 workspace of the j-split forms on t's device for n bodies."""
-    key = ('split', t.device, n, None if cfg is None else tuple(cfg))
-    ws = _workspaces.get(key)
-    if ws is None:
-        ws = torch.empty((max(split_workspace_bytes(n, cfg), 256),), dtype=torch.uint8,
-                         device=t.device)
-        _workspaces[key] = ws
-    return ws
+    """A new uint8 workspace of the j-split forms on t's device for n bodies."""
+    return scratch(split_workspace_bytes(n, cfg), t.device)
 
 
 def stage1_split_f32(posm, acc, G, eps=0.0, cfg=None, workspace=None):
     """acc (3, n) <- FP32-compensated accelerations of posm (n, 4) in the j-split
     owner-computes form (each i-tile also split over j-ranges, for small n).  cfg =
     (i_per_lane, j_waves, splits), None for the library's shape for n.  ``workspace``: a
-    uint8 device tensor of at least ``split_workspace_bytes(n, cfg)`` bytes; by default one is
-    kept per (device, n, cfg)."""
+    uint8 device tensor of at least ``split_workspace_bytes(n, cfg)`` bytes; by default the
+    call's own."""
     n = posm.shape[0]
     _check(posm, 'posm', torch.float32, (n, 4))
     _check(acc, 'acc', torch.float32, (3, n))
@@ -325,19 +332,15 @@ def stage1_sym_f32_share(posm, sums, share, shares, eps=0.0, cfg=None, workspace
     """sums (3, n) float64 <- the unscaled contribution of share `share` of `shares` of the
     symmetric form (its rows of block pairs and their diagonal blocks) to every body's
     acceleration: one GPU's part when the form is divided among GPUs.  ``workspace``: a uint8
-    device tensor of at least the share's minimum bytes (``sym_share_plan``); by default one of
-    its full size is kept per (device, n, share, shares, cfg)."""
+    device tensor of at least the share's minimum bytes (``sym_share_plan``); by default the
+    call's own, of its full size."""
     n = posm.shape[0]
     _check(posm, 'posm', torch.float32, (n, 4))
     _check(sums, 'sums', torch.float64, (3, n))
     same_device(posm, sums)
     if workspace is None:
-        key = ('sym_share', posm.device, n, share, shares, None if cfg is None else tuple(cfg))
-        workspace = _workspaces.get(key)
-        if workspace is None:
-            _, full, _ = sym_share_plan(n, share, shares, cfg)
-            workspace = torch.empty((full,), dtype=torch.uint8, device=posm.device)
-            _workspaces[key] = workspace
+        _, full, _ = sym_share_plan(n, share, shares, cfg)
+        workspace = scratch(full, posm.device)
     same_device(posm, workspace)
     k, w = cfg if cfg is not None else (0, 0)
     with on_device(posm):
@@ -376,8 +379,8 @@ def stage1_shard_f32(posm, acc, i0, G, eps=0.0, cfg=None, workspace=None):
     against all n: one GPU's share when a universe is divided among GPUs by i-range.  Bit for
     bit rows i0 .. i0 + m - 1 of ``stage1_f32(..., 'kahan', (k, s, 256))`` for cfg (k, s, 1),
     or of ``stage1_split_f32(..., cfg)`` for cfg (k, s, splits > 1).  cfg None: ``shard_cfg``'s.
-    ``workspace`` (splits > 1): at least ``split_workspace_bytes(m, cfg)`` bytes; by default one
-    is kept per (device, m, cfg)."""
+    ``workspace`` (splits > 1): at least ``split_workspace_bytes(m, cfg)`` bytes; by default the
+    call's own."""
     n = posm.shape[0]
     m = acc.shape[1] if acc.dim() == 2 else -1
     _check(posm, 'posm', torch.float32, (n, 4))
@@ -445,7 +448,9 @@ def stage1_split_f64(posm64, acc64, G, eps=0.0, cfg=None, workspace=None):
 
 
 def release_workspaces():
-    _workspaces.clear()
+    """Forgets the workspace sizes chosen so far: the next call of the symmetric form without a
+    workspace goes by the free memory of that moment."""
+    _sym_sizes.clear()
 
 
 def stage1_f64(posm64, acc64, G, eps=0.0):

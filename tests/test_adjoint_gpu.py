@@ -804,3 +804,61 @@ def test_contiguous_rows_equal_the_general_path(cuda, n):
     stages.stage2_f64m(p, *b, acc, 1e-2)
     for x, y in zip((q, *a), (p, *b)):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize('n', [1500, 3000])
+def test_passes_on_two_streams_do_not_share_scratch(cuda, n):
+    # trajectories of one size (recorded, checkpointed and eager, and through one batched
+    # engine, with odd numbers of steps) and plain stage calls, alternating between two streams
+    # without a wait: the bits of the same passes one after the other
+    from gravitation_amd import batched, stages
+    print('streams', n, flush=True)
+    rng = np.random.default_rng(n)
+    eng = batched.Engine(np.array([0, n // 3, n]), ('perstep', 8, 1, 8, 0, 4), cuda)
+    kw = dict(G=1.0, eps=1e-2, dt=1e-3)
+    states = []
+    for _ in range(2):
+        states.append([torch.from_numpy(x).to(cuda) for x in
+                       (rng.normal(size=(n, 3)), rng.normal(size=(n, 3)),
+                        rng.uniform(0.1, 1.0, n) / n)])
+    w = torch.from_numpy(rng.normal(size=(n, 3))).to(cuda)
+
+    def passes(state):
+        out = []
+        for run in (lambda *x: adjoint.trajectory(*x, 9, **kw),
+                    lambda *x: adjoint.trajectory(*x, 9, interval=4, graph=False, **kw),
+                    lambda *x: adjoint.batched_trajectory(eng, *x, 9, **kw),
+                    lambda *x: adjoint.batched_trajectory(eng, *x, 9, interval=3, **kw)):
+            leaves = [x.clone().requires_grad_(True) for x in state]
+            res = run(*leaves)
+            yield
+            out += [x.detach() for x in res] + list(torch.autograd.grad(res, leaves, [w, w]))
+            yield
+        posm = torch.cat([state[0], state[2][:, None]], 1).float()
+        for _ in range(4):
+            for f in (stages.stage1_split_f32, stages.stage1_sym_f32):
+                out.append(f(posm, torch.empty((3, n), device=cuda), 1.0, 1e-2))
+            yield
+        yield out
+
+    def last(it):
+        for x in it:
+            pass
+        return x
+
+    want = [last(passes(s)) for s in states]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        streams = [torch.cuda.Stream(cuda) for _ in states]
+        its, got = [passes(s) for s in states], [None, None]
+        for s in streams:
+            s.wait_stream(torch.cuda.current_stream())
+        for step in range(13):
+            for k, s in enumerate(streams):
+                with torch.cuda.stream(s):
+                    got[k] = next(its[k])
+        torch.cuda.synchronize()
+        for a, b in zip(want, got):
+            assert len(a) == len(b)
+            for x, y in zip(a, b):
+                assert torch.equal(x, y)

@@ -94,6 +94,16 @@ def test_symmetric_sizes_of_the_split_forms_range_get_the_whole_workspace():
         stages.sym_workspace_bytes(n)
 
 
+def test_calls_do_not_share_a_workspace():
+    # two calls of one size may run on two streams or threads: each has memory of its own
+    import torch
+    from gravitation_amd import stages
+    t = torch.empty((1500, 4))
+    a, b = stages.split_workspace(t, 1500), stages.split_workspace(t, 1500)
+    assert a.numel() >= stages.split_workspace_bytes(1500)
+    assert a.data_ptr() + a.numel() <= b.data_ptr() or b.data_ptr() + b.numel() <= a.data_ptr()
+
+
 def test_auto_form_f64_threshold():
     from gravitation_amd import stages
     assert stages.auto_form(stages.SPLIT_F64_FROM - 1, dtype='float64') == 'owner'
