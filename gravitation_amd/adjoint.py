@@ -353,8 +353,8 @@ class _SegmentGraphs:
 
     The forward and recompute state (posm, acc, r64, v64, ws) and the adjoint state (rho, nu,
     gamma, mu4, eslot, ws_adj) are separate, and there are two record buffers, so that the
-    recomputation of one segment can share launches with the adjoint steps of the next.  In
-    the j-split form a recomputed step goes from one record slot to the next (no copy), and a
+    recomputation of one segment can share launches with the adjoint steps of the next.  A
+    recomputed step goes from one record slot to the next (no copy), and with the j-split VJP a
     backward step is chained (its reduce forms the next cotangent)."""
 
     def __init__(self, n, dev, G, eps, dt, interval, form, records=2):
@@ -371,11 +371,10 @@ class _SegmentGraphs:
         self.gamma = torch.empty((n,), dtype=f64, device=dev)
         self.mu4 = torch.empty((n, 4), dtype=f32, device=dev)
         self.eslot = torch.empty((2,), dtype=torch.int32, device=dev)
-        s1 = _stage1_form(n, form)
         self.ws = _stage1_workspace(n, dev, form)
-        self.io = s1 == 'split'
         self.chain = CHAIN and _vjp_split(n, form)
-        self.paired = OVERLAP and self.io and self.chain and records == 2
+        self.paired = (OVERLAP and self.chain and records == 2
+                       and _stage1_form(n, form) == 'split')
         # the adjoint's own workspace: the j-split VJP's partials (or the paired steps' two
         # sets) and grav_adjoint_mu_ws's exponents, each finished with it before the next
         # starts on the same stream
@@ -402,12 +401,12 @@ class _SegmentGraphs:
         each one uses into record buffer ``buf``: slots 0 .. k-1 are then what the backward's
         recomputation of this segment would write (the same step kernels on the same state),
         and the last step goes back into posm."""
-        G, eps, dt, _, _ = self.cfg
+        G, eps, dt, _, form = self.cfg
         traj = self.traj[buf]
         traj[0].copy_(self.posm)
         for t in range(k):
-            stages.step_split_f64m(traj[t], self.r64, self.v64, G, eps, dt, None, self.ws,
-                                   out=traj[t + 1] if t + 1 < k else self.posm)
+            _step(traj[t], self.acc, self.r64, self.v64, G, eps, dt, form, self.ws,
+                  out=traj[t + 1] if t + 1 < k else self.posm)
 
     def load(self, r_c, v_c, mass, buf):
         """A checkpoint (r, v) into the recompute state and slot 0 of record buffer ``buf``."""
@@ -422,16 +421,9 @@ class _SegmentGraphs:
         segment's last step is not needed: its result is the next checkpoint)."""
         G, eps, dt, _, form = self.cfg
         traj = self.traj[buf]
-        if self.io:
-            for t in range(k - 1):
-                stages.step_split_f64m(traj[t], self.r64, self.v64, G, eps, dt, None, self.ws,
-                                       out=traj[t + 1])
-            return
-        if k > 1:
-            self.posm.copy_(traj[0])
         for t in range(k - 1):
-            self.step()
-            traj[t + 1].copy_(self.posm)
+            _step(traj[t], self.acc, self.r64, self.v64, G, eps, dt, form, self.ws,
+                  out=traj[t + 1])
 
     def begin_backward(self, g_r, g_v):
         """The adjoint state from the trajectory's cotangents, with a cleared exponent slot, and
@@ -520,9 +512,10 @@ def _backward_segments(sg, checkpoints, mass, steps, interval, graph, recorded=F
     sg.recorded = None
     if not sg.paired:
         for c in range(C - 1, -1, -1):
-            r_c, v_c = checkpoints[c]
-            sg.load(r_c, v_c, mass, 0)
-            sg.run('rec', seg_k[c], 0, graph=graph)
+            if not recorded or c < C - 1:
+                r_c, v_c = checkpoints[c]
+                sg.load(r_c, v_c, mass, 0)
+                sg.run('rec', seg_k[c], 0, graph=graph)
             sg.run('adj', seg_k[c], 0, c == 0, graph=graph)
         return
     if not recorded:
@@ -571,9 +564,9 @@ class _Single(torch.autograd.Function):
         while t < steps:
             checkpoints.append((r64.clone(), v64.clone()))
             k = min(interval, steps - t)
-            if sg is not None and sg.paired and t + k == steps:
+            if sg is not None and t + k == steps:
                 # the last segment records its positions for the backward pass
-                sg.run('fwdrec', k, (len(checkpoints) - 1) % 2)
+                sg.run('fwdrec', k, (len(checkpoints) - 1) % 2 if sg.paired else 0)
                 ctx.rec_token = sg.recorded = object()
             elif sg is not None:
                 sg.run('fwd', k)

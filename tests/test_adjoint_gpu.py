@@ -9,6 +9,8 @@
 * checkpoint-and-recompute equal to the recorded trajectory, bit for bit.
 """
 
+import collections
+
 import numpy as np
 import pytest
 import torch
@@ -811,7 +813,6 @@ def test_passes_on_two_streams_do_not_share_scratch(cuda, n):
     # trajectories of one size (recorded, checkpointed and eager, and through one batched
     # engine, with odd numbers of steps) and plain stage calls, alternating between two streams
     # without a wait: the bits of the same passes one after the other
-    from gravitation_amd import batched, stages
     print('streams', n, flush=True)
     rng = np.random.default_rng(n)
     eng = batched.Engine(np.array([0, n // 3, n]), ('perstep', 8, 1, 8, 0, 4), cuda)
@@ -862,3 +863,36 @@ def test_passes_on_two_streams_do_not_share_scratch(cuda, n):
             assert len(a) == len(b)
             for x, y in zip(a, b):
                 assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize('form', ['owner', 'split', 'symmetric'])
+def test_checkpointed_pass_of_every_form_recomputes_no_recorded_segment(cuda, form, monkeypatch):
+    # 2 segments of 4 and 3 steps in each stage-1 form: the backward pass takes the last
+    # segment's positions from the forward pass (its 2 recomputed steps would be seen here; the
+    # full segment replays its graph), and gives the recorded trajectory's bits
+    n = 1300
+    print('checkpointed', form, flush=True)
+    monkeypatch.setattr(stages, 'SPLIT_FROM', n + 1 if form == 'owner' else 1)
+    monkeypatch.setattr(stages, 'SYMMETRIC_FROM', 1 if form == 'symmetric' else n + 1)
+    assert stages.auto_form(n) == form
+    monkeypatch.setattr(adjoint, '_SEGMENT_GRAPHS', collections.OrderedDict())
+    rng = np.random.default_rng(17)
+    r, v, w = (torch.from_numpy(rng.normal(size=(n, 3))).to(cuda) for _ in range(3))
+    m = torch.from_numpy(rng.uniform(0.1, 1.0, n)).to(cuda)
+    names = []
+    call = _native.call
+    monkeypatch.setattr(_native, 'call', lambda name, *a: (names.append(name), call(name, *a))[1])
+    kw = dict(G=1.25, eps=1.5e-2, dt=1e-3)
+    got = []
+    for interval in (None, 4, 4):
+        leaves = [x.clone().requires_grad_(True) for x in (r, v, m)]
+        out = adjoint.trajectory(*leaves, 7, interval=interval, budget=1 << 30, **kw)
+        names.clear()
+        grads = torch.autograd.grad(out, leaves, [w, w])
+        got.append([x.detach() for x in out] + list(grads))
+    steps = [x for x in names if x.startswith(('grav_stage1_f32', 'grav_stage1_sym_f32',
+                                               'grav_step_split', 'grav_stage2'))]
+    assert steps == []
+    for other in got[1:]:
+        for x, y in zip(got[0], other):
+            assert torch.equal(x, y)
