@@ -288,11 +288,15 @@ def _stage1_form(n, form):
     return stages.auto_form(n) if form == 'auto' else form
 
 
-def _stage1_workspace(n, dev, form):
-    """A workspace of the stage-1 form for n."""
-    form = _stage1_form(n, form)
-    return stages.scratch(stages.sym_workspace_size(n, device=dev) if form == 'symmetric'
-                          else stages.split_workspace_bytes(n) if form == 'split' else 0, dev)
+def _stage1_workspace(n, dev, form, nbytes=None):
+    """A workspace of the stage-1 form for n, of ``nbytes`` if given.  How the symmetric form
+    divides its sums depends on the size it gets, which follows the free memory: a recomputed
+    step is the forward one bit for bit with as many bytes as that had."""
+    if nbytes is None:
+        form = _stage1_form(n, form)
+        nbytes = (stages.sym_workspace_size(n, device=dev) if form == 'symmetric'
+                  else stages.split_workspace_bytes(n) if form == 'split' else 0)
+    return stages.scratch(nbytes, dev)
 
 
 def _stage1(posm, acc, G, eps, form='auto', ws=None):
@@ -311,7 +315,8 @@ def _stage1(posm, acc, G, eps, form='auto', ws=None):
 def _step(posm, acc, r64, v64, G, eps, dt, form='auto', ws=None, out=None):
     """One time step: stage 1 in the form for n, then the FP64-master stage 2; the j-split
     form as one fused step (``stages.step_split_f64m``, the same bits).  Every forward and
-    recomputed step goes through here, so they agree bit for bit.  ``out``: the buffer of the
+    recomputed step goes through here, and with workspaces of one size they agree bit for bit.
+    ``out``: the buffer of the
     new positions (default: posm)."""
     if _stage1_form(posm.shape[0], form) == 'split':
         stages.step_split_f64m(posm, r64, v64, G, eps, dt, None, ws, out=out)
@@ -357,7 +362,7 @@ class _SegmentGraphs:
     recomputed step goes from one record slot to the next (no copy), and with the j-split VJP a
     backward step is chained (its reduce forms the next cotangent)."""
 
-    def __init__(self, n, dev, G, eps, dt, interval, form, records=2):
+    def __init__(self, n, dev, G, eps, dt, interval, form, records=2, ws_bytes=None):
         f32, f64 = torch.float32, torch.float64
         self.cfg = (G, eps, dt, interval, form)
         self.posm = torch.empty((n, 4), dtype=f32, device=dev)
@@ -371,7 +376,7 @@ class _SegmentGraphs:
         self.gamma = torch.empty((n,), dtype=f64, device=dev)
         self.mu4 = torch.empty((n, 4), dtype=f32, device=dev)
         self.eslot = torch.empty((2,), dtype=torch.int32, device=dev)
-        self.ws = _stage1_workspace(n, dev, form)
+        self.ws = _stage1_workspace(n, dev, form, ws_bytes)
         self.chain = CHAIN and _vjp_split(n, form)
         self.paired = (OVERLAP and self.chain and records == 2
                        and _stage1_form(n, form) == 'split')
@@ -490,11 +495,13 @@ class _SegmentGraphs:
 _SEGMENT_GRAPHS = collections.OrderedDict()
 
 
-def _segment_graphs(n, dev, G, eps, dt, interval, form):
+def _segment_graphs(n, dev, G, eps, dt, interval, form, ws_bytes=None):
+    """The kept _SegmentGraphs of a configuration, or a new one.  ``ws_bytes``: the stage-1
+    workspace of the forward pass whose backward pass this is for."""
     key = (dev, n, G, eps, dt, interval, form, CHAIN, OVERLAP)
     sg = _SEGMENT_GRAPHS.pop(key, None)
-    if sg is None:
-        sg = _SegmentGraphs(n, dev, G, eps, dt, interval, form, 2 if OVERLAP else 1)
+    if sg is None or ws_bytes not in (None, sg.ws.numel()):
+        sg = _SegmentGraphs(n, dev, G, eps, dt, interval, form, 2 if OVERLAP else 1, ws_bytes)
         while len(_SEGMENT_GRAPHS) >= 4:
             _SEGMENT_GRAPHS.popitem(last=False)
     _SEGMENT_GRAPHS[key] = sg
@@ -546,7 +553,7 @@ class _Single(torch.autograd.Function):
         sg = (_segment_graphs(n, dev, G, eps, dt, interval, form)
               if graph and not store else None)
         if sg is not None:
-            posm, acc, r64, v64 = sg.posm, sg.acc, sg.r64, sg.v64
+            posm, acc, r64, v64, ws = sg.posm, sg.acc, sg.r64, sg.v64, sg.ws
         else:
             ws = _stage1_workspace(n, dev, form)
             posm = torch.empty((n, 4), dtype=torch.float32, device=dev)
@@ -575,6 +582,7 @@ class _Single(torch.autograd.Function):
                     _step(posm, acc, r64, v64, G, eps, dt, form, ws)
             t += k
         ctx.cfg = (G, eps, dt, steps, interval, store, form, graph)
+        ctx.ws_bytes = ws.numel()
         ctx.traj = traj
         ctx.checkpoints = checkpoints
         ctx.mass = posm[:, 3] if store else posm[:, 3].clone()
@@ -586,11 +594,12 @@ class _Single(torch.autograd.Function):
         n = ctx.mass.shape[0]
         dev = ctx.mass.device
         if store:
-            sg = _SegmentGraphs(n, dev, G, eps, dt, 1, form, records=0)
+            sg = _SegmentGraphs(n, dev, G, eps, dt, 1, form, records=0, ws_bytes=0)
         elif not graph:
-            sg = _SegmentGraphs(n, dev, G, eps, dt, interval, form, 2 if OVERLAP else 1)
+            sg = _SegmentGraphs(n, dev, G, eps, dt, interval, form, 2 if OVERLAP else 1,
+                                ctx.ws_bytes)
         else:
-            sg = _segment_graphs(n, dev, G, eps, dt, interval, form)
+            sg = _segment_graphs(n, dev, G, eps, dt, interval, form, ctx.ws_bytes)
         sg.begin_backward(g_r, g_v)
         if store:
             sg.adjoint(steps, True, ctx.traj)

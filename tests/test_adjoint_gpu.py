@@ -896,3 +896,30 @@ def test_checkpointed_pass_of_every_form_recomputes_no_recorded_segment(cuda, fo
     for other in got[1:]:
         for x, y in zip(got[0], other):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize('graph', [False, True])
+def test_recomputation_uses_the_forward_passs_workspace_size(cuda, graph, monkeypatch):
+    # the symmetric form divides its sums by the size of its workspace, which is chosen by the
+    # free memory: with less free at the backward pass (and its kept graphs gone), the recomputed
+    # steps are still the forward ones and the gradients the recorded trajectory's, bit for bit
+    n = 20000
+    print('workspace of a recomputation', graph, flush=True)
+    assert stages.auto_form(n) == 'symmetric'
+    rng = np.random.default_rng(23)
+    r, v, w = (torch.from_numpy(rng.normal(size=(n, 3))).to(cuda) for _ in range(3))
+    m = torch.from_numpy(rng.uniform(0.5, 1.5, n) / n).to(cuda)
+    full = stages.sym_workspace_bytes(n)
+    kw = dict(G=1.0, eps=1e-2, dt=0.1)
+    got = []
+    for interval in (None, 2):
+        monkeypatch.setattr(adjoint, '_SEGMENT_GRAPHS', collections.OrderedDict())
+        sizes = [full]
+        monkeypatch.setattr(stages, 'sym_workspace_size',
+                            lambda *a, **k: sizes.pop() if sizes else 2 * full // 3 // 256 * 256)
+        leaves = [x.clone().requires_grad_(True) for x in (r, v, m)]
+        out = adjoint.trajectory(*leaves, 5, interval=interval, budget=1 << 30, graph=graph, **kw)
+        adjoint._SEGMENT_GRAPHS.clear()
+        got.append([x.detach() for x in out] + list(torch.autograd.grad(out, leaves, [w, w])))
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
