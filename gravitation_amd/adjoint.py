@@ -316,8 +316,7 @@ def _step(posm, acc, r64, v64, G, eps, dt, form='auto', ws=None, out=None):
     """One time step: stage 1 in the form for n, then the FP64-master stage 2; the j-split
     form as one fused step (``stages.step_split_f64m``, the same bits).  Every forward and
     recomputed step goes through here, and with workspaces of one size they agree bit for bit.
-    ``out``: the buffer of the
-    new positions (default: posm)."""
+    ``out``: the buffer of the new positions (default: posm)."""
     if _stage1_form(posm.shape[0], form) == 'split':
         stages.step_split_f64m(posm, r64, v64, G, eps, dt, None, ws, out=out)
     else:

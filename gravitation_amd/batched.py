@@ -247,6 +247,8 @@ class Engine:
         to another, through the record's slots or back and forth between posm and a buffer of
         the call's own.  A single step without a record, and steps into a record whose slots are
         no float32 position buffers of their own, run their two stages in place."""
+        if steps < 1:
+            return
         n = self.n
         for t, name, dtype, shape in ((posm, 'posm', torch.float32, (n, 4)),
                                       (r64, 'r64', torch.float64, (3, n)),
@@ -259,7 +261,7 @@ class Engine:
             if steps > 1:
                 other = torch.empty((n, 4), dtype=torch.float32, device=dev)
                 bufs = [posm, other] * (steps // 2) + [posm]
-        elif steps and _slots_of(traj, posm, steps, n):
+        elif _slots_of(traj, posm, steps, n):
             in_place = 0
             traj[0].copy_(posm)
             bufs = [traj[t] for t in range(steps)] + [posm]

@@ -424,3 +424,18 @@ def test_batched_mu_is_exact_at_the_register_limit(cuda, sizes):
         with np.errstate(over='ignore', invalid='ignore'):
             w = np.ldexp(want[:, a:b], -e).astype(np.float32).T
         assert np.array_equal(got[a:b, :3].numpy(), w, equal_nan=True)
+
+
+@pytest.mark.parametrize('mode', ['perstep', 'perstep-sym'])
+@pytest.mark.parametrize('steps', [0, -1, -2, -3])
+def test_no_steps_leave_the_state(cuda, mode, steps):
+    print('no steps', mode, steps, flush=True)
+    rng = np.random.default_rng(3)
+    r, v, m = rng.normal(size=(300, 3)), rng.normal(size=(300, 3)), rng.uniform(0.1, 1.0, 300)
+    b = batched.Batch(r, v, m, [0, 100, 300], config=(mode, 8, 1, 8, 0, 4))
+    traj = torch.full((2, 300, 4), 7.0, device=cuda)
+    before = [x.clone() for x in (b.posm, b.r64, b.v64, traj)]
+    b.step(steps)
+    b.engine.forward(b.posm, b.r64, b.v64, b.G, b.eps, b.dt, steps, traj)
+    for x, y in zip((b.posm, b.r64, b.v64, traj), before):
+        assert torch.equal(x, y)
