@@ -234,13 +234,12 @@ def _check_state(r0, v0, m):
 def _rows(*tensors):
     """Whether the kernels can read these (n, 3) or (n,) tensors as rows where they lie."""
     return all(t.is_contiguous() and t.dtype == torch.float64 and not t.is_neg()
-               and t.numel() > 0 for t in tensors)
+               and t.numel() > 0 and t.device == tensors[0].device for t in tensors)
 
 
 def _load_state(r0, v0, m, posm, r64, v64):
     """The state's buffers from r0, v0 (n, 3) and m (n,)."""
     if _rows(r0, v0, m):
-        stages.same_device(r0, v0, m, posm)
         with stages.on_device(posm):
             _native.call('grav_state_from_rows', r0.data_ptr(), v0.data_ptr(), m.data_ptr(),
                          posm.data_ptr(), r64.data_ptr(), v64.data_ptr(), r0.shape[0],

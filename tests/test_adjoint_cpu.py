@@ -2,6 +2,7 @@
 
 import numpy as np
 import pytest
+import torch
 
 from gravitation_amd import adjoint
 
@@ -28,3 +29,16 @@ def test_trajectory_form_is_checked_first():
     z = np.zeros((4, 3))
     with pytest.raises(ValueError, match='form'):
         adjoint.trajectory(z, z, np.ones(4), 3, form='split')
+
+
+def test_rows_are_read_in_place_on_one_device_only():
+    # a tensor on another device than the others is copied over by torch, not handed to a kernel
+    a = torch.zeros((4, 3), dtype=torch.float64)
+    other = torch.zeros((4,), dtype=torch.float64, device='meta')
+    assert adjoint._rows(a, a + 1, a[:, 0].contiguous())
+    assert not adjoint._rows(a, a + 1, other)
+    assert not adjoint._rows(a, a.t().contiguous().t())
+    assert not adjoint._rows(a.float())
+    assert not adjoint._rows(torch._neg_view(a))
+    assert not adjoint._rows(a[:0])
+    assert adjoint._rows()
