@@ -17,7 +17,12 @@ namespace grav {
 
 // Accumulates, for K owners per lane, the partials P += s (w - 3 (d.w)/q d) and
 // Pg += s (d . mu_j) of U j-bodies (q = x, y, z, m; u = mu_j; indices j + t), in the order of t.
-// PRIO: the rsq of the U * K pairs together at a raised wave priority (prio_up).
+// PRIO: the rsq of the U * K pairs together at a raised wave priority (prio_up).  Without it pair
+// by pair: in phases, two and four bodies per lane took 94 and 168 VGPRs instead of 59 and 126
+// and lost wavefronts.  MI355X, in phases and pair by pair: a quarter of the rows of 65536
+// bodies with (2, 8) 1787 and 1677 us, the j-split VJP of 16384 with (2, 4) in 4 ranges 234 and 225
+// us, of 65536 with (2, 2) in 8 ranges 3.36 and 3.12 ms.  (The other way round where the grid left
+// the wavefronts unused: 40000 with (2, 2) 1.22 and 1.39 ms.)
 template <int K, bool MASK, bool PRIO, int U>
 __device__ __forceinline__ void vjp_pairs(const float4 (&q)[U], const float4 (&u)[U],
                                           const int j, const float (&xk)[K],
@@ -26,6 +31,25 @@ __device__ __forceinline__ void vjp_pairs(const float4 (&q)[U], const float4 (&u
                                           const float (&uyk)[K], const float (&uzk)[K],
                                           const int (&kk)[K], const float eps2, float (&px)[K],
                                           float (&py)[K], float (&pz)[K], float (&pg)[K]) {
+  if constexpr (!PRIO && (U > 1 || K > 1)) {
+#pragma unroll
+    for (int t = 0; t < U; ++t)
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const float4 q1[1] = {q[t]}, u1[1] = {u[t]};
+        const float x1[1] = {xk[k]}, y1[1] = {yk[k]}, z1[1] = {zk[k]}, m1[1] = {mk[k]};
+        const float ux1[1] = {uxk[k]}, uy1[1] = {uyk[k]}, uz1[1] = {uzk[k]};
+        const int k1[1] = {kk[k]};
+        float sx[1] = {px[k]}, sy[1] = {py[k]}, sz[1] = {pz[k]}, sg[1] = {pg[k]};
+        vjp_pairs<1, MASK, false>(q1, u1, j + t, x1, y1, z1, m1, ux1, uy1, uz1, k1, eps2, sx, sy,
+                                  sz, sg);
+        px[k] = sx[0];
+        py[k] = sy[0];
+        pz[k] = sz[0];
+        pg[k] = sg[0];
+      }
+    return;
+  }
   float dx[U][K], dy[U][K], dz[U][K], iv[U][K];
 #pragma unroll
   for (int t = 0; t < U; ++t)
