@@ -30,7 +30,9 @@ def _kernels():
 
 
 @pytest.mark.parametrize('name, bodies, limit', [('k_stage1_vjp_f32', 2, 64),
-                                                 ('k_stage1_vjp_f32', 4, 128)])
+                                                 ('k_stage1_vjp_f32', 4, 128),
+                                                 ('k_step_items_f64m', 2, 64),
+                                                 ('k_step_items_f64m', 4, 128)])
 def test_pair_kernels_keep_their_wavefronts(name, bodies, limit):
     of = {k: v for k, v in _kernels().items() if re.search(r'%sILi%dE' % (name, bodies), k)}
     assert of and max(of.values()) <= limit, of
