@@ -688,7 +688,7 @@ int launch_vjp(const float4 *posm, const float4 *mu4, double *rho, double *gamma
   const size_t lds = (S > 1) ? sizeof(float) * (S - 1) * 8 * per_block : 0;
   if (grid == 0) return GRAV_OK;
   if constexpr (K == 1) {
-    if (items != nullptr && nitems <= kHalvesVjpItems && halves_of(max_bodies, S)) {
+    if (items != nullptr && int64_t(nitems) * S <= kHalvesVjpWaves && halves_of(max_bodies, S)) {
       const int slots = half_slots(max_bodies, S);
       hipLaunchKernelGGL((k_stage1_vjp_f32<K, S, 2>), dim3(grid), dim3(2 * kWave * S),
                          lds + sizeof(float) * S * slots * 4 * kWave, stream, posm, mu4, rho,

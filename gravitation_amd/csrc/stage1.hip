@@ -233,7 +233,7 @@ int launch_step_items(const float4 *posm, int n, float G, float eps2, int mask,
   const size_t lds = (S > 1) ? sizeof(float) * (S - 1) * 6 * kWave * K : 0;
   constexpr int kNarrow = K >= 4 ? 8 : K == 1 ? 4 : 2;   // pair_loop_width's other value
   if constexpr (K == 1) {
-    if (nitems <= kHalvesStepItems && halves_of(max_bodies, S)) {
+    if (int64_t(nitems) * S <= kHalvesStepWaves && halves_of(max_bodies, S)) {
       const int slots = half_slots(max_bodies, S);
       const size_t more = sizeof(float) * S * slots * 3 * kWave;
       if (pair_loop_width(nitems, K, false) == 8)

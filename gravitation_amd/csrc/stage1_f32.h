@@ -183,13 +183,15 @@ __device__ __forceinline__ void sum_segment_f32(const float4 *__restrict__ posm,
 // A wavefront whose counterpart has one block or none ends at once.  Taken where there is a
 // second block (up to 1024 j-bodies per wavefront, for the sums' LDS) and the launch is
 // small: with wavefronts enough on every SIMD the second set gives nothing and costs its
-// workgroups' slots.  MI355X, without and with, forward and backward over 8 or 12 steps:
-// 30 universes of 64-2048 bodies (289 items) 0.728 and 0.501 ms, 60 of 32-1500 (392) 0.575
-// and 0.464, 100 of 100-1200 (743) 0.499 and 0.453, 128 of 64-2048 (1219) 1.131 and 1.090, 200
-// of 100-1200 (1482) 0.570 and 0.592; forward alone over 10 steps: 200 of 32-2048 (1619)
-// 0.366 and 0.332, 400 (3227) 0.550 and 0.572; over 20 steps 10 of 64-2048 (102) 0.631 and 0.370.
-constexpr int kHalvesStepItems = 2048;   // largest launches in halves, of steps
-constexpr int kHalvesVjpItems = 1280;    // and of VJPs
+// workgroups' slots.  So the limits count the first set's wavefronts, items times j_waves, on 1024
+// SIMDs: six for steps, four for VJPs, whose workgroups hold more registers and LDS.  MI355X,
+// eight launches without and with, us (wavefronts; universes of 64-2048 and 300-1000 bodies).
+// Steps, one j-wave: 957 501 and 306, 2874 554 and 388, 6702 769 and 788; two: 3794 545 and 399,
+// 5306 568 and 501, 7580 686 and 673; four: 4720 297 and 268, 7588 339 and 346, 10612 456 and 472.
+// VJPs, one: 957 563 and 377, 2874 786 and 793; two: 1914 312 and 342, 2476 623 and 510, 3794 788
+// and 735, 5748 688 and 750; four: 2360 320 and 275, 4720 474 and 512, 4952 442 and 486.
+constexpr int kHalvesStepWaves = 6144;   // largest launches in halves, of steps
+constexpr int kHalvesVjpWaves = 4096;    // and of VJPs
 constexpr int kHalvesChunk = 1024;
 
 // Whether the longest j-range of a wavefront has a second block and at most kHalvesChunk bodies.

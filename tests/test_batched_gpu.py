@@ -439,3 +439,32 @@ def test_no_steps_leave_the_state(cuda, mode, steps):
     b.engine.forward(b.posm, b.r64, b.v64, b.G, b.eps, b.dt, steps, traj)
     for x, y in zip((b.posm, b.r64, b.v64, traj), before):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize('jw', [1, 2, 4])
+@pytest.mark.parametrize('waves', [4096, 6144])
+def test_perstep_at_the_limits_of_the_halves_is_bitwise_equal(cuda, jw, waves):
+    # a second set of wavefronts up to a number of wavefronts of the launch, items times j_waves:
+    # the same bits of a universe in launches of a few, of exactly that many and of one item more
+    from gravitation_amd import adjoint
+    print('halves limit', jw, waves, flush=True)
+    sizes = [300 * jw, 1000 * jw]
+    big = sum(-(-s // 64) for s in sizes)
+    n = sum(sizes)
+    out = []
+    for extra in (0, waves // jw - big, waves // jw - big + 1):
+        off = np.concatenate([[0], np.cumsum(sizes + [2] * extra)])
+        total = int(off[-1])
+        rng = np.random.default_rng(jw)
+        one = [rng.normal(size=(n, 3)), rng.normal(size=(n, 3)), rng.uniform(0.1, 1.0, n) / n,
+               rng.normal(size=(n, 3))]
+        r, v, m, w = [np.concatenate([x, rng.normal(size=(total - n,) + x.shape[1:])])
+                      for x in one]
+        eng = batched.Engine(off, ('perstep', 8, 1, 8, 0, jw), cuda)
+        leaves = [torch.from_numpy(x).to(cuda).requires_grad_(True) for x in (r, v, np.abs(m))]
+        r1, v1 = adjoint.batched_trajectory(eng, *leaves, 2, G=1.0, eps=1e-2, dt=1e-3)
+        ((r1 + v1) * torch.from_numpy(w).to(cuda)).sum().backward()
+        out.append([x[:n].clone() for x in (r1.detach(), v1.detach(), *[y.grad for y in leaves])])
+    for other in out[1:]:
+        for x, y in zip(out[0], other):
+            assert torch.equal(x, y)
