@@ -65,8 +65,9 @@ def tune_stage1(posm, G=1.0, eps=1e-3, candidates=None, reps=3):
     return best, table
 
 
-SYM_CANDIDATES = [None, (4, 2), (4, 4), (8, 2), (8, 4)]
-SYM_F64_CANDIDATES = [None, (2, 2), (2, 4), (4, 2), (4, 4)]
+# with the library's own shape at any size among them, so no None beside them
+SYM_CANDIDATES = [(4, 2), (4, 4), (8, 2), (8, 4)]
+SYM_F64_CANDIDATES = [(2, 2), (2, 4), (4, 2), (4, 4)]
 OWNER_FORM_CANDIDATES = [(1, 8, 256), (2, 8, 256), (2, 16, 256), (4, 4, 256), (8, 2, 256)]
 SPLIT_CANDIDATES = [(1, 8, 4), (1, 8, 8), (1, 4, 8), (2, 8, 8), (2, 8, 16), (1, 8, 16)]
 SPLIT_F64_CANDIDATES = [(1, 8, 16), (1, 8, 32), (2, 8, 16), (1, 4, 32)]

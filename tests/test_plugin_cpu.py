@@ -127,3 +127,11 @@ def test_bench_refuses_more_than_one_gpu():
                        cwd=root, capture_output=True, text=True, timeout=120)
     assert p.returncode != 0
     assert 'one GPU' in p.stderr
+
+
+def test_tuner_times_every_symmetric_shape_once():
+    # None stands for one of the shapes below at every size: naming both times one kernel twice
+    from gravitation_amd import tune
+    for shapes, own in ((tune.SYM_CANDIDATES, {(4, 2), (8, 2)}),
+                        (tune.SYM_F64_CANDIDATES, {(2, 2), (4, 2), (4, 4)})):
+        assert None not in shapes and own <= set(shapes) and len(set(shapes)) == len(shapes)
