@@ -6,9 +6,10 @@
 // With rho = dL/dr', nu = dL/dv' and mu = nu + h rho, one backward step is
 //   rho <- rho + h J_r^T mu,   gamma <- gamma + h J_m^T mu,   nu <- mu
 // (gamma = dL/dm).  grav_adjoint_mu does the element-wise part (mu, nu, and an FP32 copy of
-// mu scaled per universe by a power of two); grav_stage1_vjp_f32 the all-pairs part, owner-computes like stage 1: lane l owns K bodies, j-bodies (x,y,z,m)
-// and mu_j are wave-uniform loads (SMEM), S wavefronts split the j-range, FP32 pair terms with
-// blocked TwoSum partials, FP64 adjoint state.
+// mu scaled per universe by a power of two); grav_stage1_vjp_f32 the all-pairs part,
+// owner-computes like stage 1: lane l owns K bodies, j-bodies (x,y,z,m) and mu_j are wave-uniform
+// loads (SMEM), S wavefronts split the j-range, FP32 pair terms with blocked TwoSum partials, FP64
+// adjoint state.
 #include <algorithm>
 #include <cfloat>
 #include <climits>
@@ -810,8 +811,8 @@ int launch_backward_pair(const float4 *pa, float4 *mu4, double *rho, double *nu,
   if (rc != GRAV_OK) return rc;
   const int nb = (n + kReduceBodies - 1) / kReduceBodies;
   hipLaunchKernelGGL(k_backward_pair_reduce, dim3(2 * nb), dim3(4 * kReduceBodies), 0, stream,
-                     part_a, mu4, rho, nu, gamma, splits_a, hG, eslot, part_r, pr, pr_out, r64, v64, splits_r,
-                     G, dt, n, nb);
+                     part_a, mu4, rho, nu, gamma, splits_a, hG, eslot, part_r, pr, pr_out, r64,
+                     v64, splits_r, G, dt, n, nb);
   return check_launch("k_backward_pair_reduce");
 }
 }  // namespace

@@ -21,7 +21,7 @@
 //     a fold kernel adds its partials into each body's FP64 sum in a fixed order, so the
 //     workspace is bounded (one slab down to one row) and the result is deterministic;
 //   * one universe of middle size (sizes at kUnitsFrom) has the work of all rows, the pairs inside
-//     the blocks among it, divided evenly among workgroups that are resident at once;
+//     the blocks among it, divided evenly among a number of workgroups (kUnitGroups);
 //   * batched universes list their block pairs as items, and one reduction kernel adds every
 //     body's diagonal-block sum and partials in a fixed order in FP64.
 #include <algorithm>
@@ -69,8 +69,8 @@ __device__ __forceinline__ float4 load_or_far(const float4 *__restrict__ posm, i
 // needs no negating (8-byte) FMA.  Adding the step's j-side sum in the move itself leaves the time
 // as it was (2^18 11.36 against 11.43 ms on one box) and about halves the error against 64 bits
 // (Plummer, eps 1e-3: 20000 bodies 1.5e-7 to 7e-8, 65536 9.3e-8 to 5.7e-8).  MI355X, (8, 2),
-// before and after: 2^18 bodies 13.40 and 11.13 ms (59 to 49 cycles per pair and SIMD), 2^17 3.44 and 2.87 ms; (4, 2) at
-// 49999 bodies 0.652 and 0.496 ms.  G = 4 pairs need 138 VGPRs with K = 8 for 11.05 ms, G = 1
+// before and after: 2^18 bodies 13.40 and 11.13 ms (59 to 49 cycles per pair and SIMD), 2^17 3.44
+// and 2.87 ms; (4, 2) at 49999 bodies 0.652 and 0.496 ms.  G = 4 pairs need 138 VGPRs with K = 8 for 11.05 ms, G = 1
 // takes 11.19 ms.  Measured and not kept: the j-bodies read from LDS instead of rotated (3 DPP
 // moves per step instead of 7) is no faster once the moves have priority (2.95 against 2.86 ms
 // at 2^17), and temporaries pinned to registers of alternating parity (an FMA whose three
@@ -79,8 +79,8 @@ __device__ __forceinline__ float4 load_or_far(const float4 *__restrict__ posm, i
 //
 // WIDE: the weights are (m/r) (1/r^2), as in the owner-computes and j-split forms, and hold for
 // every r whose square is an FP32 number (1e-19 to 1e19).  Otherwise both bodies share 1/r^3,
-// one multiplication less per pair (5 % of the time: 32768 bodies 240 against 253 us, 65536 846
-// against 886), which overflows below r = 1.4e-13 and loses its bits above 4.4e12.
+// one multiplication less per pair (5 % of the time: 32768 bodies 221 against 235 us, 49999 465
+// against 489), which overflows below r = 1.4e-13 and loses its bits above 4.4e12.
 template <int K, bool OWN, bool PRIO = true, bool WIDE = false>
 __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const float eps2,
                                           const float (&xi)[K], const float (&yi)[K],
@@ -149,10 +149,11 @@ __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const
 
 // One block pair (beta, gamma) for one workgroup: its wavefronts hold K block-beta bodies per
 // lane (xi..zi, the masses negated in mn) and take the K*W chunks of 64 block-gamma bodies from
-// jb0 (bodies at or past jend load as far, massless padding).  The i-side sums of every chunk fold into the TwoSum
-// pairs (hx, lx) .. (hz, lz), which the caller may carry over several gamma blocks; the j-side
-// sums of a chunk, added over the W wavefronts through the double-buffered LDS `red` (buffer
-// chunk & 1, chunk counting on across calls), go to pj[c * IB + jc * 64 + l], 3 * IB floats.
+// jb0 (bodies at or past jend load as far, massless padding).  The i-side sums of every chunk
+// fold into the TwoSum pairs (hx, lx) .. (hz, lz), which the caller may carry over several gamma
+// blocks; the j-side sums of a chunk, added over the W wavefronts through the double-buffered LDS
+// `red` (buffer chunk & 1, chunk counting on across calls), go to pj[c * IB + jc * 64 + l],
+// 3 * IB floats.
 template <int K, int W, bool PRIO>
 __device__ __forceinline__ void sym_block_pair(const float4 *__restrict__ posm, int jb0,
                                                int jend, float eps2, const float (&xi)[K],
@@ -459,17 +460,18 @@ __global__ __launch_bounds__(kWave *W) void k_sym_segments_f64(const double4 *__
 }
 
 // ---------------------------------------------------------------------------------------------
-// One universe, balanced form.  The work of row beta is a list of units: the 64-body chunks
-// c = beta*K*W .. nc-1 (nc chunks in all), first the K*W chunks of block beta itself (i side
-// only: every ordered pair of the block once) and then those of the later blocks (both sides).
-// The units of all rows, numbered row-major, are divided evenly among `groups` workgroups, all
-// resident at once: group g takes units [g*U/groups, (g+1)*U/groups).  It keeps the i-side sums
-// of a row in registers while it stays in that row and writes them once, to slot g + beta of
-// p_i (3*IB values; g + beta is unique to the pair); the j-side sums of a unit go to p_j at block
-// pair (beta, gamma) as in the row-segment form.  A fold kernel adds every body's partials in
-// FP64 in a fixed order.
+// One universe, balanced form, in blocks of 64*K*W bodies with (K, W) = (kUnitK, kUnitW).  The
+// work of row beta is a list of units: the 64-body chunks c = beta*K*W .. nc-1 (nc chunks in all),
+// first the K*W chunks of block beta itself (i side only: every ordered pair of the block once)
+// and then those of the later blocks (both sides).  The units of all rows, numbered row-major,
+// are divided evenly among `groups` workgroups: group g takes units [g*U/groups, (g+1)*U/groups).
+// It keeps the i-side sums of a row in registers while it stays in that row and writes them once,
+// to slot g + beta of p_i (3*IB values; g + beta is unique to the pair); the j-side sums of a unit
+// go to p_j at block pair (beta, gamma) as in the row-segment form.  A fold kernel adds every
+// body's partials in FP64 in a fixed order.
 
-constexpr int kCus = 256;   // compute units of an MI355X
+constexpr int kUnitK = 4, kUnitW = 4;
+constexpr int kCus = 256;   // compute units of an MI355X; another number costs balance only
 
 // First unit of row beta; a row's units end where the next row's begin.
 __host__ __device__ inline int64_t unit_row(int64_t beta, int64_t nc, int kw) {
@@ -545,23 +547,23 @@ constexpr T kMassSign = sizeof(T) == 4 ? T(-1) : T(1);
 
 // Bound by VALU issue (sym_chunk).  Against the row segments: no block-diagonal pass of its own
 // (FP64, 40000 bodies: 23 of 690 us), no last round of workgroups that leaves half the compute
-// units idle, i-side partials once per group and row.  FP32 65536 bodies: 744 us = 55 cycles per
-// unordered pair and SIMD, of 50 that the loop can reach; 32768: 200 us, 59 cycles.
-template <typename T, typename T4, int K, int W, bool WIDE>
-__global__ __launch_bounds__(kWave *W) void k_sym_units(const T4 *__restrict__ posm, int n,
-                                                         int nb, int nc, int64_t units, T eps2,
-                                                         T *__restrict__ p_i,
-                                                         T *__restrict__ p_j) {
-  constexpr int KW = K * W, IB = kWave * KW;
+// units idle, i-side partials once per group and row.  FP32 65536 bodies: 767 us = 57 cycles per
+// unordered pair and SIMD, of 50 that the loop can reach; 32768 with WIDE: 235 us, 69 cycles,
+// of 53 (its workspace holds five groups per compute unit).
+template <typename T, typename T4, bool WIDE>
+__global__ __launch_bounds__(kWave *kUnitW) void k_sym_units(const T4 *__restrict__ posm, int n,
+                                                              int nb, int nc, int64_t units,
+                                                              T eps2, T *__restrict__ p_i,
+                                                              T *__restrict__ p_j) {
+  constexpr int K = kUnitK, W = kUnitW, KW = K * W, IB = kWave * KW;
   __shared__ T red[2][W][3][kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  // workgroups b, b + kCus, b + 2*kCus, .. go to one compute unit: they take neighbouring ranges, so
-  // that the units of a compute unit differ by at most one
+  // The workgroups that are resident first go to the compute units in turn, b, b + kCus, .. to
+  // one: they take neighbouring ranges, so that the compute units start with equal work.  groups
+  // is a multiple of kCus (unit_plan).
   const int64_t groups = gridDim.x;
-  const int64_t g = groups % kCus == 0
-                        ? int64_t(blockIdx.x % kCus) * (groups / kCus) + blockIdx.x / kCus
-                        : blockIdx.x;
+  const int64_t g = int64_t(blockIdx.x % kCus) * (groups / kCus) + blockIdx.x / kCus;
   int64_t u = g * units / groups;
   const int64_t u_end = (g + 1) * units / groups;
   int beta = 0;
@@ -611,24 +613,19 @@ __global__ __launch_bounds__(kWave *W) void k_sym_units(const T4 *__restrict__ p
       const int gamma = c / KW;
       T *pj = p_j + (pair_row(beta, nb) + (gamma - beta - 1)) * (3 * IB) +
               (c - gamma * KW) * kWave;
-      if constexpr (W == 1) {
+      // two buffers: a wave writes one again only after the other's barrier, which every wave
+      // reaches after it has read this one
+      T(*r)[3][kWave] = red[buf];
+      buf ^= 1;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) pj[q * IB + lane] = aj[q];
-      } else {
-        // two buffers: a wave writes one again only after the other's barrier, which every
-        // wave reaches after it has read this one
-        T(*r)[3][kWave] = red[buf];
-        buf ^= 1;
+      for (int q = 0; q < 3; ++q) r[wave][q][lane] = aj[q];
+      __syncthreads();
+      for (int t = threadIdx.x; t < 3 * kWave; t += kWave * W) {
+        const int q = t / kWave, l = t % kWave;
+        T v = 0;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) r[wave][q][lane] = aj[q];
-        __syncthreads();
-        for (int t = threadIdx.x; t < 3 * kWave; t += kWave * W) {
-          const int q = t / kWave, l = t % kWave;
-          T v = 0;
-#pragma unroll
-          for (int w = 0; w < W; ++w) v += r[w][q][l];
-          pj[q * IB + l] = v;
-        }
+        for (int w = 0; w < W; ++w) v += r[w][q][l];
+        pj[q * IB + l] = v;
       }
     }
     T *out = p_i + (g + beta) * (3 * IB) + wave * (K * kWave) + lane;
@@ -640,14 +637,15 @@ __global__ __launch_bounds__(kWave *W) void k_sym_units(const T4 *__restrict__ p
 }
 
 // acc = G * (every partial of the body) of the balanced form, or with `sums` the unscaled FP64
-// sum itself, for the 64 bodies of chunk blockIdx.x: 3 * 64 (component, body) columns in kFoldSlices slices of the body's partials
-// (its row's i-side slots, then its j-side partials from the rows before), each slice added in
-// order in FP64, the slices' sums in order.  A wave keeps eight coalesced reads in flight.
+// sum itself, for the 64 bodies of chunk blockIdx.x: 3 * 64 (component, body) columns in
+// kFoldSlices slices of the body's partials (its row's i-side slots, then its j-side partials
+// from the rows before), each slice added in order in FP64, the slices' sums in order.  A wave keeps eight coalesced reads in flight.
 constexpr int kFoldSlices = 4;
 template <typename T>
 __global__ __launch_bounds__(3 * kWave *kFoldSlices) void k_sym_units_fold(
     T *__restrict__ acc, double *__restrict__ sums, const T *__restrict__ p_i,
-    const T *__restrict__ p_j, int n, int nb, int nc, int kw, int64_t units, int64_t groups, double G) {
+    const T *__restrict__ p_j, int n, int nb, int nc, int kw, int64_t units, int64_t groups,
+    double G) {
   __shared__ double part[kFoldSlices][3 * kWave];
   const int ib = kw * kWave;
   const size_t stride = static_cast<size_t>(3) * ib;
@@ -960,7 +958,7 @@ int sym_run(const SymPlan &P, const SymRange &R, int n, T *acc, double *sums, do
   return GRAV_OK;
 }
 
-// The balanced form of n bodies in blocks of 64*K*W: `groups` workgroups of W wavefronts.
+// The balanced form of n bodies: `groups` workgroups of kUnitW wavefronts.
 struct UnitPlan {
   int nb, nc, kw;
   int64_t units, groups, j_bytes;
@@ -972,15 +970,16 @@ struct UnitPlan {
 // 291; 65536 773, 762, 744, 746; 100000 1788, 1773, 1696, 1690.
 constexpr int64_t kUnitGroups = 10 * kCus;
 
-// Where the default shape (named or as (0, 0)) takes the balanced form, in blocks of 1024 bodies
-// (K 4, W 4) whatever that shape is, if its workspace holds it.  Below, only one group per compute unit fits the workspace (FP32
-// 18500 bodies: 128 us against 124 for the row segments); above, a static division into few
-// thousand groups loses to the row segments, whose workgroups are dispatched as they end.
+// Where the default shape (named or as (0, 0), bit for bit the same call) takes the balanced form,
+// in blocks of 1024 bodies whatever that shape is, if its workspace holds it.  Below, only one
+// group per compute unit fits the workspace (FP32 18500 bodies: 128 us against 124 for the row
+// segments); above, a static division into few thousand groups loses to the row segments, whose
+// workgroups are dispatched as they end.
 // Stage 1, us, row segments in their default shape and this form (in parentheses the j-split
-// form): FP32 19000 bodies 124 and 81 (92), 20480 124 and 92 (104), 32768 221 and 200 (251), 49999
-// 479 and 450 (577), 65536 922 and 744 (971), 100000 1795 and 1709, 114687 2297 and 2237, 131072
-// 2854 and 2862; FP64 9000 74 and 50 (52), 12288 100 and 77 (88), 20000 202 and 168 (227), 40000
-// 690 and 592 (876), 60000 1332 and 1297.
+// form): FP32 19000 bodies 125 and 90 (95), 20480 126 and 100 (107), 32768 241 and 235 (257), 49999
+// 496 and 489 (584), 60000 789 and 700 (836), 65536 932 and 767 (984), 100000 1851 and 1760, 114687
+// 2365 and 2291, 131072 2854 and 2862; FP64 9000 75 and 52 (54), 12288 101 and 78 (92), 20000 207
+// and 184 (236), 40000 711 and 619 (920), 60000 1410 and 1365.
 constexpr int64_t kUnitsFrom = 18945, kUnitsTo = 114688;
 // FP32 sizes whose weights are WIDE (sym_chunk).  Below this size the form stands beside the
 // j-split form, whose range of distances it has to have, and is faster than it with the wider
@@ -990,9 +989,9 @@ constexpr int64_t kUnitsFromF64 = 8961, kUnitsToF64 = 65536;
 
 // groups: kUnitGroups, or the multiple of kCus below it whose i-side slots fit the workspace;
 // 0: the form does not fit.
-UnitPlan unit_plan(int64_t n, int K, int W, int64_t elem, int64_t workspace_bytes) {
+UnitPlan unit_plan(int64_t n, int64_t elem, int64_t workspace_bytes) {
   UnitPlan P{};
-  P.kw = K * W;
+  P.kw = kUnitK * kUnitW;
   const int64_t ib = int64_t(kWave) * P.kw, slot = 3 * ib * elem;
   P.nb = static_cast<int>((n + ib - 1) / ib);
   P.nc = static_cast<int>((n + kWave - 1) / kWave);
@@ -1004,15 +1003,15 @@ UnitPlan unit_plan(int64_t n, int K, int W, int64_t elem, int64_t workspace_byte
   return P;
 }
 
-template <typename T, typename T4, int K, int W>
+template <typename T, typename T4>
 int sym_units_run(const T4 *posm, T *acc, double *sums, int n, const UnitPlan &P, double G,
                   T eps2, void *ws, hipStream_t s) {
   T *p_j = static_cast<T *>(ws);
   T *p_i = reinterpret_cast<T *>(static_cast<char *>(ws) + P.j_bytes);
   auto launch = [&](auto wide) {
-    hipLaunchKernelGGL((k_sym_units<T, T4, K, W, decltype(wide)::value>),
-                       dim3(static_cast<unsigned>(P.groups)), dim3(kWave * W), 0, s, posm, n, P.nb,
-                       P.nc, P.units, eps2, p_i, p_j);
+    hipLaunchKernelGGL((k_sym_units<T, T4, decltype(wide)::value>),
+                       dim3(static_cast<unsigned>(P.groups)), dim3(kWave * kUnitW), 0, s, posm, n,
+                       P.nb, P.nc, P.units, eps2, p_i, p_j);
   };
   if (sizeof(T) == 4 && n < kUnitsWideTo)
     launch(std::integral_constant<bool, sizeof(T) == 4>());
@@ -1086,10 +1085,10 @@ bool sym_supported(int K, int W) {
   return (K == 4 || K == 8) && (W == 2 || W == 4);
 }
 
-// (0, 0) selects the shape by n, from MI355X measurements on Plummer spheres: blocks of 512
-// (K 4, W 2) below 57344 bodies, where blocks of 1024 leave too few block pairs to fill 256
-// CUs (at 49152 bodies (4, 2) takes 0.60 ms against 0.77), and blocks of 1024 (K 8, W 2)
-// above (1.27x over owner-computes at 2^18 in its own default shape, (1, 16)).
+// (0, 0) selects the shape by n, from MI355X measurements of the row segments on Plummer spheres:
+// blocks of 512 (K 4, W 2) below 57344 bodies, where blocks of 1024 leave too few block pairs to
+// fill 256 CUs, and blocks of 1024 (K 8, W 2) above.  Between kUnitsFrom and kUnitsTo this is
+// also the workspace that is asked for, and the shape that its segments have in a smaller one.
 void sym_shape(int64_t n, int &K, int &W) {
   if (K == 0 && W == 0) {
     K = n < 57344 ? 4 : 8;
@@ -1269,10 +1268,10 @@ int grav_stage1_sym_f32(const void *posm, void *acc, int64_t n, double G, double
   hipStream_t s = static_cast<hipStream_t>(stream);
   const float4 *p = static_cast<const float4 *>(posm);
   if (sym_units_shape(n, K, W)) {
-    const UnitPlan U = unit_plan(n, 4, 4, 4, workspace_bytes);
+    const UnitPlan U = unit_plan(n, 4, workspace_bytes);
     if (U.groups > 0)
-      return sym_units_run<float, float4, 4, 4>(p, static_cast<float *>(acc), nullptr, nn, U, G,
-                                                eps2, workspace, s);
+      return sym_units_run<float, float4>(p, static_cast<float *>(acc), nullptr, nn, U, G, eps2,
+                                          workspace, s);
   }
   // pairs inside each block: owner-computes over the blocks of IB bodies (a multiple of 256)
   auto diag_fn = [&](float *diag) {
@@ -1340,10 +1339,10 @@ int grav_stage1_sym_f32_share(const void *posm, void *sums64, int64_t n, double 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const float4 *p = static_cast<const float4 *>(posm);
   if (shares == 1 && sym_units_shape(n, K, W)) {   // the one-GPU form
-    const UnitPlan U = unit_plan(n, 4, 4, 4, workspace_bytes);
+    const UnitPlan U = unit_plan(n, 4, workspace_bytes);
     if (U.groups > 0)
-      return sym_units_run<float, float4, 4, 4>(p, nullptr, static_cast<double *>(sums64), nn, U,
-                                                1.0, eps2, workspace, s);
+      return sym_units_run<float, float4>(p, nullptr, static_cast<double *>(sums64), nn, U, 1.0,
+                                          eps2, workspace, s);
   }
   const int i0 = R.d_lo * P.ib;
   const int m = std::min(nn, R.d_hi * P.ib) - i0;
@@ -1411,10 +1410,10 @@ int grav_stage1_sym_f64(const void *posm64, void *acc64, int64_t n, double G, do
   hipStream_t s = static_cast<hipStream_t>(stream);
   const double4 *p = static_cast<const double4 *>(posm64);
   if (sym_units_shape_f64(n, K, W)) {
-    const UnitPlan U = unit_plan(n, 4, 4, 8, workspace_bytes);
+    const UnitPlan U = unit_plan(n, 8, workspace_bytes);
     if (U.groups > 0)
-      return sym_units_run<double, double4, 4, 4>(p, static_cast<double *>(acc64), nullptr, nn,
-                                                  U, G, eps2, workspace, s);
+      return sym_units_run<double, double4>(p, static_cast<double *>(acc64), nullptr, nn, U, G,
+                                            eps2, workspace, s);
   }
   auto diag_fn = [&](double *diag) {
     return stage1_f64_launch(p, diag, nn, 1.0, eps2, mask, P.ib, s);

@@ -57,10 +57,6 @@ def _stream(t):
     return current_stream(t.device)
 
 
-def ctypes_stream(s):
-    return s.cuda_stream
-
-
 def _check(t, name, dtype, shape):
     if not isinstance(t, torch.Tensor):
         raise TypeError('%s must be a torch.Tensor' % name)
@@ -113,13 +109,13 @@ def stage1_f32(posm, acc, G, eps=0.0, accum='kahan', cfg=None):
 # 13.4; with the host views refreshed, where the wait hides the launches, 512 21.3 and 21.4, 1000
 # 25.4 and 22.2, 2000 32.9 and 22.4).  The j-split form beats the symmetric one below 19456,
 # where few groups of its balanced form fit its workspace (stage 1, Plummer, us, j-split against
-# symmetric: 17000 76 against 114, 18500 92 against 128, 19456 95 against 82, 24576 146 against
-# 132, 32768 251 against 200, 49999 577 against 450).  FP64: j-split from 448 bodies (a hip1 step
+# symmetric: 17000 84 against 128, 18500 96 against 126, 19456 97 against 89, 24576 149 against
+# 142, 32768 257 against 235, 49999 584 against 489).  FP64: j-split from 448 bodies (a hip1 step
 # of the galaxy, us, owner-computes against j-split, on the device and with the host views
 # refreshed: 384 12.0 and 13.3, 25.1 and 22.5; 448 14.0 and 13.2, 26.3 and 22.4; 640 17.0 and
 # 13.3, 30.7 and 22.7; 1000 26.0 and 13.2, 38.3 and 23.5), symmetric from 10500 (us, j-split
-# against symmetric: 9000 52 against 50, 10000 62 against 63, 10500 70 against 64, 12288 88
-# against 77, 16384 151 against 119, 40000 876 against 591).
+# against symmetric: 9000 54 against 52, 10000 65 against 65, 10500 73 against 65, 12288 92
+# against 78, 16384 157 against 122, 40000 921 against 619).
 SPLIT_FROM = 1088
 SYMMETRIC_FROM = 19456
 SPLIT_F64_FROM = 448
