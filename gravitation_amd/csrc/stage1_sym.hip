@@ -25,7 +25,6 @@
 //   * batched universes list their block pairs as items, and one reduction kernel adds every
 //     body's diagonal-block sum and partials in a fixed order in FP64.
 #include <algorithm>
-#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -80,7 +79,9 @@ __device__ __forceinline__ float4 load_or_far(const float4 *__restrict__ posm, i
 // WIDE: the weights are (m/r) (1/r^2), as in the owner-computes and j-split forms, and hold for
 // every r whose square is an FP32 number (1e-19 to 1e19).  Otherwise both bodies share 1/r^3,
 // one multiplication less per pair (5 % of the time: 32768 bodies 221 against 235 us, 49999 465
-// against 489), which overflows below r = 1.4e-13 and loses its bits above 4.4e12.
+// against 489), which overflows below r = 1.4e-13 and loses its bits above 4.4e12.  The balanced
+// form looks at the coordinates of each chunk and takes the one or the other (Ordinary, 1 % of
+// the time); row segments and batches always share 1/r^3.
 template <int K, bool OWN, bool PRIO = true, bool WIDE = false>
 __device__ __forceinline__ void sym_chunk(const float4 q, const int kself, const float eps2,
                                           const float (&xi)[K], const float (&yi)[K],
@@ -487,10 +488,10 @@ __host__ __device__ inline int64_t pair_row(int64_t beta, int64_t nb) {
 }
 
 // The i-side sums of K bodies per lane: FP32 chunk sums folded into TwoSum pairs, FP64 as is.
-template <typename T, int K, bool WIDE>
+template <typename T, int K>
 struct ISum;
-template <int K, bool WIDE>
-struct ISum<float, K, WIDE> {
+template <int K>
+struct ISum<float, K> {
   float h[3][K], l[3][K];
   __device__ __forceinline__ void clear() {
 #pragma unroll
@@ -500,12 +501,15 @@ struct ISum<float, K, WIDE> {
   }
   template <bool OWN>
   __device__ __forceinline__ void chunk(const float4 q, int kself, float eps2,
-                                        const float (&x)[4][K], float (&aj)[3]) {
+                                        const float (&x)[4][K], float (&aj)[3], bool wide) {
     float px[K], py[K], pz[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) px[k] = py[k] = pz[k] = 0.0f;
-    sym_chunk<K, OWN, true, WIDE>(q, kself, eps2, x[0], x[1], x[2], x[3], px, py, pz, aj[0],
-                                  aj[1], aj[2]);
+    if (wide)
+      sym_chunk<K, OWN, true, true>(q, kself, eps2, x[0], x[1], x[2], x[3], px, py, pz, aj[0],
+                                    aj[1], aj[2]);
+    else
+      sym_chunk<K, OWN>(q, kself, eps2, x[0], x[1], x[2], x[3], px, py, pz, aj[0], aj[1], aj[2]);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       two_sum_sym(h[0][k], l[0][k], px[k]);
@@ -515,8 +519,8 @@ struct ISum<float, K, WIDE> {
   }
   __device__ __forceinline__ float get(int c, int k) const { return h[c][k] + l[c][k]; }
 };
-template <int K, bool WIDE>
-struct ISum<double, K, WIDE> {
+template <int K>
+struct ISum<double, K> {
   double p[3][K];
   __device__ __forceinline__ void clear() {
 #pragma unroll
@@ -526,7 +530,7 @@ struct ISum<double, K, WIDE> {
   }
   template <bool OWN>
   __device__ __forceinline__ void chunk(const double4 q, int kself, double eps2,
-                                        const double (&x)[4][K], double (&aj)[3]) {
+                                        const double (&x)[4][K], double (&aj)[3], bool) {
     sym_chunk<K, OWN>(q, kself, eps2, x[0], x[1], x[2], x[3], p[0], p[1], p[2], aj[0], aj[1],
                       aj[2]);
   }
@@ -541,16 +545,35 @@ __device__ __forceinline__ double4 body_or_far(const double4 *__restrict__ posm,
 }
 __device__ __forceinline__ float uniform_operand(float x) { return in_vgpr(x); }
 __device__ __forceinline__ double uniform_operand(double x) { return x; }
+// Ordinary coordinates: 0, or in size from `least` to below `most`.  From 2^-18 on they are
+// multiples of 2^-41, so that two bodies are in one point or at least that far apart, and below
+// 2^40 they are less than 2^42 apart with eps^2 below 2^82: 1/r^3 is an ordinary FP32 number.  A
+// softening of 2^-42 takes care of the lower limit.
+struct Ordinary {
+  float least, most;
+  __device__ __forceinline__ explicit Ordinary(float eps2)
+      : least(eps2 >= 0x1p-84f ? 0.0f : 0x1p-18f), most(eps2 < 0x1p82f ? 0x1p40f : 0.0f) {}
+  __device__ __forceinline__ explicit Ordinary(double) : least(0.0f), most(0.0f) {}
+  __device__ __forceinline__ bool of(float c) const {
+    const float a = __builtin_fabsf(c);
+    return a < most && (a >= least || a == 0.0f);
+  }
+  // whether the bodies p of the whole wavefront have ordinary coordinates (FP64 needs none)
+  __device__ __forceinline__ bool all(const float4 p) const {
+    return __all(of(p.x) && of(p.y) && of(p.z));
+  }
+  __device__ __forceinline__ bool all(const double4) const { return true; }
+};
 // The sign of the i-bodies' masses that sym_chunk takes.
 template <typename T>
 constexpr T kMassSign = sizeof(T) == 4 ? T(-1) : T(1);
 
 // Bound by VALU issue (sym_chunk).  Against the row segments: no block-diagonal pass of its own
 // (FP64, 40000 bodies: 23 of 690 us), no last round of workgroups that leaves half the compute
-// units idle, i-side partials once per group and row.  FP32 65536 bodies: 767 us = 57 cycles per
-// unordered pair and SIMD, of 50 that the loop can reach; 32768 with WIDE: 235 us, 69 cycles,
-// of 53 (its workspace holds five groups per compute unit).
-template <typename T, typename T4, bool WIDE>
+// units idle, i-side partials once per group and row.  FP32 65536 bodies: 745 us = 55 cycles per
+// unordered pair and SIMD, of 50 that the loop can reach; 32768: 220 us, 65 cycles (its workspace
+// holds five groups per compute unit).
+template <typename T, typename T4>
 __global__ __launch_bounds__(kWave *kUnitW) void k_sym_units(const T4 *__restrict__ posm, int n,
                                                               int nb, int nc, int64_t units,
                                                               T eps2, T *__restrict__ p_i,
@@ -579,6 +602,7 @@ __global__ __launch_bounds__(kWave *kUnitW) void k_sym_units(const T4 *__restric
     beta = lo;
   }
   const T eps2v = uniform_operand(eps2);
+  const Ordinary ordinary(eps2);
   int buf = 0;
   for (; u < u_end; ++beta) {
     const int64_t r0 = unit_row(beta, nc, KW), r1 = unit_row(beta + 1, nc, KW);
@@ -586,9 +610,10 @@ __global__ __launch_bounds__(kWave *kUnitW) void k_sym_units(const T4 *__restric
     const int c_end = beta * KW + static_cast<int>((u_end < r1 ? u_end : r1) - r0);
     u += c_end - c;
     T x[4][K];
-    ISum<T, K, WIDE> sum;
+    ISum<T, K> sum;
     sum.clear();
     const int i0 = beta * IB + wave * (K * kWave);
+    bool near = true;   // the i-bodies of this wavefront are ordinary
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const T4 p = body_or_far(posm, i0 + k * kWave + lane, n);
@@ -596,6 +621,7 @@ __global__ __launch_bounds__(kWave *kUnitW) void k_sym_units(const T4 *__restric
       x[1][k] = p.y;
       x[2][k] = p.z;
       x[3][k] = kMassSign<T> * p.w;
+      near &= ordinary.all(p);
     }
     T aj[3] = {0, 0, 0};
     const int own_end = min(c_end, (beta + 1) * KW);
@@ -603,13 +629,14 @@ __global__ __launch_bounds__(kWave *kUnitW) void k_sym_units(const T4 *__restric
 #pragma unroll 1
     for (; c < own_end; ++c, q = qn) {
       qn = body_or_far(posm, (c + 1) * kWave + lane, n);
-      sum.template chunk<true>(q, c - beta * KW - wave * K, eps2v, x, aj);
+      sum.template chunk<true>(q, c - beta * KW - wave * K, eps2v, x, aj,
+                               !(near && ordinary.all(q)));
     }
 #pragma unroll 1
     for (; c < c_end; ++c, q = qn) {
       qn = body_or_far(posm, (c + 1) * kWave + lane, n);
       aj[0] = aj[1] = aj[2] = 0;
-      sum.template chunk<false>(q, -1, eps2v, x, aj);
+      sum.template chunk<false>(q, -1, eps2v, x, aj, !(near && ordinary.all(q)));
       const int gamma = c / KW;
       T *pj = p_j + (pair_row(beta, nb) + (gamma - beta - 1)) * (3 * IB) +
               (c - gamma * KW) * kWave;
@@ -976,15 +1003,11 @@ constexpr int64_t kUnitGroups = 10 * kCus;
 // segments); above, a static division into few thousand groups loses to the row segments, whose
 // workgroups are dispatched as they end.
 // Stage 1, us, row segments in their default shape and this form (in parentheses the j-split
-// form): FP32 19000 bodies 125 and 90 (95), 20480 126 and 100 (107), 32768 241 and 235 (257), 49999
-// 496 and 489 (584), 60000 789 and 700 (836), 65536 932 and 767 (984), 100000 1851 and 1760, 114687
-// 2365 and 2291, 131072 2854 and 2862; FP64 9000 75 and 52 (54), 12288 101 and 78 (92), 20000 207
-// and 184 (236), 40000 711 and 619 (920), 60000 1410 and 1365.
+// form): FP32 19000 bodies 125 and 85 (93), 20480 125 and 94 (104), 32768 235 and 220 (251), 49999
+// 479 and 452 (564), 60000 778 and 646 (803), 65536 918 and 745 (957), 100000 1774 and 1689, 114687
+// 2263 and 2204, 131072 2854 and 2862; FP64 9000 74 and 52 (53), 12288 100 and 78 (89), 20000 202
+// and 179 (227), 40000 691 and 599 (882), 60000 1358 and 1321.
 constexpr int64_t kUnitsFrom = 18945, kUnitsTo = 114688;
-// FP32 sizes whose weights are WIDE (sym_chunk).  Below this size the form stands beside the
-// j-split form, whose range of distances it has to have, and is faster than it with the wider
-// weights too; from here on it stands beside the row segments, which share 1/r^3.
-constexpr int64_t kUnitsWideTo = 65536;
 constexpr int64_t kUnitsFromF64 = 8961, kUnitsToF64 = 65536;
 
 // groups: kUnitGroups, or the multiple of kCus below it whose i-side slots fit the workspace;
@@ -1008,15 +1031,8 @@ int sym_units_run(const T4 *posm, T *acc, double *sums, int n, const UnitPlan &P
                   T eps2, void *ws, hipStream_t s) {
   T *p_j = static_cast<T *>(ws);
   T *p_i = reinterpret_cast<T *>(static_cast<char *>(ws) + P.j_bytes);
-  auto launch = [&](auto wide) {
-    hipLaunchKernelGGL((k_sym_units<T, T4, decltype(wide)::value>),
-                       dim3(static_cast<unsigned>(P.groups)), dim3(kWave * kUnitW), 0, s, posm, n,
-                       P.nb, P.nc, P.units, eps2, p_i, p_j);
-  };
-  if (sizeof(T) == 4 && n < kUnitsWideTo)
-    launch(std::integral_constant<bool, sizeof(T) == 4>());
-  else
-    launch(std::false_type());
+  hipLaunchKernelGGL((k_sym_units<T, T4>), dim3(static_cast<unsigned>(P.groups)),
+                     dim3(kWave * kUnitW), 0, s, posm, n, P.nb, P.nc, P.units, eps2, p_i, p_j);
   const int rc = check_launch("k_sym_units");
   if (rc != GRAV_OK) return rc;
   hipLaunchKernelGGL((k_sym_units_fold<T>), dim3(static_cast<unsigned>(P.nc)),

@@ -109,21 +109,22 @@ def stage1_f32(posm, acc, G, eps=0.0, accum='kahan', cfg=None):
 # 13.4; with the host views refreshed, where the wait hides the launches, 512 21.3 and 21.4, 1000
 # 25.4 and 22.2, 2000 32.9 and 22.4).  The j-split form beats the symmetric one below 19456,
 # where few groups of its balanced form fit its workspace (stage 1, Plummer, us, j-split against
-# symmetric: 17000 84 against 128, 18500 96 against 126, 19456 97 against 89, 24576 149 against
-# 142, 32768 257 against 235, 49999 584 against 489).  FP64: j-split from 448 bodies (a hip1 step
+# symmetric: 17000 83 against 127, 18500 94 against 126, 19456 95 against 83, 24576 144 against
+# 136, 32768 250 against 220, 49999 564 against 452).  FP64: j-split from 448 bodies (a hip1 step
 # of the galaxy, us, owner-computes against j-split, on the device and with the host views
 # refreshed: 384 12.0 and 13.3, 25.1 and 22.5; 448 14.0 and 13.2, 26.3 and 22.4; 640 17.0 and
 # 13.3, 30.7 and 22.7; 1000 26.0 and 13.2, 38.3 and 23.5), symmetric from 10500 (us, j-split
-# against symmetric: 9000 54 against 52, 10000 65 against 65, 10500 73 against 65, 12288 92
-# against 78, 16384 157 against 122, 40000 921 against 619).
+# against symmetric: 9000 53 against 52, 10000 64 against 65, 10500 71 against 65, 12288 89
+# against 78, 16384 152 against 121, 40000 882 against 599).
 SPLIT_FROM = 1088
 SYMMETRIC_FROM = 19456
 SPLIT_F64_FROM = 448
 SYMMETRIC_F64_FROM = 10500
 VJP_SPLIT_FROM = 1024
-# Below this size the symmetric form, given its one-slab workspace, weighs a pair as the owner and
-# j-split forms do, for distances r from 1e-19 to 1e19; from here on it shares 1/r^3 between the
-# two bodies of a pair and needs r between 1.4e-13 and 4.4e12 (or eps above the lower limit).
+# Below this size the symmetric form stands in the j-split form's place and always gets its one-slab
+# workspace: with it the library takes distances r from 1e-19 to 1e19, as the j-split form does
+# (up to 114687 bodies); in row segments it shares 1/r^3 between the two bodies of a pair, which
+# needs r from 1.4e-13 to 4.4e12.
 SYMMETRIC_WIDE_TO = 65536
 
 

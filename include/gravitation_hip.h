@@ -89,10 +89,10 @@ int grav_stage1_f32_cfg(const void *posm, void *acc, int64_t n, double G, double
  * of 19000 to 115000 bodies the work of all rows is instead divided evenly among up to 2560
  * workgroups, where the workspace holds their partial sums (grav_stage1_sym_workspace's size
  * does).
- * A pair's two accelerations share 1/r^3 (r^2 = d^2 + eps^2), which is an FP32 number for r from
- * 1.4e-13 to 4.4e12: nearer pairs give infinities or NaN, farther ones lose their bits.  The
- * evenly divided work of fewer than 65536 bodies is free of that limit: there m/r and 1/r^2 are
- * formed as in grav_stage1_f32, whose r reaches from 1e-19 to 1e19.
+ * In segments a pair's two accelerations share 1/r^3 (r^2 = d^2 + eps^2), which is an FP32 number
+ * for r from 1.4e-13 to 4.4e12: nearer pairs give infinities or NaN, farther ones lose their
+ * bits.  The evenly divided work is free of that limit: where coordinates allow such distances it
+ * forms m/r and 1/r^2 as grav_stage1_f32 does, whose r reaches from 1e-19 to 1e19.
  * grav_stage1_sym_workspace gives the size that holds every segment at once (12 n bytes +
  * 12 block (1 + seglen) bytes per segment: about 12 n + 6 n^2 / block (1 + seglen) / seglen,
  * 510 MB at 2^18 bodies); any size down to grav_stage1_sym_workspace_min's (one row of block

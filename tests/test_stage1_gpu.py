@@ -565,7 +565,7 @@ def test_symmetric_default_shape_at_its_size_limits(cuda, n, dtype):
     stages.release_workspaces()
 
 
-@pytest.mark.parametrize('n', [19456, 57344, 65535])
+@pytest.mark.parametrize('n', [19456, 57344, 65535, 114687])
 @pytest.mark.parametrize('size, mass', [(1e15, 1e20), (1e-10, 1e-12), (1.0, 1.0)])
 def test_symmetric_middle_sizes_have_the_range_of_the_split_form(cuda, n, size, mass):
     # Sizes that the j-split form served before the symmetric one took them over: universes in
@@ -584,6 +584,41 @@ def test_symmetric_middle_sizes_have_the_range_of_the_split_form(cuda, n, size, 
         a = acc.cpu().numpy().T.astype(np.float64)
         assert np.all(np.isfinite(a)), run
         assert O.rel_err(a[rows], ref) < TOL32, run
+
+
+@pytest.mark.parametrize('n', [19456, 65535, 114687])
+@pytest.mark.parametrize('eps', [0.0, 1e-6, 1e14])
+def test_symmetric_range_holds_chunk_by_chunk(cuda, n, eps):
+    # the balanced form chooses between two ways to weigh a pair by the coordinates of each chunk
+    # of 64 bodies: a tight group around the origin (1/r^3 above FP32's largest number), bodies
+    # of ordinary coordinates with some at 0 and at the limits, and a far group (1/r^3 below the
+    # smallest), each to the bar by itself, without softening, with one above the tight group and
+    # with one above all distances
+    print('sym chunks n=%d eps=%g' % (n, eps), flush=True)
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(-1.0, 1.0, (n, 3))
+    m = np.exp(rng.uniform(-3, 3, n)) / n
+    tight, far = np.arange(700), np.arange(n - 900, n)
+    pos[tight] = rng.uniform(-1e-11, 1e-11, (700, 3))
+    m[tight] = 1e-15
+    pos[far] = rng.uniform(-1e14, 1e14, (900, 3))
+    m[far] = 1e20
+    pos[3000, 0] = pos[3001, 1] = 0.0
+    pos[3002], pos[3003], pos[3004] = 2.0 ** -18, -2.0 ** -19, 2.0 ** 40
+    posm = _posm(pos, m, cuda)
+    pos, m = _inputs(posm)
+    groups = [np.arange(0, 700, 11), np.concatenate([np.arange(700, n - 900, n // 60),
+                                                     [3000, 3001, 3002, 3003]]), far[::13]]
+    rows = np.concatenate(groups)
+    ref = oracle_rows(pos, m, 1.0, eps, rows)
+    acc = torch.full((3, n), float('nan'), dtype=torch.float32, device=cuda)
+    stages.stage1_sym_f32(posm, acc, 1.0, eps)
+    a = acc.cpu().numpy().T.astype(np.float64)
+    assert np.all(np.isfinite(a))
+    at = 0
+    for g in groups:
+        assert O.rel_err(a[g], ref[at:at + len(g)]) < TOL32, (eps, len(g))
+        at += len(g)
 
 
 @pytest.mark.parametrize('n', [65, 4096, 5000, 20000])
