@@ -99,7 +99,10 @@ constexpr int kLdsBytes = 160 * 1024;
 // plain loop exposes), full ones by VALU issue.  MI355X, plain loop unrolled by four and this one:
 // 512 universes of 32-256 bodies over 20 steps 196 and 171 us; 1000 of 100-1024 over 10 steps
 // 1016 and 891 us; 1000 of 32-2048 over 5 steps 1778 and 1495 us.  Half-steps of four and
-// without priority: 174, 1001, 1748 us; of four with it: 180, 897, 1537 us.
+// without priority: 174, 1001, 1748 us; of four with it: 180, 897, 1537 us.  The sets take VGPRs
+// (116 instead of 50, with two and four bodies per lane 127 and 237 instead of 98 and 141),
+// which costs less than it gives there too: 8 steps of 1000 universes of 100-1024 bodies, two and
+// four per lane, 1005 and 856 us, 1186 and 989 us; of 2000 of 32-512, 363 and 319 us, 639 and 643.
 template <int KT, bool MASK>
 __device__ __forceinline__ void tile_range(const float4 *cur, int j0, int j1,
                                            const float (&xi)[KT], const float (&yi)[KT],
@@ -286,7 +289,8 @@ __global__ __launch_bounds__(512) void k_batched_fused(
 // The VJP pairs of j in [j0, j1), as tile_range.  MI355X, forward and backward, plain loop
 // unrolled by two (with the forward above) and this one: 120 universes of 100-500 bodies over 8
 // steps 594 and 532 us, 200 of 64-2048 over 4 steps 4.11 and 3.81 ms; half-steps of two: 542 us
-// and 3.89 ms.
+// and 3.89 ms.  Two and four bodies per lane (119 and 161 VGPRs, 88 and 113 before), 1000
+// universes of 100-1024 bodies over 8 steps: 3.04 and 2.66 ms, 4.29 and 3.14 ms.
 template <int KT, bool MASK>
 __device__ __forceinline__ void vjp_tile_range(
     const float4 *pos, const float4 *mub, int j0, int j1, const float (&xk)[KT],
